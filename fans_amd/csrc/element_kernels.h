@@ -555,43 +555,6 @@ __device__ __forceinline__ void PointModel<T, H, NGP, PNL, VISCO>::visco_eval(in
         visco_gp(*this, gp, e, s);
 }
 
-// sigma of the linear models only (the linear matvec K d never sees another
-// kind; anything else gives NaN)
-template <typename T, int H>
-__device__ __forceinline__ void linear_point(const Phase<T> &P, const T (&e)[H == 1 ? 3 : 6],
-                                             T (&s)[H == 1 ? 3 : 6])
-{
-    constexpr int n = H == 1 ? 3 : 6;
-    if (P.kind == MODEL_THERMAL_ISO || P.kind == MODEL_ELASTIC_ISO) {
-        if constexpr (H == 1) {
-#pragma unroll
-            for (int i = 0; i < 3; ++i)
-                s[i] = P.p[0] * e[i];
-        } else {
-            const T b1 = P.p[0] * (e[0] + e[1] + e[2]), b2 = (T) 2 * P.p[1];
-#pragma unroll
-            for (int i = 0; i < 3; ++i)
-                s[i] = b1 + b2 * e[i];
-#pragma unroll
-            for (int i = 3; i < 6; ++i)
-                s[i] = b2 * e[i];
-        }
-    } else if (P.kind == MODEL_THERMAL_TRI || P.kind == MODEL_ELASTIC_TRI) {
-#pragma unroll
-        for (int i = 0; i < n; ++i) {
-            T a = 0;
-#pragma unroll
-            for (int j = 0; j < n; ++j)
-                a += P.p[n * i + j] * e[j];
-            s[i] = a;
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < n; ++i)
-            s[i] = (T) NAN;
-    }
-}
-
 // material_point for any strain vector length (finite strain: NS = 9)
 template <typename T, int H, int NS>
 __device__ __forceinline__ void material_point_ns(const Phase<T> &P, const T (&e)[NS], T (&s)[NS])
@@ -884,158 +847,40 @@ __device__ __forceinline__ void element_forces(const T (&u)[8][H], const Geom &g
     grad_factors_T<T, H, NGP>(Sx, Sy, Sz, g, f);
 }
 
-// Isotropic fast path: with sigma = lambda tr(eps) I + 2 mu eps (Mandel), the
-// Gauss-point loop collapses.  T[c][d] = lambda tr(grad u) delta_cd +
-// mu (du_c/dx_d + du_d/dx_c) is linear in the gradient factors, and the sums
-// over the Gauss index that a factor does not depend on reduce to pairwise
-// sums.  lw = lambda * w, mw = mu * w (w = v_e / n_gp); T0 is the traction
-// tensor of the macroscopic gradient (already multiplied by w), added once
-// per Gauss point.
-template <typename T, int NGP>
-__device__ __forceinline__ void element_forces_iso3(const T (&u)[8][3], const Geom &g, T lw, T mw, const T (&T0)[3][3],
-                                                    T (&f)[8][3])
-{
-    T Gx[2][2][3], Gy[2][2][3], Gz[2][2][3];
-    grad_factors<T, 3, NGP>(u, g, Gx, Gy, Gz);
-    T Sx[2][2][3], Sy[2][2][3], Sz[2][2][3];
-    if constexpr (NGP == 8) {
-        const T l2m2 = (T) 2 * (lw + (T) 2 * mw), m2 = (T) 2 * mw, g2 = (T) 2;
-#pragma unroll
-        for (int a = 0; a < 2; ++a)
-#pragma unroll
-            for (int b = 0; b < 2; ++b) {
-                // sums over the Gauss index the factor does not depend on
-                const T sGy_i0 = Gy[0][b][0] + Gy[1][b][0], sGy_i1 = Gy[0][b][1] + Gy[1][b][1];  // [k=b]
-                const T sGz_i0 = Gz[0][a][0] + Gz[1][a][0], sGz_i2 = Gz[0][a][2] + Gz[1][a][2];  // [j=a]
-                Sx[a][b][0] = l2m2 * Gx[a][b][0] + lw * (sGy_i1 + sGz_i2) + g2 * T0[0][0];
-                Sx[a][b][1] = m2 * Gx[a][b][1] + mw * sGy_i0 + g2 * T0[1][0];
-                Sx[a][b][2] = m2 * Gx[a][b][2] + mw * sGz_i0 + g2 * T0[2][0];
-                const T sGx_j0 = Gx[0][b][0] + Gx[1][b][0], sGx_j1 = Gx[0][b][1] + Gx[1][b][1];  // [k=b]
-                const T sGz_j1 = Gz[a][0][1] + Gz[a][1][1], sGz_j2 = Gz[a][0][2] + Gz[a][1][2];  // [i=a]
-                Sy[a][b][0] = m2 * Gy[a][b][0] + mw * sGx_j1 + g2 * T0[0][1];
-                Sy[a][b][1] = l2m2 * Gy[a][b][1] + lw * (sGx_j0 + sGz_j2) + g2 * T0[1][1];
-                Sy[a][b][2] = m2 * Gy[a][b][2] + mw * sGz_j1 + g2 * T0[2][1];
-                const T sGx_k0 = Gx[b][0][0] + Gx[b][1][0], sGx_k2 = Gx[b][0][2] + Gx[b][1][2];  // [j=b]
-                const T sGy_k1 = Gy[a][0][1] + Gy[a][1][1], sGy_k2 = Gy[a][0][2] + Gy[a][1][2];  // [i=a]
-                Sz[a][b][0] = m2 * Gz[a][b][0] + mw * sGx_k2 + g2 * T0[0][2];
-                Sz[a][b][1] = m2 * Gz[a][b][1] + mw * sGy_k2 + g2 * T0[1][2];
-                Sz[a][b][2] = l2m2 * Gz[a][b][2] + lw * (sGx_k0 + sGy_k1) + g2 * T0[2][2];
-            }
-    } else {
-        const T gr[3][3] = {{Gx[0][0][0], Gy[0][0][0], Gz[0][0][0]},
-                            {Gx[0][0][1], Gy[0][0][1], Gz[0][0][1]},
-                            {Gx[0][0][2], Gy[0][0][2], Gz[0][0][2]}};
-        const T tr       = gr[0][0] + gr[1][1] + gr[2][2];
-        T       Tt[3][3];
-#pragma unroll
-        for (int c = 0; c < 3; ++c)
-#pragma unroll
-            for (int d = 0; d < 3; ++d)
-                Tt[c][d] = mw * (gr[c][d] + gr[d][c]) + (c == d ? lw * tr : (T) 0) + T0[c][d];
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            Sx[0][0][c] = Tt[c][0];
-            Sy[0][0][c] = Tt[c][1];
-            Sz[0][0][c] = Tt[c][2];
-        }
-    }
-#pragma unroll
-    for (int a = 0; a < 8; ++a)
-#pragma unroll
-        for (int c = 0; c < 3; ++c)
-            f[a][c] = (T) 0;
-    grad_factors_T<T, 3, NGP>(Sx, Sy, Sz, g, f);
-}
-
-// isotropic conduction: sigma = k grad + k g0, the Gauss sums are factors of 2
-template <typename T, int NGP>
-__device__ __forceinline__ void element_forces_iso1(const T (&u)[8][1], const Geom &g, T kw, const T (&T0)[3],
-                                                    T (&f)[8][1])
-{
-    T Gx[2][2][1], Gy[2][2][1], Gz[2][2][1];
-    grad_factors<T, 1, NGP>(u, g, Gx, Gy, Gz);
-    const T s = NGP == 8 ? (T) 2 * kw : kw, s0 = NGP == 8 ? (T) 2 : (T) 1;
-    T       Sx[2][2][1], Sy[2][2][1], Sz[2][2][1];
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b) {
-            Sx[a][b][0] = s * Gx[a][b][0] + s0 * T0[0];
-            Sy[a][b][0] = s * Gy[a][b][0] + s0 * T0[1];
-            Sz[a][b][0] = s * Gz[a][b][0] + s0 * T0[2];
-        }
-    f[0][0] = f[1][0] = f[2][0] = f[3][0] = f[4][0] = f[5][0] = f[6][0] = f[7][0] = (T) 0;
-    grad_factors_T<T, 1, NGP>(Sx, Sy, Sz, g, f);
-}
-
 // ---------------------------------------------------------------------------
-// Modal form of the isotropic element operators.
+// Modal form of the linear element operators.
 //
 // With reference coordinates (xi, eta, zeta) in [-1,1]^3, the derivative of the
 // trilinear field along x is bilinear in (eta, zeta):
 //   du/dx = kx/4 (A0 + A1 eta + A2 zeta + A3 eta zeta),  kx = 1/hx,
-// where A = H Dx is the 4-point Hadamard transform of the four x-edge
-// differences (likewise for y over (xi, zeta) and z over (xi, eta)).  The
-// products of two such fields have degree <= 3 in every coordinate, so the
-// 2x2x2 Gauss rule integrates the energy density exactly, and the modes
-// {1, xi, eta, zeta, xi eta, ...} are orthogonal under it (norms 8 / 3^deg).
-// The element energy lambda/2 tr(eps)^2 + mu eps:eps therefore splits into
-// independent modal blocks:
+// where A is the 4-point Hadamard transform of the four x-edge differences
+// (likewise for y over (xi, zeta) and z over (xi, eta)).  The products of two
+// such fields have degree <= 3 in every coordinate, so the 2x2x2 Gauss rule
+// integrates the energy density exactly, and the modes {1, xi, eta, zeta,
+// xi eta, ...} are orthogonal under it (norms 8 / 3^deg).  The element energy
+// eps : C : eps / 2 therefore splits, for any constant C, into independent
+// modal blocks:
 //   mode 1        : all nine gradient entries
 //   mode xi       : d/dy, d/dz   (eta: d/dx, d/dz; zeta: d/dx, d/dy)
 //   mode eta zeta : d/dx only    (xi zeta: d/dy; xi eta: d/dz)
-// and the forces are the transposed Hadamard / edge-difference maps applied to
-// the modal stresses.  With 8 Gauss points both maps are one 3-D Walsh
-// transform of the corner values per component (walsh8: the Hadamard modes of
-// the edge differences are Walsh coefficients, and the mixed modes that two
-// derivative directions share are the same coefficient).  This is the same
-// operator as the Gauss-point loop (the quadrature is exact for it) at about
-// 250 instead of ~600 FP64 operations per element.  For one Gauss point
-// (HEX8R) only mode 1 remains.
-// ---------------------------------------------------------------------------
-
-// forward: D[p][q] (p, q in {0,1}) -> A0..A3
-template <typename T>
-__device__ __forceinline__ void hadamard4(T &d00, T &d10, T &d01, T &d11)
-{
-    const T s0 = d00 + d01, s1 = d10 + d11, e0 = d01 - d00, e1 = d11 - d10;
-    d00 = s0 + s1;  // A0
-    d10 = s1 - s0;  // A1 (slope in p)
-    d01 = e0 + e1;  // A2 (slope in q)
-    d11 = e1 - e0;  // A3 (p q)
-}
-// transpose: A0..A3 -> D[p][q]
-template <typename T>
-__device__ __forceinline__ void hadamard4_T(T &a0, T &a1, T &a2, T &a3)
-{
-    const T p0 = a0 - a2, p1 = a1 - a3, q0 = a0 + a2, q1 = a1 + a3;
-    a0 = p0 - p1;  // D00
-    a1 = p0 + p1;  // D10
-    a2 = q0 - q1;  // D01
-    a3 = q0 + q1;  // D11
-}
-
-// unnormalised 3-D Walsh-Hadamard transform of the 8 corner values (corner /
-// coefficient index i + 2j + 4k): W[ijk] = sum_xyz (-1)^(ix+jy+kz) v[xyz].
-// The Hadamard modes of the edge differences are Walsh coefficients:
+// The Hadamard modes of the edge differences are coefficients of the 3-D Walsh
+// transform of the corner values, W[i + 2j + 4k] = sum (-1)^(ix+jy+kz) v[xyz]:
 //   d/dx: A0..A3 = -W100, W110, W101, -W111   (d/dy: -W010, W110, W011, -W111;
 //   d/dz: -W001, W101, W011, -W111)
-// so one transform of 24 additions replaces the 3 x (4 differences + 8-addition
-// Hadamard) per component, and the transposed maps are one transform of the
-// mode sums.  The transform is symmetric (its own transpose).
-template <typename T>
-__device__ __forceinline__ void walsh8(T (&v)[8])
-{
-#pragma unroll
-    for (int s = 1; s < 8; s <<= 1)
-#pragma unroll
-        for (int a = 0; a < 8; ++a)
-            if ((a & s) == 0) {
-                const T x = v[a], y = v[a + s];
-                v[a]      = x + y;
-                v[a + s]  = x - y;
-            }
-}
+// and the nodal forces are the Walsh transform (its own transpose) of the mode
+// sums b.  The functions below map W[1..7] to b[1..7] (W[0], the mean, carries
+// no gradient); the transforms are the assembly's, which shares their y-z half
+// between the two elements at a node plane.  This is the same operator as the
+// Gauss-point loop (the quadrature is exact for it).  For one Gauss point
+// (HEX8R) only mode 1 remains, b[3], b[5], b[6] and b[7] being zero.
+//
+// The macroscopic gradient of the residual enters mode 1, where it is constant:
+// sh holds 4 gamma(g0) / (CUBIC ? 1/h : 1), gamma the three normal entries and
+// the three sums of shear entries (thermal: the gradient), subtracted from
+// the negated gradient that W[1], W[2] and W[4] are.  SHIFT = false: no
+// gradient (the linear matvec).  CUBIC (hx = hy = hz): the 1/h of the edge
+// differences and of their transpose fold into the modal constants.
+// ---------------------------------------------------------------------------
 
 // modal block with two derivative directions dA, dB present (third missing):
 // a[c] = coefficient of d u_c / d x_dA, b[c] of d u_c / d x_dB
@@ -1054,78 +899,62 @@ __device__ __forceinline__ void modal_pair(T (&a)[3], T (&b)[3], T L, T M)
     b[c0] *= M;
 }
 
-template <typename T, int d>
-__device__ __forceinline__ void modal_single(T (&a)[3], T L, T M)
+// index of gradient entry (c, d) among the six symmetric entries
+// (00 11 22 01 02 12) of a Mandel vector
+__device__ constexpr int sym_idx(int c, int d) { return c == d ? c : c + d + 2; }
+// position of entry (i, j) of a symmetric 6x6 stored by its upper triangle
+__device__ constexpr int tri_idx(int i, int j)
 {
-#pragma unroll
-    for (int c = 0; c < 3; ++c)
-        a[c] *= (c == d) ? (L + M + M) : M;
+    return i <= j ? i * 6 - i * (i - 1) / 2 + j - i : j * 6 - j * (j - 1) / 2 + i - j;
 }
 
-// f = Ke(lambda, mu) u (+ the forces of the traction T0 = w sigma(g0)); same
-// arguments as element_forces_iso3.  CUBIC (hx = hy = hz): the 1/h of the edge
-// differences and of their transpose fold into the modal constants (k^2) and
-// the traction term (k), which saves 72 multiplications per element.
-template <typename T, int NGP, bool CUBIC = false>
-__device__ __forceinline__ void element_forces_iso3_modal(const T (&u)[8][3], const Geom &g, T lw, T mw,
-                                                          const T (&T0)[3][3], T (&f)[8][3])
+// the six symmetric sums of the mode-1 gradient of W, less the shift
+template <typename T, bool SHIFT>
+__device__ __forceinline__ void mode1_sums(const T (&w)[8][3], const T (&k)[3], const T (&sh)[6], T (&g)[6])
 {
-    const T kc   = (T) g.ilx;
-    const T k[3] = {CUBIC ? (T) 1 : (T) g.ilx, CUBIC ? (T) 1 : (T) g.ily, CUBIC ? (T) 1 : (T) g.ilz};
-    // A[d][mode][c]: Hadamard modes of the edge differences along d, scaled by 1/h_d
-    T A[3][4][3];
-    if constexpr (NGP == 8) {
+    g[0] = w[1][0] * k[0];
+    g[1] = w[2][1] * k[1];
+    g[2] = w[4][2] * k[2];
+    g[3] = w[2][0] * k[1] + w[1][1] * k[0];
+    g[4] = w[4][0] * k[2] + w[1][2] * k[0];
+    g[5] = w[4][1] * k[2] + w[2][2] * k[1];
+    if constexpr (SHIFT)
 #pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            T w[8];
+        for (int i = 0; i < 6; ++i)
+            g[i] -= sh[i];
+}
+
+// mode-1 forces of the symmetric stress t (00 11 22 01 02 12)
+template <typename T>
+__device__ __forceinline__ void mode1_forces(const T (&t)[6], const T (&k)[3], T (&b)[8][3])
+{
 #pragma unroll
-            for (int n = 0; n < 8; ++n)
-                w[n] = u[n][c];
-            walsh8(w);
-            A[0][0][c] = -w[1] * k[0], A[0][1][c] = w[3] * k[0], A[0][2][c] = w[5] * k[0], A[0][3][c] = -w[7] * k[0];
-            A[1][0][c] = -w[2] * k[1], A[1][1][c] = w[3] * k[1], A[1][2][c] = w[6] * k[1], A[1][3][c] = -w[7] * k[1];
-            A[2][0][c] = -w[4] * k[2], A[2][1][c] = w[5] * k[2], A[2][2][c] = w[6] * k[2], A[2][3][c] = -w[7] * k[2];
-        }
-    } else {
+    for (int d = 0; d < 3; ++d)
 #pragma unroll
         for (int c = 0; c < 3; ++c)
-#pragma unroll
-            for (int p = 0; p < 2; ++p)
-#pragma unroll
-                for (int q = 0; q < 2; ++q) {
-                    A[0][p + 2 * q][c] = (u[1 + 2 * p + 4 * q][c] - u[2 * p + 4 * q][c]) * k[0];
-                    A[1][p + 2 * q][c] = (u[p + 2 + 4 * q][c] - u[p + 4 * q][c]) * k[1];
-                    A[2][p + 2 * q][c] = (u[p + 2 * q + 4][c] - u[p + 2 * q][c]) * k[2];
-                }
-    }
-    // Gauss weight w = V / NGP; mode weights NGP / 3^deg; 1/16 from the two
-    // factors 1/4 of the bilinear expansion
-    const T s  = CUBIC ? (T) NGP / (T) 16 * kc * kc : (T) NGP / (T) 16;
+            b[1 << d][c] = t[sym_idx(c, d)] * k[d];
+}
+
+// isotropic elasticity: lw = lambda w, mw = mu w, w the Gauss weight
+template <typename T, int NGP, bool CUBIC, bool SHIFT>
+__device__ __forceinline__ void modal_iso3(const T (&w)[8][3], const Geom &g, T lw, T mw, const T (&sh)[6],
+                                           T (&b)[8][3])
+{
+    const T k[3] = {CUBIC ? (T) 1 : (T) g.ilx, CUBIC ? (T) 1 : (T) g.ily, CUBIC ? (T) 1 : (T) g.ilz};
+    // mode weights NGP / 3^deg; 1/16 from the two factors 1/4 of the bilinear
+    // expansion
+    const T s  = CUBIC ? (T) NGP / (T) 16 * (T) g.ilx * (T) g.ilx : (T) NGP / (T) 16;
     const T L0 = s * lw, M0 = s * mw;
-    if constexpr (NGP == 1) {
-#pragma unroll
-        for (int d = 0; d < 3; ++d)
-#pragma unroll
-            for (int c = 0; c < 3; ++c)
-                A[d][0][c] = (A[d][0][c] + A[d][2][c]) + (A[d][1][c] + A[d][3][c]);
-    }
-    // mode 1: all nine entries
     {
-        const T t  = L0 * (A[0][0][0] + A[1][0][1] + A[2][0][2]);
-        const T m2 = M0 + M0;
-        const T t0 = CUBIC ? (T) NGP * (T) 0.25 * kc : (T) NGP * (T) 0.25;
+        T e[6], t[6];
+        mode1_sums<T, SHIFT>(w, k, sh, e);
+        const T tr = L0 * (e[0] + e[1] + e[2]), m2 = M0 + M0;
 #pragma unroll
-        for (int d = 0; d < 3; ++d)
-            A[d][0][d] = t + m2 * A[d][0][d] + t0 * T0[d][d];
-#pragma unroll
-        for (int d = 0; d < 3; ++d)
-#pragma unroll
-            for (int c = d + 1; c < 3; ++c) {
-                // entry (c, d) holds du_c/dx_d, entry (d, c) du_d/dx_c
-                const T v  = M0 * (A[d][0][c] + A[c][0][d]);
-                A[d][0][c] = v + t0 * T0[c][d];
-                A[c][0][d] = v + t0 * T0[d][c];
-            }
+        for (int i = 0; i < 3; ++i) {
+            t[i]     = tr + m2 * e[i];
+            t[3 + i] = M0 * e[3 + i];
+        }
+        mode1_forces(t, k, b);
     }
     if constexpr (NGP == 8) {
         // B-bar keeps only the element-mean trace: the trace energy of the
@@ -1133,132 +962,222 @@ __device__ __forceinline__ void element_forces_iso3_modal(const T (&u)[8][3], co
         const T third = (T) (1.0 / 3.0);
         const T Lh = g.bbar ? (T) (-2.0 / 3.0) * M0 : L0;
         const T L1 = Lh * third, M1 = M0 * third, L2 = L1 * third, M2 = M1 * third;
-        // xi: d/dy mode 1, d/dz mode 1; eta: d/dx mode 1, d/dz mode 2; zeta: d/dx mode 2, d/dy mode 2
-        modal_pair<T, 1, 2>(A[1][1], A[2][1], L1, M1);
-        modal_pair<T, 0, 2>(A[0][1], A[2][2], L1, M1);
-        modal_pair<T, 0, 1>(A[0][2], A[1][2], L1, M1);
-        modal_single<T, 0>(A[0][3], L2, M2);  // eta zeta
-        modal_single<T, 1>(A[1][3], L2, M2);  // xi zeta
-        modal_single<T, 2>(A[2][3], L2, M2);  // xi eta
-        // transposed maps: the Walsh transform of the mode sums
+        // xi: d/dy, d/dz; eta: d/dx, d/dz; zeta: d/dx, d/dy
+        T xy[3], xz[3], ex[3], ez[3], zx[3], zy[3];
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
-            T b[8];
-            b[0] = (T) 0;
-            b[1] = -A[0][0][c] * k[0];
-            b[2] = -A[1][0][c] * k[1];
-            b[4] = -A[2][0][c] * k[2];
-            b[3] = A[0][1][c] * k[0] + A[1][1][c] * k[1];
-            b[5] = A[0][2][c] * k[0] + A[2][1][c] * k[2];
-            b[6] = A[1][2][c] * k[1] + A[2][2][c] * k[2];
-            b[7] = -(A[0][3][c] * k[0] + A[1][3][c] * k[1] + A[2][3][c] * k[2]);
-            walsh8(b);
-#pragma unroll
-            for (int n = 0; n < 8; ++n)
-                f[n][c] = b[n];
+            xy[c] = w[3][c] * k[1], xz[c] = w[5][c] * k[2];
+            ex[c] = w[3][c] * k[0], ez[c] = w[6][c] * k[2];
+            zx[c] = w[5][c] * k[0], zy[c] = w[6][c] * k[1];
         }
-        return;
-    } else {
+        modal_pair<T, 1, 2>(xy, xz, L1, M1);
+        modal_pair<T, 0, 2>(ex, ez, L1, M1);
+        modal_pair<T, 0, 1>(zx, zy, L1, M1);
 #pragma unroll
-        for (int d = 0; d < 3; ++d)
-#pragma unroll
-            for (int c = 0; c < 3; ++c)
-                A[d][1][c] = A[d][2][c] = A[d][3][c] = A[d][0][c];
-    }
-    // transposed edge differences (one Gauss point)
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-#pragma unroll
-        for (int n = 0; n < 8; ++n)
-            f[n][c] = (T) 0;
-#pragma unroll
-        for (int p = 0; p < 2; ++p)
-#pragma unroll
-            for (int q = 0; q < 2; ++q) {
-                const T dx = A[0][p + 2 * q][c] * k[0], dy = A[1][p + 2 * q][c] * k[1],
-                        dz = A[2][p + 2 * q][c] * k[2];
-                f[1 + 2 * p + 4 * q][c] += dx;
-                f[2 * p + 4 * q][c] -= dx;
-                f[p + 2 + 4 * q][c] += dy;
-                f[p + 4 * q][c] -= dy;
-                f[p + 2 * q + 4][c] += dz;
-                f[p + 2 * q][c] -= dz;
-            }
+        for (int c = 0; c < 3; ++c) {
+            b[3][c] = ex[c] * k[0] + xy[c] * k[1];
+            b[5][c] = zx[c] * k[0] + xz[c] * k[2];
+            b[6][c] = zy[c] * k[1] + ez[c] * k[2];
+            // eta zeta: d/dx; xi zeta: d/dy; xi eta: d/dz
+            const T kc = k[c] * k[c], ko = k[(c + 1) % 3] * k[(c + 1) % 3] + k[(c + 2) % 3] * k[(c + 2) % 3];
+            b[7][c]    = w[7][c] * (CUBIC ? L2 + (T) 4 * M2 : (L2 + M2 + M2) * kc + M2 * ko);
+        }
     }
 }
 
-// isotropic conduction in modal form: every mode of every derivative is its
-// own block, weighted by NGP / 3^deg
-template <typename T, int NGP, bool CUBIC = false>
-__device__ __forceinline__ void element_forces_iso1_modal(const T (&u)[8][1], const Geom &g, T kw, const T (&T0)[3],
-                                                          T (&f)[8][1])
+// stress sums of a higher mode with the gradient entries present in PRESENT
+// (bit per symmetric entry): t[i] = sum_j C[i][j] e[j] over the present ones
+template <typename T, unsigned PRESENT>
+__device__ __forceinline__ void modal_aniso_block(const T (&C)[21], const T (&e)[6], T (&t)[6])
 {
-    const T kc   = (T) g.ilx;
-    const T k[3] = {CUBIC ? (T) 1 : (T) g.ilx, CUBIC ? (T) 1 : (T) g.ily, CUBIC ? (T) 1 : (T) g.ilz};
-    const T c0   = CUBIC ? (T) NGP / (T) 16 * kw * kc * kc : (T) NGP / (T) 16 * kw;
-    const T t0   = CUBIC ? (T) NGP * (T) 0.25 * kc : (T) NGP * (T) 0.25;
+#pragma unroll
+    for (int i = 0; i < 6; ++i)
+        if ((PRESENT >> i) & 1u) {
+            T a = (T) 0;
+#pragma unroll
+            for (int j = 0; j < 6; ++j)
+                if ((PRESENT >> j) & 1u)
+                    a += C[tri_idx(i, j)] * e[j];
+            t[i] = a;
+        }
+}
+
+// a mode with the two derivative directions dA, dB: gradient entries a[c] and
+// b[c] in, their stresses out
+template <typename T, int dA, int dB>
+__device__ __forceinline__ void modal_aniso_pair(const T (&C)[21], T (&a)[3], T (&b)[3])
+{
+    constexpr int c0 = 3 - dA - dB;
+    T             e[6], t[6];
+    e[dA]               = a[dA];
+    e[dB]               = b[dB];
+    e[sym_idx(dA, dB)]  = a[dB] + b[dA];
+    e[sym_idx(c0, dA)]  = a[c0];
+    e[sym_idx(c0, dB)]  = b[c0];
+    modal_aniso_block<T, 0x3fu & ~(1u << c0)>(C, e, t);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        a[c] = t[sym_idx(c, dA)];
+        b[c] = t[sym_idx(c, dB)];
+    }
+}
+
+// a mode with the single derivative direction d: adds the force of w to b7
+template <typename T, int d>
+__device__ __forceinline__ void modal_aniso_single(const T (&C)[21], const T (&w)[3], T k2, T (&b7)[3])
+{
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+#pragma unroll
+        for (int e = 0; e < 3; ++e)
+            b7[c] += C[tri_idx(sym_idx(c, d), sym_idx(e, d))] * (w[e] * k2);
+}
+
+// entry e of a phase's tensor in the modal blocks' scale, from the phase table's
+// p (full row-major) and the Gauss weight wg: the upper triangle of the 6x6
+// Mandel stiffness, taken to the entries' own scale (a shear stress is sqrt(1/2)
+// of its Mandel component and the Mandel strain sqrt(1/2) of the shear sum, so
+// that stress = C * symmetric sums), or the 3x3 conductivity
+template <typename T, int H, int NGP>
+__device__ __forceinline__ T modal_tensor_entry(const T *__restrict__ p, int e, T wg)
+{
+    const T s = (T) NGP / (T) 16 * wg;
+    if constexpr (H == 1) {
+        return p[e] * s;
+    } else {
+        int i = 0, r = e;  // row i, offset r from its diagonal
+        while (r >= 6 - i)
+            r -= 6 - i++;
+        const int j = i + r;
+        return p[6 * i + j] * (i < 3 ? (j < 3 ? s : s * (T) kSqrtHalf) : s * (T) 0.5);
+    }
+}
+
+// any linear elasticity: Ct from modal_tensor_entry.  B-bar removes the trace of
+// every mode but the first on both sides: C becomes P C P.
+template <typename T, int NGP, bool SHIFT>
+__device__ __forceinline__ void modal_aniso3(const T (&w)[8][3], const Geom &g, const T *Ct, const T (&sh)[6],
+                                             T (&b)[8][3])
+{
+    const T k[3] = {(T) g.ilx, (T) g.ily, (T) g.ilz};
+    T       C[21];
+#pragma unroll
+    for (int i = 0; i < 21; ++i)
+        C[i] = Ct[i];
+    {
+        T e[6], t[6];
+        mode1_sums<T, SHIFT>(w, k, sh, e);
+        modal_aniso_block<T, 0x3fu>(C, e, t);
+        mode1_forces(t, k, b);
+    }
     if constexpr (NGP == 8) {
-        // Walsh coefficients -> modes (see walsh8), modal scaling, mode sums -> Walsh
-        T w[8];
+        const T third = (T) (1.0 / 3.0);
+        if (g.bbar) {
+            T rs[6];
 #pragma unroll
-        for (int n = 0; n < 8; ++n)
-            w[n] = u[n][0];
-        walsh8(w);
+            for (int j = 0; j < 6; ++j)
+                rs[j] = (C[tri_idx(0, j)] + C[tri_idx(1, j)] + C[tri_idx(2, j)]) * third;
+            const T all = (rs[0] + rs[1] + rs[2]) * third;
+#pragma unroll
+            for (int i = 0; i < 3; ++i)
+#pragma unroll
+                for (int j = i; j < 6; ++j)
+                    C[tri_idx(i, j)] -= j < 3 ? rs[i] + rs[j] - all : rs[j];
+        }
+#pragma unroll
+        for (int i = 0; i < 21; ++i)
+            C[i] *= third;
+        T xy[3], xz[3], ex[3], ez[3], zx[3], zy[3];
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+            xy[c] = w[3][c] * k[1], xz[c] = w[5][c] * k[2];
+        modal_aniso_pair<T, 1, 2>(C, xy, xz);
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+            ex[c] = w[3][c] * k[0], ez[c] = w[6][c] * k[2];
+        modal_aniso_pair<T, 0, 2>(C, ex, ez);
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+            zx[c] = w[5][c] * k[0], zy[c] = w[6][c] * k[1];
+        modal_aniso_pair<T, 0, 1>(C, zx, zy);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            b[3][c] = ex[c] * k[0] + xy[c] * k[1];
+            b[5][c] = zx[c] * k[0] + xz[c] * k[2];
+            b[6][c] = zy[c] * k[1] + ez[c] * k[2];
+            b[7][c] = (T) 0;
+        }
+        modal_aniso_single<T, 0>(C, w[7], k[0] * k[0] * third, b[7]);
+        modal_aniso_single<T, 1>(C, w[7], k[1] * k[1] * third, b[7]);
+        modal_aniso_single<T, 2>(C, w[7], k[2] * k[2] * third, b[7]);
+    }
+}
+
+// isotropic conduction: every mode of every derivative is its own block
+template <typename T, int NGP, bool CUBIC, bool SHIFT>
+__device__ __forceinline__ void modal_iso1(const T (&w)[8][1], const Geom &g, T kw, const T (&sh)[3], T (&b)[8][1])
+{
+    const T k[3] = {CUBIC ? (T) 1 : (T) g.ilx, CUBIC ? (T) 1 : (T) g.ily, CUBIC ? (T) 1 : (T) g.ilz};
+    const T c0   = CUBIC ? (T) NGP / (T) 16 * kw * (T) g.ilx * (T) g.ilx : (T) NGP / (T) 16 * kw;
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+        b[1 << d][0] = c0 * (w[1 << d][0] * k[d] - (SHIFT ? sh[d] : (T) 0)) * k[d];
+    if constexpr (NGP == 8) {
         const T c1 = c0 * (T) (1.0 / 3.0), c2 = c1 * (T) (1.0 / 3.0);
-        T       b[8];
-        b[0]        = (T) 0;
-        b[1]        = -(c0 * (-w[1] * k[0]) + t0 * T0[0]) * k[0];
-        b[2]        = -(c0 * (-w[2] * k[1]) + t0 * T0[1]) * k[1];
-        b[4]        = -(c0 * (-w[4] * k[2]) + t0 * T0[2]) * k[2];
-        b[3]        = c1 * w[3] * (k[0] * k[0] + k[1] * k[1]);
-        b[5]        = c1 * w[5] * (k[0] * k[0] + k[2] * k[2]);
-        b[6]        = c1 * w[6] * (k[1] * k[1] + k[2] * k[2]);
-        b[7]        = c2 * w[7] * (k[0] * k[0] + k[1] * k[1] + k[2] * k[2]);
-        walsh8(b);
-#pragma unroll
-        for (int n = 0; n < 8; ++n)
-            f[n][0] = b[n];
-        return;
+        b[3][0] = c1 * w[3][0] * (k[0] * k[0] + k[1] * k[1]);
+        b[5][0] = c1 * w[5][0] * (k[0] * k[0] + k[2] * k[2]);
+        b[6][0] = c1 * w[6][0] * (k[1] * k[1] + k[2] * k[2]);
+        b[7][0] = c2 * w[7][0] * (k[0] * k[0] + k[1] * k[1] + k[2] * k[2]);
     }
-    T A[3][4];
+}
+
+// conduction with any symmetric tensor: Kt from modal_tensor_entry
+template <typename T, int NGP, bool SHIFT>
+__device__ __forceinline__ void modal_aniso1(const T (&w)[8][1], const Geom &g, const T *Kt, const T (&sh)[3],
+                                             T (&b)[8][1])
+{
+    const T s1 = (T) (1.0 / 3.0), s2 = (T) (1.0 / 9.0);
+    const T k[3] = {(T) g.ilx, (T) g.ily, (T) g.ilz};
+    T       K[3][3], q[3];
 #pragma unroll
-    for (int p = 0; p < 2; ++p)
+    for (int i = 0; i < 3; ++i) {
 #pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            A[0][p + 2 * q] = (u[1 + 2 * p + 4 * q][0] - u[2 * p + 4 * q][0]) * k[0];
-            A[1][p + 2 * q] = (u[p + 2 + 4 * q][0] - u[p + 4 * q][0]) * k[1];
-            A[2][p + 2 * q] = (u[p + 2 * q + 4][0] - u[p + 2 * q][0]) * k[2];
-        }
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        if constexpr (NGP == 8) {
-            const T c1 = c0 * (T) (1.0 / 3.0), c2 = c1 * (T) (1.0 / 3.0);
-            hadamard4(A[d][0], A[d][1], A[d][2], A[d][3]);
-            A[d][0] = c0 * A[d][0] + t0 * T0[d];
-            A[d][1] *= c1;
-            A[d][2] *= c1;
-            A[d][3] *= c2;
-            hadamard4_T(A[d][0], A[d][1], A[d][2], A[d][3]);
-        } else {
-            const T a = c0 * ((A[d][0] + A[d][2]) + (A[d][1] + A[d][3])) + t0 * T0[d];
-            A[d][0] = A[d][1] = A[d][2] = A[d][3] = a;
-        }
+        for (int j = 0; j < 3; ++j)
+            K[i][j] = Kt[3 * i + j] * k[i] * k[j];
+        q[i] = w[1 << i][0] - (SHIFT ? sh[i] / k[i] : (T) 0);
     }
 #pragma unroll
-    for (int n = 0; n < 8; ++n)
-        f[n][0] = (T) 0;
-#pragma unroll
-    for (int p = 0; p < 2; ++p)
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            const T dx = A[0][p + 2 * q] * k[0], dy = A[1][p + 2 * q] * k[1], dz = A[2][p + 2 * q] * k[2];
-            f[1 + 2 * p + 4 * q][0] += dx;
-            f[2 * p + 4 * q][0] -= dx;
-            f[p + 2 + 4 * q][0] += dy;
-            f[p + 4 * q][0] -= dy;
-            f[p + 2 * q + 4][0] += dz;
-            f[p + 2 * q][0] -= dz;
-        }
+    for (int i = 0; i < 3; ++i)
+        b[1 << i][0] = K[i][0] * q[0] + K[i][1] * q[1] + K[i][2] * q[2];
+    if constexpr (NGP == 8) {
+        const T w3 = w[3][0], w5 = w[5][0], w6 = w[6][0];
+        // xi: d/dy of w3, d/dz of w5; eta: d/dx of w3, d/dz of w6; zeta: d/dx of
+        // w5, d/dy of w6
+        b[3][0] = s1 * ((K[0][0] + K[1][1]) * w3 + K[0][2] * w6 + K[1][2] * w5);
+        b[5][0] = s1 * ((K[0][0] + K[2][2]) * w5 + K[0][1] * w6 + K[1][2] * w3);
+        b[6][0] = s1 * ((K[1][1] + K[2][2]) * w6 + K[0][1] * w5 + K[0][2] * w3);
+        b[7][0] = s2 * (K[0][0] + K[1][1] + K[2][2]) * w[7][0];
+    }
+}
+
+template <typename T, int H, int NGP, bool SHIFT, int NS>
+__device__ __forceinline__ void modal_aniso(const T (&w)[8][H], const Geom &g, const T *Ct, const T (&sh)[NS],
+                                            T (&b)[8][H])
+{
+    if constexpr (H == 3)
+        modal_aniso3<T, NGP, SHIFT>(w, g, Ct, sh, b);
+    else
+        modal_aniso1<T, NGP, SHIFT>(w, g, Ct, sh, b);
+}
+
+// a value staged in LDS by words, one array of 256 words per 4 bytes of it
+template <typename T>
+__device__ __forceinline__ T staged_value(const int *p)
+{
+    if constexpr (sizeof(T) == 8)
+        return __hiloint2double(p[256], p[0]);
+    else
+        return __int_as_float(p[0]);
 }
 
 // lane l <- lane l-1 inside each row of 16 lanes (DPP row_shr:1); row starts get 0

@@ -342,7 +342,8 @@ struct fans_gpu_ctx {
     std::array<int, 7>    batch_sig{};
 
     // launch geometry
-    int     cx = 16, nty = 0, ntz = 0, nblk_asm = 0, nblk_vec = 0, nblk_el = 0;
+    int     cx = 1, nty = 0, ntz = 0, nblk_asm = 0, nblk_vec = 0, nblk_el = 0;
+    bool    cx_set = false;  // the caller chose cx (FANS_OPT_ASM_PLANES)
     int64_t nslot = 0;      // J2 state slots per component and Gauss point
     int     js_comps = 0;   // components of the allocated J2 state
     int     nblk_slot = 0;  // workgroups of the state commit (one thread per slot)
@@ -916,53 +917,125 @@ AsmArgs<T> asm_args(fans_gpu_ctx *c)
     return a;
 }
 
+// x planes per assembly workgroup for `tiles` y-z tiles: the depth of least
+// cost, a workgroup of cx planes computing cx + 1 (its first plane only feeds
+// the next one's carry).  Planes run at one unit per CU while the chip is full;
+// a workgroup alone on its CU takes 1.75 units per plane in the modal kernel
+// (latency; three fit) and 1 in the per-Gauss-point one, so too few workgroups
+// cost more than the extra plane of thin ones: the 48^3 elastic matvec (16 tiles)
+// took 24 us at 12 planes (64 workgroups), the 64^3 J2 residual (25 tiles) 118 us
+// at 16 (100 workgroups).
+int asm_planes_rule(int nx, int64_t tiles, bool modal, int grp = 1)
+{
+    constexpr int kCus = 256, kMaxPlanes = 16;
+    int           best = grp;
+    double        best_cost = 1e300;
+    for (int cx = grp; cx <= std::max(grp, std::min(nx, kMaxPlanes)); cx += grp) {
+        const int64_t nb   = (int64_t) ((nx + cx - 1) / cx) * tiles;
+        const double  per  = (double) ((nb + kCus - 1) / kCus);
+        const double  cost = (cx + 1) * (modal ? std::max(per, 1.75) : per);
+        if (cost <= best_cost) {
+            best      = cx;
+            best_cost = cost;
+        }
+    }
+    return best;
+}
+
+int ensure_partials(fans_gpu_ctx *c);
+
+// every phase linear, small strain: the modal kernel
+bool asm_modal(const fans_gpu_ctx *c) { return c->all_linear && c->nstr != 9; }
+
+void set_planes(fans_gpu_ctx *c, int cx)
+{
+    c->cx       = cx;
+    c->nblk_asm = (c->nx + cx - 1) / cx * c->nty * c->ntz;
+}
+
+// the depth of the context's materials, unless the caller set one
+int choose_planes(fans_gpu_ctx *c)
+{
+    const int cx = c->cx_set ? c->cx : asm_planes_rule(c->nx, (int64_t) c->nty * c->ntz, asm_modal(c));
+    if (cx != c->cx) {
+        set_planes(c, cx);
+        drop_graphs(c);
+    }
+    return ensure_partials(c);
+}
+
+// k_assemble_modal for the context's materials.  Byte ids find their phase in
+// the workgroup's staged table; tensors are staged while they leave room for two
+// workgroups per CU (the registers' limit): 64 KiB, about 120 phases in FP64.
+template <typename T, int H, int NGP, int MODE>
+void launch_modal(fans_gpu_ctx *c, const AsmArgs<T> &a, dim3 g)
+{
+#define MODAL(VAR, MAT, LDS) \
+    hipLaunchKernelGGL((k_assemble_modal<T, H, NGP, MODE, VAR, MAT>), g, dim3(kThreads), LDS, c->stream, a)
+    if (!c->all_iso) {
+        const size_t lds = sizeof(T) * kTensorLen<T, H>() * std::min(c->nphases, kStagedPhases);
+        if (!c->ms16 && lds + modal_static_lds<T, H>() <= 64 * 1024)
+            MODAL(ASM_ANISO, MAT_STAGED, lds);
+        else
+            MODAL(ASM_ANISO, MAT_TABLE, 0);
+    } else if (c->cubic) {
+        if (c->voxel_moduli)
+            MODAL(ASM_ISO_CUBIC, MAT_VOXEL, 0);
+        else if (c->ms16)
+            MODAL(ASM_ISO_CUBIC, MAT_TABLE, 0);
+        else
+            MODAL(ASM_ISO_CUBIC, MAT_STAGED, 0);
+    } else {
+        if (c->voxel_moduli)
+            MODAL(ASM_ISO, MAT_VOXEL, 0);
+        else if (c->ms16)
+            MODAL(ASM_ISO, MAT_TABLE, 0);
+        else
+            MODAL(ASM_ISO, MAT_STAGED, 0);
+    }
+#undef MODAL
+}
+
 template <typename T, int MODE>
 int launch_assemble(fans_gpu_ctx *c, AsmArgs<T> a)
 {
     Timed t(c, MODE == ASM_CGLIN ? KF_ASSEMBLE_LIN : KF_ASSEMBLE_RES);
-#define ASM(HH, GG)                                                                                             \
-    do {                                                                                                        \
-        if (c->all_iso && c->cubic)                                                                             \
-            hipLaunchKernelGGL((k_assemble<T, HH, GG, MODE, ASM_ISO_CUBIC>), dim3(c->nblk_asm, 1, c->gz), dim3(kThreads), \
-                               0, c->stream, a);                                                                \
-        else if (c->all_iso)                                                                                    \
-            hipLaunchKernelGGL((k_assemble<T, HH, GG, MODE, ASM_ISO>), dim3(c->nblk_asm, 1, c->gz), dim3(kThreads), 0,    \
-                               c->stream, a);                                                                   \
-        else if (MODE == ASM_RESID && HH == 3 && c->has_visco)                                                  \
-            hipLaunchKernelGGL(                                                                                 \
-                (k_assemble<T, HH, GG, MODE, MODE == ASM_RESID && HH == 3 ? ASM_GENERAL_VISCO : ASM_GENERAL>),   \
-                dim3(c->nblk_asm, 1, c->gz), dim3(kThreads), 0, c->stream, a);                                            \
-        else if (MODE == ASM_RESID && c->has_pnl)                                                               \
-            hipLaunchKernelGGL((k_assemble<T, HH, GG, MODE, MODE == ASM_RESID ? ASM_GENERAL_PNL : ASM_GENERAL>),   \
-                               dim3(c->nblk_asm, 1, c->gz), dim3(kThreads), 0, c->stream, a);                             \
-        else                                                                                                    \
-            hipLaunchKernelGGL((k_assemble<T, HH, GG, MODE, ASM_GENERAL>), dim3(c->nblk_asm, 1, c->gz), dim3(kThreads),   \
-                               0, c->stream, a);                                                                \
-    } while (0)
-    if (c->nstr == 9) {
-        // finite strain: only the residual (the models are nonlinear)
-        if constexpr (MODE == ASM_RESID) {
-            if (c->ngp == 8)
-                hipLaunchKernelGGL((k_assemble<T, 3, 8, MODE, ASM_LARGE>), dim3(c->nblk_asm, 1, c->gz), dim3(kThreads), 0,
-                                   c->stream, a);
-            else
-                hipLaunchKernelGGL((k_assemble<T, 3, 1, MODE, ASM_LARGE>), dim3(c->nblk_asm, 1, c->gz), dim3(kThreads), 0,
-                                   c->stream, a);
-        } else {
-            return fail(c, FANS_GPU_EINVAL, "linear matvec needs linear materials");
+    if (asm_modal(c)) {
+        // partials come per c->cx planes whatever depth runs: a batch of many
+        // slots takes deeper workgroups without moving any slot's sums
+        int nblk = c->nblk_asm;
+        a.grp    = c->cx;
+        if (MODE == ASM_CGLIN && c->gz > 1 && !c->cx_set) {
+            a.cx = asm_planes_rule(c->nx, (int64_t) c->nty * c->ntz * c->gz, true, c->cx);
+            nblk = (c->nx + a.cx - 1) / a.cx * c->nty * c->ntz;
         }
-    } else if (c->h == 1) {
-        if (c->ngp == 8)
-            ASM(1, 8);
+        const dim3 g(nblk, 1, c->gz);
+        if (c->h == 1)
+            c->ngp == 8 ? launch_modal<T, 1, 8, MODE>(c, a, g) : launch_modal<T, 1, 1, MODE>(c, a, g);
         else
-            ASM(1, 1);
-    } else {
-        if (c->ngp == 8)
-            ASM(3, 8);
+            c->ngp == 8 ? launch_modal<T, 3, 8, MODE>(c, a, g) : launch_modal<T, 3, 1, MODE>(c, a, g);
+    } else if constexpr (MODE == ASM_RESID) {
+        // nonlinear materials (thermal models are all linear)
+        const dim3 g(c->nblk_asm, 1, c->gz);
+#define ASM(VAR)                                                                                               \
+    do {                                                                                                       \
+        if (c->ngp == 8)                                                                                       \
+            hipLaunchKernelGGL((k_assemble<T, 3, 8, VAR>), g, dim3(kThreads), 0, c->stream, a);                \
+        else                                                                                                   \
+            hipLaunchKernelGGL((k_assemble<T, 3, 1, VAR>), g, dim3(kThreads), 0, c->stream, a);                \
+    } while (0)
+        if (c->nstr == 9)
+            ASM(ASM_LARGE);
+        else if (c->has_visco)
+            ASM(ASM_GENERAL_VISCO);
+        else if (c->has_pnl)
+            ASM(ASM_GENERAL_PNL);
         else
-            ASM(3, 1);
-    }
+            ASM(ASM_GENERAL);
 #undef ASM
+    } else {
+        return fail(c, FANS_GPU_EINVAL, "linear matvec needs linear materials");
+    }
     HIPCHK(c, hipGetLastError());
     return 0;
 }
@@ -1364,8 +1437,8 @@ int cg_linear_loop(fans_gpu_ctx *c, Fft3D<T> &P, T *r, T *const *ring, T *rnew, 
         a.sl         = launch_slots(c, true);
         if ((e = launch_assemble<T, ASM_CGLIN>(c, a)))
             return e;
-        // quantity 1 of the first iteration: the matvec's zero slot 1
-        if ((e = reduce(c, c->partial, c->nblk_asm, 2, RED_ALPHA, j > 0 ? c->partial_e : nullptr,
+        // quantity 1, <d, K d_prev>, is zero in the first iteration
+        if ((e = reduce(c, c->partial, c->nblk_asm, j > 0 ? 2 : 1, RED_ALPHA, j > 0 ? c->partial_e : nullptr,
                         (int) P.nblk_z)))
             return e;
         if (j % kDirRing == kDirRing - 1 && (e = ring_update(kDirRing, true)))
@@ -2457,9 +2530,7 @@ static int create_ctx(fans_gpu_ctx **out, const fans_gpu_desc *d, int slots)
     // launch geometry
     c->nty      = (c->ny + NOUT - 1) / NOUT;
     c->ntz      = (c->nz + NOUT - 1) / NOUT;
-    c->cx       = c->nx >= 64 ? 16 : std::max(1, c->nx / 4);
-    const int nbx = (c->nx + c->cx - 1) / c->cx;
-    c->nblk_asm = nbx * c->nty * c->ntz;
+    set_planes(c, asm_planes_rule(c->nx, (int64_t) c->nty * c->ntz, c->nstr != 9));
     c->nblk_vec = grid_vec(c->Nh);
     c->nblk_el  = (int) ((c->N + kThreads - 1) / kThreads);
     // J2 state slots (J2State); the state commit walks them
@@ -2793,7 +2864,13 @@ int fans_gpu_set_materials(fans_gpu_ctx *c, int32_t ng, const int32_t *kind, con
         for (int k = 0; k < ns * ns; ++k)
             c->kref[k] /= (double) ng;
     }
-    // per-phase device tables
+    // per-phase device tables; linear phases that are not all isotropic all
+    // hold full tensors (ASM_ANISO)
+    c->all_iso = true;
+    for (int p = 0; p < c->nphases; ++p)
+        if (c->phase_kind[p] != (c->h == 1 ? FANS_MODEL_THERMAL_ISO : FANS_MODEL_ELASTIC_ISO))
+            c->all_iso = false;
+    const bool aniso = c->all_linear && !c->all_iso;
     c->ph64.assign(c->nphases, Phase<double>{});
     c->ph32.assign(c->nphases, Phase<float>{});
     for (int p = 0; p < c->nphases; ++p) {
@@ -2801,10 +2878,22 @@ int fans_gpu_set_materials(fans_gpu_ctx *c, int32_t ng, const int32_t *kind, con
         P.kind           = c->phase_kind[p];
         const double *q  = pp[p];
         switch (P.kind) {
-        case FANS_MODEL_THERMAL_ISO: P.p[0] = q[0]; break;
+        case FANS_MODEL_THERMAL_ISO:
+            if (aniso) {
+                P.kind = FANS_MODEL_THERMAL_TRI;
+                linear_C(ns, FANS_MODEL_THERMAL_ISO, q, P.p);
+            } else {
+                P.p[0] = q[0];
+            }
+            break;
         case FANS_MODEL_THERMAL_TRI:
         case FANS_MODEL_ELASTIC_TRI: linear_C(ns, P.kind, q, P.p); break;
         case FANS_MODEL_ELASTIC_ISO:
+            if (aniso) {
+                P.kind = FANS_MODEL_ELASTIC_TRI;
+                linear_C(ns, FANS_MODEL_ELASTIC_ISO, q, P.p);
+                break;
+            }
             P.p[0] = q[0] - (2.0 / 3.0) * q[1];
             P.p[1] = q[1];
             break;
@@ -2880,10 +2969,8 @@ int fans_gpu_set_materials(fans_gpu_ctx *c, int32_t ng, const int32_t *kind, con
     if (const int rcg = rebuild_green(c))
         return rcg;
     HIPCHK(c, hipStreamSynchronize(c->stream));
-    c->all_iso = true;
-    for (int p = 0; p < c->nphases; ++p)
-        if (c->phase_kind[p] != (c->h == 1 ? FANS_MODEL_THERMAL_ISO : FANS_MODEL_ELASTIC_ISO))
-            c->all_iso = false;
+    if (const int rcp = choose_planes(c))
+        return rcp;
     c->have_mat = true;
     if (c->nb == 1)  // batched solves check their graphs themselves
         refresh_graphs(c);
@@ -3883,9 +3970,8 @@ int fans_gpu_set_option(fans_gpu_ctx *c, int32_t opt, int64_t value)
         // x planes per assembly workgroup (tile shape of the stencil pass)
         if (value < 1 || value > c->nx)
             return fail(c, FANS_GPU_EINVAL, "assembly planes per block must be in [1, n_x]");
-        c->cx           = (int) value;
-        const int nbx   = (c->nx + c->cx - 1) / c->cx;
-        c->nblk_asm     = nbx * c->nty * c->ntz;
+        c->cx_set = true;
+        set_planes(c, (int) value);
         drop_graphs(c);
         return ensure_partials(c);
     }

@@ -33,7 +33,7 @@ constexpr int kDirRing = 8;
 enum {
     RED_ERR_INIT = 0,  // q0 = norm partials      -> err0, iter = 0, delta = 1, deltamid = 0
     RED_DELTA    = 1,  // q0 = <r,s> partials     -> delta, beta
-    RED_ALPHA    = 2,  // q0 = <d,rnew>, q1 = <d,rnew_prev> (nq 2) -> alpha (and deltamid)
+    RED_ALPHA    = 2,  // q0 = <d,rnew>, q1 = <d,rnew_prev> (nq 1: zero) -> alpha, deltamid
     RED_ERR_NEXT = 4,  // q0 = norm partials      -> err, iter++
     RED_SUM      = 5,  // q0..q(nq-1) sums        -> SC_RES0 + q
     RED_ERR_SET  = 6   // q0 = norm partials      -> err, stop test (iteration and CG scalars kept)
@@ -143,8 +143,7 @@ __global__ __launch_bounds__(kReduceThreads) void k_reduce(const double *__restr
                     // deltamid of the next iteration, <r - alpha K d, s> with
                     // s = d - beta d_prev (solverCG.h:87, 91 and 104):
                     // delta - alpha (<d, K d> - beta <K d_prev, d>), K symmetric
-                    if (nq == 2)
-                        sc[SC_DELTAMID] = S.delta - alpha * (v[0] - S.beta * v[1]);
+                    sc[SC_DELTAMID] = S.delta - alpha * (v[0] - S.beta * v[1]);
                 } else if (stage == RED_ERR_NEXT) {
                     is[IS_ITER] = S.iter + 1;
                     record_error(sc, is, hist, S, S.iter + 1, finish_norm(v[0], measure));
@@ -342,16 +341,6 @@ __global__ __launch_bounds__(256) void k_axpby(T *__restrict__ y, const TX *__re
     }
     for (int64_t i = (int64_t) blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t) gridDim.x * blockDim.x)
         y[i] = (T) (a * (double) x[i] + b * (double) y[i]);
-}
-
-// d = s + beta d with beta from the device scalars (nonlinear CG, solverCG.h:94)
-template <typename T>
-__global__ __launch_bounds__(256) void k_direction(T *__restrict__ d, const T *__restrict__ s, const double *__restrict__ sc,
-                                                   int64_t n)
-{
-    const T beta = (T) sc[SC_BETA];
-    for (int64_t i = (int64_t) blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t) gridDim.x * blockDim.x)
-        d[i] = s[i] + beta * d[i];
 }
 
 // start of the secant line search in one pass (solverCG.h:94, :127-129): the
