@@ -3,14 +3,17 @@
     python -m fans_amd.build            # compile the HIP library
     python -m fans_amd.build --verbose
 
-The library is a single translation unit (csrc/fans_gpu.hip including the
-kernel headers) compiled with hipcc for gfx950 only.  Packed FP32 VALU ops are
+The library is the translation units of csrc/*.hip (the kernels by family and
+precision, so that they compile in parallel), compiled with hipcc for gfx950
+only and linked into one shared object.  Packed FP32 VALU ops are
 disabled (-packed-fp32-ops) so the compiler never emits v_pk_{add,mul,fma}_f32.
 """
 import os
 import shutil
 import subprocess
 import sys
+import tempfile
+from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
@@ -37,17 +40,26 @@ def flags():
 
 
 def build(verbose=False):
-    src = os.path.join(CSRC, "fans_gpu.hip")
+    units = sorted(f for f in os.listdir(CSRC) if f.endswith(".hip"))
     tmp = LIB + ".tmp"
-    cmd = [hipcc()] + flags() + ["-o", tmp, src]
-    if verbose:
-        print(" ".join(cmd), flush=True)
-    res = subprocess.run(cmd, capture_output=True, text=True)
-    if res.returncode != 0:
-        sys.stderr.write(res.stdout + res.stderr)
-        raise RuntimeError("hipcc failed to build libfans_gpu.so")
-    if verbose and res.stderr.strip():
-        sys.stderr.write(res.stderr)
+    with tempfile.TemporaryDirectory() as d:
+        objs = [os.path.join(d, u + ".o") for u in units]
+
+        def run(cmd):
+            if verbose:
+                print(" ".join(cmd), flush=True)
+            res = subprocess.run(cmd, capture_output=True, text=True)
+            if res.returncode != 0:
+                sys.stderr.write(res.stdout + res.stderr)
+                raise RuntimeError("hipcc failed to build libfans_gpu.so")
+            if verbose and res.stderr.strip():
+                sys.stderr.write(res.stderr)
+
+        compile_flags = [f for f in flags() if f != "-shared"]
+        with ThreadPoolExecutor(max_workers=min(len(units), os.cpu_count() or 1)) as ex:
+            list(ex.map(run, [[hipcc()] + compile_flags + ["-c", "-o", o, os.path.join(CSRC, u)]
+                              for u, o in zip(units, objs)]))
+        run([hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", tmp] + objs)
     os.replace(tmp, LIB)
     return LIB
 

@@ -20,36 +20,13 @@
 #include <string>
 #include <vector>
 
-#include "assemble_kernels.h"
-#include "common.h"
-#include "element_kernels.h"
-#include "fft_kernels.h"
-#include "fft_reg_kernels.h"
+#include "context.h"
 #include "green_kernels.h"
 #include "vec_kernels.h"
 
-using namespace fans;
-
 namespace {
 
-constexpr int kThreads = 256;
-
-// kernel families for the timing report
-enum {
-    KF_FFT_Z_FWD = 0,
-    KF_FFT_Y_FWD,
-    KF_FFT_X_GREEN,
-    KF_FFT_Y_INV,
-    KF_FFT_Z_INV,
-    KF_ASSEMBLE_LIN,
-    KF_ASSEMBLE_RES,
-    KF_CG_UPDATE,
-    KF_REDUCE,
-    KF_VECTOR,
-    KF_ELEMENT,
-    KF_CG_FFT_Z_FWD,  // CG update fused into the forward z pass
-    KF_COUNT
-};
+// names of the kernel families of the timing report
 const char *kFamilyNames[KF_COUNT] = {"fft_z_r2c",    "fft_y_fwd",    "fft_x_green",  "fft_y_inv",
                                       "fft_z_c2r",    "assemble_lin", "assemble_res", "cg_update",
                                       "reduce",       "vector",       "element_pass", "cg_update_fft_z_r2c"};
@@ -74,315 +51,6 @@ int nparams(int kind)
 bool model_visco(int kind) { return kind == FANS_MODEL_J2_VISCO_LIN || kind == FANS_MODEL_J2_VISCO_NL; }
 bool model_linear(int kind) { return kind >= 1 && kind <= 4; }
 bool model_large(int kind) { return kind == FANS_MODEL_SVK || kind == FANS_MODEL_NEO_HOOKE; }
-
-// ---- host twiddles (long double, then rounded) ------------------------------
-template <typename T>
-std::vector<cplx<T>> twiddles(int n)
-{
-    std::vector<cplx<T>> w(n);
-    const long double    pi = 3.14159265358979323846264338327950288L;
-    for (int k = 0; k < n; ++k) {
-        long double th = -2.0L * pi * (long double) k / (long double) n;
-        w[k]           = cplx<T>{(T) cosl(th), (T) sinl(th)};
-    }
-    return w;
-}
-
-bool make_len(int n, int tws, FftLen &L)
-{
-    L.n   = n;
-    L.tws = tws;
-    L.nst = 0;
-    int m = n;
-    for (int r : {5, 3})
-        while (m % r == 0) {
-            if (L.nst >= 14)
-                return false;
-            L.rad[L.nst++] = r;
-            m /= r;
-        }
-    while (m % 8 == 0) {
-        L.rad[L.nst++] = 8;
-        m /= 8;
-    }
-    while (m % 4 == 0) {
-        L.rad[L.nst++] = 4;
-        m /= 4;
-    }
-    while (m % 2 == 0) {
-        L.rad[L.nst++] = 2;
-        m /= 2;
-    }
-    return m == 1;
-}
-
-// lines per block of the compile-time z kernels (0: generic kernels)
-int zct_lines(int h, int M)
-{
-    switch (M) {
-    case 128: return h == 1 ? zct_lpb<1, 128>() : zct_lpb<3, 128>();
-    case 64: return h == 1 ? zct_lpb<1, 64>() : zct_lpb<3, 64>();
-    case 48: return h == 1 ? zct_lpb<1, 48>() : zct_lpb<3, 48>();
-    case 40: return h == 1 ? zct_lpb<1, 40>() : zct_lpb<3, 40>();
-    case 32: return h == 1 ? zct_lpb<1, 32>() : zct_lpb<3, 32>();
-    case 24: return h == 1 ? zct_lpb<1, 24>() : zct_lpb<3, 24>();
-    case 16: return h == 1 ? zct_lpb<1, 16>() : zct_lpb<3, 16>();
-    default: return 0;
-    }
-}
-
-template <typename T>
-struct Fft3D {
-    int           nx = 0, ny = 0, nz = 0, h = 0, M = 0, Mc = 0;
-    FftLen        Lz{}, Ly{}, Lx{};
-    cplx<T>      *twz = nullptr, *twy = nullptr, *twx = nullptr;
-    int           lpb = 1, bc = 8, bk = 2, bcx = 8;
-    size_t        smz = 0, smy = 0, smx = 0, smx_plain = 0;
-    // LDS budget of one workgroup of the generic (LDS-tiled) passes; it sets
-    // their lines / columns per workgroup (FANS_OPT_FFT_LDS_KIB)
-    int           lds_kib = 40;
-
-    // largest power of two <= min(limit, cap), at least 1
-    static int pow2_cols(int limit, int cap)
-    {
-        int v = 1;
-        while (v * 2 <= limit && v * 2 <= cap)
-            v *= 2;
-        return v;
-    }
-    int64_t       nblk_z = 0;
-    bool          zct    = false;  // compile-time z kernels in use
-    bool          ready  = false;
-
-    hipError_t init(int nx_, int ny_, int nz_, int h_)
-    {
-        hipError_t e = plan(nx_, ny_, nz_, h_);
-        if (e != hipSuccess)
-            return e;
-        ready   = false;
-        auto up = [](cplx<T> *&dst, const std::vector<cplx<T>> &v) {
-            hipError_t e = hipMalloc(&dst, sizeof(cplx<T>) * v.size());
-            if (e != hipSuccess)
-                return e;
-            return hipMemcpy(dst, v.data(), sizeof(cplx<T>) * v.size(), hipMemcpyHostToDevice);
-        };
-        if ((e = up(twz, twiddles<T>(nz))) != hipSuccess)
-            return e;
-        if ((e = up(twy, twiddles<T>(ny))) != hipSuccess)
-            return e;
-        if ((e = up(twx, twiddles<T>(nx))) != hipSuccess)
-            return e;
-        ready = true;
-        return hipSuccess;
-    }
-    // launch shapes and length factorisations only (host arithmetic, no device
-    // memory): the twiddle tables twz / twy / twx are the caller's to provide
-    hipError_t plan(int nx_, int ny_, int nz_, int h_)
-    {
-        nx = nx_, ny = ny_, nz = nz_, h = h_;
-        M  = nz / 2;
-        Mc = M + 1;
-        if (!make_len(M, 2, Lz) || !make_len(ny, 1, Ly) || !make_len(nx, 1, Lx))
-            return hipErrorInvalidValue;
-        // One padded LDS tile per workgroup, n * columns <= FFT_MAX_ELEMS so the
-        // in-place stages keep every butterfly input in registers.
-        const size_t cb = sizeof(cplx<T>);
-        if ((int64_t) M * h > FFT_MAX_ELEMS || ny > FFT_MAX_ELEMS || (int64_t) nx * h > FFT_MAX_ELEMS)
-            return hipErrorInvalidValue;
-        // the default 40 KiB of LDS per workgroup keeps four workgroups
-        // resident per CU
-        const int lds_elems = (int) ((int64_t) lds_kib * 1024 / cb);
-        const int lim       = std::min(FFT_MAX_ELEMS, lds_elems);
-        lpb                 = std::max(1, std::min(16, lim / (M * h)));
-        smz                 = cb * M * (lpb * h + 1);
-        const int Kc        = Mc * h;
-        bc                  = pow2_cols(lim / ny, std::min(Kc, 16));
-        smy                 = cb * ny * (bc + 1);
-        bk                  = std::max(1, std::min(Mc, lim / (nx * h)));
-        smx                 = cb * nx * (bk * h + 1);
-        bcx                 = pow2_cols(lim / nx, 16);
-        smx_plain    = cb * nx * (bcx + 1);
-        nblk_z       = ((int64_t) nx * ny + lpb - 1) / lpb;
-        const int lct = zct_lines(h, M);
-        zct           = lct > 0 && ((int64_t) nx * ny) % lct == 0;
-        if (zct)
-            nblk_z = (int64_t) nx * ny / lct;
-        ready = true;
-        return hipSuccess;
-    }
-    void release()
-    {
-        (void) hipFree(twz);
-        (void) hipFree(twy);
-        (void) hipFree(twx);
-        twz = twy = twx = nullptr;
-        ready           = false;
-    }
-};
-
-// RVE slots of one batched context at most
-constexpr int kMaxSlots = 4096;
-
-// per-RVE device buffers of a context and the stride kind of each (Slots);
-// g0 holds 9 entries per slot, the device scalars SC_COUNT / IS_COUNT
-#define FANS_SLOT_BUFFERS(X)                                                                                   \
-    X(double, u, field) X(double, u_prev, field) X(double, r, field) X(double, s, field) X(double, dA, field)   \
-    X(double, dB, field) X(double, rnew, field) X(cplx<double>, spec64, spec) X(double, G64, green)            \
-    X(float, G32, green) X(uint8_t, ms, ms) X(Phase<double>, dph64, ph) X(Phase<float>, dph32, ph)            \
-    X(double, g0d, g0) X(float, g0f, g0) X(double, partial, part) X(double, partial_e, part) X(double, sc, sc) \
-    X(int, is, is) X(double, hist, hist) X(float, r32, field) X(float, s32, field) X(float, dA32, field)       \
-    X(float, dB32, field) X(float, rnew32, field) X(float, x32, field) X(cplx<float>, spec32, spec)
-enum SlotKind { SK_field, SK_spec, SK_green, SK_ms, SK_ph, SK_g0, SK_part, SK_sc, SK_is, SK_hist };
-
-// slot 0's address of every per-RVE buffer of a batched context
-struct SlotBase {
-#define X(T, name, kind) T *name = nullptr;
-    FANS_SLOT_BUFFERS(X)
-#undef X
-    double *ring64[kDirRing]{};
-    float  *ring32[kDirRing]{};
-};
-
-// host state of one RVE of a batched context while another slot is selected
-#define FANS_SLOT_HOST(X)                                                                                      \
-    X(have_ms) X(have_mat) X(ms16) X(ms_max) X(nphases) X(phase_kind) X(all_linear) X(has_j2) X(all_iso)        \
-    X(has_pnl) X(has_visco) X(user_ref) X(voxel_moduli) X(ph64) X(ph32) X(gxq) X(gyq) X(iter) X(inner_iters)    \
-    X(outer_iters) X(err_hist) X(solve_ms) X(kref) X(keref) X(g0) X(gvec) X(gvec_prev)
-struct SlotHost {
-    bool                       have_ms = false, have_mat = false, ms16 = false;
-    int                        ms_max = -1, nphases = 0;
-    std::vector<int>           phase_kind;
-    bool                       all_linear = true, has_j2 = false, all_iso = false, has_pnl = false;
-    bool                       has_visco = false, user_ref = false, voxel_moduli = false;
-    std::vector<Phase<double>> ph64;
-    std::vector<Phase<float>>  ph32;
-    int                        gxq = 0, gyq = 0, iter = 0, inner_iters = 0, outer_iters = 0;
-    std::vector<double>        err_hist;
-    double                     solve_ms = 0;
-    double                     kref[81]{}, keref[576]{}, g0[9]{}, gvec[9]{}, gvec_prev[9]{};
-};
-
-}  // namespace
-
-struct fans_gpu_ctx {
-    fans_gpu_desc d{};
-    std::string   err;
-    int           nx = 0, ny = 0, nz = 0, h = 0, nstr = 0, ngp = 0;
-    int64_t       N = 0, Nh = 0, Nf = 0;
-    hipStream_t   stream = nullptr;
-    int           tol_type = 0;  // current error type (tangent switches it, solver.h:749)
-    double        tol      = 0;
-
-    // materials
-    bool                        have_ms = false, have_mat = false;
-    int                         ms_max  = -1;  // largest phase id of the microstructure
-    int                         nphases = 0;
-    std::vector<int>            phase_kind;
-    bool                        all_linear = true, has_j2 = false, all_iso = false;
-    bool                        has_pnl = false;  // a PseudoPlasticNonLinearHardening phase
-    bool                        has_visco = false;  // a J2ViscoPlastic phase
-    bool                        cubic = false;  // hx == hy == hz
-    double                      kref[81]{};
-    double                      keref[576]{};
-    std::vector<Phase<double>>  ph64;
-    std::vector<Phase<float>>   ph32;
-
-    // device buffers
-    uint8_t       *ms = nullptr;  // phase ids: bytes, or 16-bit ids when ms16
-    bool           ms16 = false;
-    int64_t        ms_bytes = 0;  // allocated bytes of ms
-    int            nph_cap  = 0;  // allocated entries of dph64 / dph32
-    Phase<double> *dph64 = nullptr;
-    Phase<float>  *dph32 = nullptr;
-    double        *u = nullptr, *u_prev = nullptr, *r = nullptr, *s = nullptr, *dA = nullptr, *dB = nullptr,
-           *rnew = nullptr;
-    cplx<double> *spec64 = nullptr;
-    double       *G64 = nullptr, *keref_d = nullptr;
-    float        *G32 = nullptr;
-    int           gxq = 0, gyq = 0;  // stored kx / ky counts of the Green operator
-    // per-voxel isotropic moduli (K, G; thermal: k in vk), replacing the phase table
-    bool          voxel_moduli = false, user_ref = false;
-    double       *vk64 = nullptr, *vg64 = nullptr;
-    float        *vk32 = nullptr, *vg32 = nullptr;
-    double       *ub_d = nullptr, *sens_d = nullptr;
-    double       *js = nullptr;
-    double       *g0d = nullptr;
-    float        *g0f = nullptr;
-    double       *partial = nullptr;
-    int64_t       partial_len = 0;
-    double       *partial_e   = nullptr;  // [nblk_z] of the linear CG's inverse z pass
-    int64_t       partial_e_len = 0;
-    double       *sc = nullptr;
-    int          *is = nullptr;
-    double       *hist = nullptr;
-    // FP32 inner solve (mixed form)
-    float        *r32 = nullptr, *s32 = nullptr, *dA32 = nullptr, *dB32 = nullptr, *rnew32 = nullptr, *x32 = nullptr;
-    cplx<float>  *spec32 = nullptr;
-    // linear CG direction rings: slots 0 and 1 are dA / dB (dA32 / dB32), the
-    // others are allocated by the first linear CG solve
-    double *ring64[kDirRing]{};
-    float  *ring32[kDirRing]{};
-    Fft3D<double> fft64;
-    Fft3D<float>  fft32;
-
-    // RVE slots (fans_gpu_create_batch): nb same-shape RVEs whose per-RVE
-    // device buffers lie nb times at the strides of `strides`.  The buffer
-    // fields above address the selected slot `cur`, `base` keeps slot 0's
-    // addresses and `parked` the host state of the slots not selected.  A
-    // batched solve points the fields at slot 0 and launches gz slots per
-    // kernel (grid z) through the device map `slot_map`.
-    int                   nb = 1, cur = 0, gz = 1;
-    bool                  use_map  = false;
-    int                  *slot_map = nullptr;
-    int                   map_cap  = 0;
-    std::vector<int>      map_h, map_slots;  // uploaded map and the slots it holds
-    Slots                 strides{};
-    SlotBase              base{};
-    std::vector<SlotHost> parked;
-    std::array<int, 7>    batch_sig{};
-
-    // launch geometry
-    int     cx = 1, nty = 0, ntz = 0, nblk_asm = 0, nblk_vec = 0, nblk_el = 0;
-    bool    cx_set = false;  // the caller chose cx (FANS_OPT_ASM_PLANES)
-    int64_t nslot = 0;      // J2 state slots per component and Gauss point
-    int     js_comps = 0;   // components of the allocated J2 state
-    int     nblk_slot = 0;  // workgroups of the state commit (one thread per slot)
-    double  g0[9]{};
-    Geom    geom{};
-
-    // mixed BC (mixedBCs.h)
-    bool                mixed_active = false;
-    std::vector<int>    idxE, idxF;
-    std::vector<double> FE, PF, M;
-    int                 nsteps = 0, step = 0;
-    double              gvec[9]{}, gvec_prev[9]{};
-    double              alpha_warm = 0.1;
-
-    // results
-    int                 iter = 0, inner_iters = 0, outer_iters = 0;
-    std::vector<double> err_hist;
-    double              solve_ms = 0;
-
-    // timing
-    bool                                                timing = false;
-    int                                                 fft_chunks = 1;
-    // the single-operator entry points run the mixed form's FP32 kernels
-    bool                                                op_fp32 = false;
-    // single-RVE mixed form with restarted inner solves (as batched contexts)
-    bool                                                mixed_restart = false;
-    // captured CG iterations (hipGraph), keyed by precision and the direction
-    // buffer current at the first captured iteration
-    bool                                                use_graphs = true;
-    // key: the direction buffer and the slots per launch (gz)
-    std::vector<std::pair<std::pair<const void *, int>, hipGraphExec_t>> graphs;
-    std::array<int, 7>                                  graph_sig{};
-    std::vector<std::pair<int, std::pair<hipEvent_t, hipEvent_t>>> ev_used;
-    std::vector<hipEvent_t>                             ev_pool;
-    double                                              fam_ms[KF_COUNT]{};
-    int                                                 fam_n[KF_COUNT]{};
-};
-
-namespace {
 
 // message of the last failed context-free call of this thread
 thread_local char g_noalloc_err[256] = "";
@@ -576,17 +244,6 @@ void select_slot(fans_gpu_ctx *c, int b)
     set_views(c, b);
 }
 
-// slots of a launch: the selected slot alone (its buffers are the fields), or
-// during a batched solve the slots of the device map; `gated`: finished slots
-// return at entry
-Slots launch_slots(const fans_gpu_ctx *c, bool gated)
-{
-    Slots s = c->strides;
-    s.map   = c->use_map ? c->slot_map : nullptr;
-    s.is    = gated ? c->is : nullptr;
-    return s;
-}
-
 // launch the given slots from now on, one grid z plane each
 int set_map(fans_gpu_ctx *c, const std::vector<int> &slots)
 {
@@ -607,191 +264,8 @@ void clear_map(fans_gpu_ctx *c)
     c->map_slots.clear();
 }
 
-// ---------------------------------------------------------------------------
-// power-of-two lengths 16..256 use the register four-step kernels
-// ---------------------------------------------------------------------------
-bool reg_len(int n) { return n == 16 || n == 32 || n == 64 || n == 128 || n == 256; }
-// mixed-radix lengths of the register y pass (24 x 4, 20 x 4, 12 x 4); the
-// FP32 x+Green pass takes them too
-bool reg_len_y(int n) { return n == 96 || n == 80 || n == 48; }
-
-// columns per block: a power of two (>= 4) within ~72 KiB of LDS (two
-// workgroups per CU) and at most MAXT threads; at 256^3 FP64 this gives 16
-// columns (256-byte row segments) for the y pass and 4 frequencies for the x
-// pass.  The FP32 y pass takes 512 threads (32 columns, 256-byte segments:
-// 0.095 -> 0.085 ms at 256^3); the FP32 x pass stays at 256 (wider was slower).
-constexpr int kRegLdsKiB = 72;
-template <typename T, int N1, int N2, int MAXT = 256>
-constexpr int reg_cols()
-{
-    constexpr int n   = N1 * N2;
-    constexpr int lim = (int) (kRegLdsKiB * 1024 / (n * sizeof(cplx<T>)));
-    int           c   = 4;
-    while (c * 2 <= lim && c * 2 * N2 <= MAXT)
-        c *= 2;
-    return c;
-}
-template <typename T>
-constexpr int strided_max_threads()
-{
-    return sizeof(T) == 4 ? 512 : 256;
-}
-
-template <typename T, bool INV, int N1, int N2>
-void launch_strided_reg(fans_gpu_ctx *c, cplx<T> *spec, const cplx<T> *tw, int64_t sn, int c0, int c1,
-                        int64_t ostride, int nouter, const int *done)
-{
-    constexpr int C   = reg_cols<T, N1, N2, strided_max_threads<T>()>();
-    const int     nbx = (c1 - c0 + C - 1) / C;
-    hipLaunchKernelGGL((k_fft_strided_reg<T, N1, N2, C, INV>), dim3(nbx * nouter, 1, c->gz), dim3(C * N2), 0,
-                       c->stream, spec, tw, sn, c0, c1, ostride, nbx, launch_slots(c, done != nullptr));
-}
-
-template <typename T, bool INV>
-void launch_strided(fans_gpu_ctx *c, const FftLen &L, const cplx<T> *tw, int bc, size_t smem, cplx<T> *spec,
-                    int64_t sn, int c0, int c1, int64_t ostride, int nouter, const int *done)
-{
-    switch (reg_len(L.n) || reg_len_y(L.n) ? L.n : 0) {
-    case 96: launch_strided_reg<T, INV, 24, 4>(c, spec, tw, sn, c0, c1, ostride, nouter, done); break;
-    case 80: launch_strided_reg<T, INV, 20, 4>(c, spec, tw, sn, c0, c1, ostride, nouter, done); break;
-    case 48: launch_strided_reg<T, INV, 12, 4>(c, spec, tw, sn, c0, c1, ostride, nouter, done); break;
-    case 256: launch_strided_reg<T, INV, 16, 16>(c, spec, tw, sn, c0, c1, ostride, nouter, done); break;
-    case 128: launch_strided_reg<T, INV, 16, 8>(c, spec, tw, sn, c0, c1, ostride, nouter, done); break;
-    case 64: launch_strided_reg<T, INV, 8, 8>(c, spec, tw, sn, c0, c1, ostride, nouter, done); break;
-    case 32: launch_strided_reg<T, INV, 8, 4>(c, spec, tw, sn, c0, c1, ostride, nouter, done); break;
-    case 16: launch_strided_reg<T, INV, 4, 4>(c, spec, tw, sn, c0, c1, ostride, nouter, done); break;
-    default:
-        hipLaunchKernelGGL((k_fft_strided<T, INV>), dim3((c1 - c0 + bc - 1) / bc, nouter, c->gz), dim3(kThreads),
-                           smem, c->stream, spec, L, tw, sn, c0, c1, ostride, bc, launch_slots(c, done != nullptr));
-    }
-}
-
-// Split transposes (fourstep_split) for the x+Green pass: measured at 256^3
-// FP64 they took the pass from 0.29 to 0.50 ms (twice the barriers outweigh the
-// doubled residency), so the complex tile stays
-constexpr bool kXGreenSplit = false;
-
-// x+Green launches return their block count (one partial of the spectral
-// <r, s> per block when `partial` is set)
-template <typename T, int H, int N1, int N2>
-int launch_x_green_reg(fans_gpu_ctx *c, cplx<T> *spec, const cplx<T> *tw, const GreenView<T> &gv, int kz_lo,
-                       int kz_hi, double *partial, const int *done)
-{
-    constexpr int C   = reg_cols<T, N1, N2>();
-    constexpr int KB  = H == 3 ? (C == 16 ? 5 : C / 4) : C;
-    const int     nbk = (kz_hi - kz_lo + KB - 1) / KB;
-    // the complex transpose tile of the 256-point FP64 pass (70 KB) allows two
-    // workgroups per CU; the split tile (35 KB) four
-    constexpr bool SPLIT = kXGreenSplit && (int64_t) N1 * N2 * (C + 1) * sizeof(cplx<T>) > 48 * 1024;
-    hipLaunchKernelGGL((k_fft_x_green_reg<T, H, N1, N2, KB, C, SPLIT>), dim3(nbk * c->ny, 1, c->gz), dim3(C * N2),
-                       0, c->stream, spec, tw, gv, kz_lo, kz_hi, nbk, partial, launch_slots(c, done != nullptr));
-    return nbk * c->ny;
-}
-
-template <typename T, int H>
-int launch_x_green(fans_gpu_ctx *c, Fft3D<T> &P, cplx<T> *spec, const T *G, int kz_lo, int kz_hi, double *partial,
-                   const int *done)
-{
-    const GreenView<T> gv{G, c->nx, c->ny, c->gxq, c->gyq, P.Mc};
-    if constexpr (sizeof(T) == 4) {  // FP64 at 20 x 4 and 24 x 4 would spill (one wave)
-        switch (P.Lx.n) {
-        case 96: return launch_x_green_reg<T, H, 24, 4>(c, spec, P.twx, gv, kz_lo, kz_hi, partial, done);
-        case 80: return launch_x_green_reg<T, H, 20, 4>(c, spec, P.twx, gv, kz_lo, kz_hi, partial, done);
-        case 48: return launch_x_green_reg<T, H, 12, 4>(c, spec, P.twx, gv, kz_lo, kz_hi, partial, done);
-        default: break;
-        }
-    }
-    switch (reg_len(P.Lx.n) ? P.Lx.n : 0) {
-    case 256: return launch_x_green_reg<T, H, 16, 16>(c, spec, P.twx, gv, kz_lo, kz_hi, partial, done);
-    case 128: return launch_x_green_reg<T, H, 16, 8>(c, spec, P.twx, gv, kz_lo, kz_hi, partial, done);
-    case 64: return launch_x_green_reg<T, H, 8, 8>(c, spec, P.twx, gv, kz_lo, kz_hi, partial, done);
-    case 32: return launch_x_green_reg<T, H, 8, 4>(c, spec, P.twx, gv, kz_lo, kz_hi, partial, done);
-    case 16: return launch_x_green_reg<T, H, 4, 4>(c, spec, P.twx, gv, kz_lo, kz_hi, partial, done);
-    default: {
-        dim3 g((kz_hi - kz_lo + P.bk - 1) / P.bk, c->ny, c->gz);
-        hipLaunchKernelGGL((k_fft_x_green<T, H>), g, dim3(kThreads), P.smx, c->stream, spec, P.Lx, P.twx, gv, kz_lo,
-                           kz_hi, P.bk, partial, launch_slots(c, done != nullptr));
-        return (int) (g.x * g.y);
-    }
-    }
-}
-
-// blocks of one x+Green launch over all kz (the size of its partial array)
-template <typename T>
-int64_t x_green_blocks(const Fft3D<T> &P, int h, int ny)
-{
-    int kb = 0;
-    if constexpr (sizeof(T) == 4)  // the same choice as launch_x_green
-        switch (P.Lx.n) {
-        case 96: kb = reg_cols<T, 24, 4>(); break;
-        case 80: kb = reg_cols<T, 20, 4>(); break;
-        case 48: kb = reg_cols<T, 12, 4>(); break;
-        default: break;
-        }
-    switch (kb ? -1 : (reg_len(P.Lx.n) ? P.Lx.n : 0)) {
-    case -1: break;
-    case 256: kb = reg_cols<T, 16, 16>(); break;
-    case 128: kb = reg_cols<T, 16, 8>(); break;
-    case 64: kb = reg_cols<T, 8, 8>(); break;
-    case 32: kb = reg_cols<T, 8, 4>(); break;
-    case 16: kb = reg_cols<T, 4, 4>(); break;
-    default: return (int64_t) ((P.Mc + P.bk - 1) / P.bk) * ny;
-    }
-    if (h == 3)
-        kb = kb == 16 ? 5 : kb / 4;
-    return (int64_t) ((P.Mc + kb - 1) / kb) * ny;
-}
-
 int reduce(fans_gpu_ctx *c, const double *partial, int nblk, int nq, int stage, const double *partial_b = nullptr,
            int nblk_b = 0);
-
-// z passes: compile-time kernels where M = nz/2 is in {16, 24, 32, 40, 48, 64,
-// 128} and the line count divides evenly, else the generic ones
-template <typename T, int H, int PRO>
-void launch_z_r2c(fans_gpu_ctx *c, Fft3D<T> &P, T *rin, cplx<T> *spec, const ProArgs<T> &pa, const int *done)
-{
-    const int64_t nlines = (int64_t) c->nx * c->ny;
-    const Slots   sl     = launch_slots(c, done != nullptr);
-#define ZF(MM)                                                                                                  \
-    hipLaunchKernelGGL((k_fft_z_r2c_ct<T, H, MM, PRO>), dim3((unsigned) (nlines / zct_lpb<H, MM>()), 1, c->gz),  \
-                       dim3(zct_threads<H, MM>()), 0, c->stream, rin, spec, P.twz, pa, sl)
-    switch (P.zct ? P.M : 0) {
-    case 128: ZF(128); break;
-    case 64: ZF(64); break;
-    case 48: ZF(48); break;
-    case 40: ZF(40); break;
-    case 32: ZF(32); break;
-    case 24: ZF(24); break;
-    case 16: ZF(16); break;
-    default:
-        hipLaunchKernelGGL((k_fft_z_r2c<T, H, PRO>), dim3(P.nblk_z, 1, c->gz), dim3(kThreads), P.smz, c->stream, rin,
-                           spec, P.Lz, P.twz, c->nz, nlines, P.lpb, pa, sl);
-    }
-#undef ZF
-}
-
-template <typename T, int H, int EPI>
-void launch_z_c2r(fans_gpu_ctx *c, Fft3D<T> &P, const cplx<T> *spec, const EpiArgs<T> &ep, const int *done)
-{
-    const int64_t nlines = (int64_t) c->nx * c->ny;
-    const Slots   sl     = launch_slots(c, done != nullptr);
-#define ZI(MM)                                                                                                  \
-    hipLaunchKernelGGL((k_fft_z_c2r_ct<T, H, MM, EPI>), dim3((unsigned) (nlines / zct_lpb<H, MM>()), 1, c->gz),  \
-                       dim3(zct_threads<H, MM>()), 0, c->stream, spec, P.twz, ep, sl)
-    switch (P.zct ? P.M : 0) {
-    case 128: ZI(128); break;
-    case 64: ZI(64); break;
-    case 48: ZI(48); break;
-    case 40: ZI(40); break;
-    case 32: ZI(32); break;
-    case 24: ZI(24); break;
-    case 16: ZI(16); break;
-    default:
-        hipLaunchKernelGGL((k_fft_z_c2r<T, H, EPI>), dim3(P.nblk_z, 1, c->gz), dim3(kThreads), P.smz, c->stream, spec,
-                           P.Lz, P.twz, c->nz, nlines, P.lpb, ep, sl);
-    }
-#undef ZI
-}
 
 // ---------------------------------------------------------------------------
 // FFT convolution: out = G * r  with the requested epilogue.  With `pro` the
@@ -964,38 +438,6 @@ int choose_planes(fans_gpu_ctx *c)
     return ensure_partials(c);
 }
 
-// k_assemble_modal for the context's materials.  Byte ids find their phase in
-// the workgroup's staged table; tensors are staged while they leave room for two
-// workgroups per CU (the registers' limit): 64 KiB, about 120 phases in FP64.
-template <typename T, int H, int NGP, int MODE>
-void launch_modal(fans_gpu_ctx *c, const AsmArgs<T> &a, dim3 g)
-{
-#define MODAL(VAR, MAT, LDS) \
-    hipLaunchKernelGGL((k_assemble_modal<T, H, NGP, MODE, VAR, MAT>), g, dim3(kThreads), LDS, c->stream, a)
-    if (!c->all_iso) {
-        const size_t lds = sizeof(T) * kTensorLen<T, H>() * std::min(c->nphases, kStagedPhases);
-        if (!c->ms16 && lds + modal_static_lds<T, H>() <= 64 * 1024)
-            MODAL(ASM_ANISO, MAT_STAGED, lds);
-        else
-            MODAL(ASM_ANISO, MAT_TABLE, 0);
-    } else if (c->cubic) {
-        if (c->voxel_moduli)
-            MODAL(ASM_ISO_CUBIC, MAT_VOXEL, 0);
-        else if (c->ms16)
-            MODAL(ASM_ISO_CUBIC, MAT_TABLE, 0);
-        else
-            MODAL(ASM_ISO_CUBIC, MAT_STAGED, 0);
-    } else {
-        if (c->voxel_moduli)
-            MODAL(ASM_ISO, MAT_VOXEL, 0);
-        else if (c->ms16)
-            MODAL(ASM_ISO, MAT_TABLE, 0);
-        else
-            MODAL(ASM_ISO, MAT_STAGED, 0);
-    }
-#undef MODAL
-}
-
 template <typename T, int MODE>
 int launch_assemble(fans_gpu_ctx *c, AsmArgs<T> a)
 {
@@ -1015,24 +457,7 @@ int launch_assemble(fans_gpu_ctx *c, AsmArgs<T> a)
         else
             c->ngp == 8 ? launch_modal<T, 3, 8, MODE>(c, a, g) : launch_modal<T, 3, 1, MODE>(c, a, g);
     } else if constexpr (MODE == ASM_RESID) {
-        // nonlinear materials (thermal models are all linear)
-        const dim3 g(c->nblk_asm, 1, c->gz);
-#define ASM(VAR)                                                                                               \
-    do {                                                                                                       \
-        if (c->ngp == 8)                                                                                       \
-            hipLaunchKernelGGL((k_assemble<T, 3, 8, VAR>), g, dim3(kThreads), 0, c->stream, a);                \
-        else                                                                                                   \
-            hipLaunchKernelGGL((k_assemble<T, 3, 1, VAR>), g, dim3(kThreads), 0, c->stream, a);                \
-    } while (0)
-        if (c->nstr == 9)
-            ASM(ASM_LARGE);
-        else if (c->has_visco)
-            ASM(ASM_GENERAL_VISCO);
-        else if (c->has_pnl)
-            ASM(ASM_GENERAL_PNL);
-        else
-            ASM(ASM_GENERAL);
-#undef ASM
+        launch_general<T>(c, a, dim3(c->nblk_asm, 1, c->gz));
     } else {
         return fail(c, FANS_GPU_EINVAL, "linear matvec needs linear materials");
     }
@@ -3984,8 +3409,8 @@ int fans_gpu_set_option(fans_gpu_ctx *c, int32_t opt, int64_t value)
         // than the powers of two 16..256, whose kernels fix their tiles)
         if (value < 8 || value > 64)
             return fail(c, FANS_GPU_EINVAL, "FFT LDS budget must be in [8, 64] KiB");
-        c->fft64.lds_kib = (int) value;
-        c->fft32.lds_kib = (int) value;
+        c->fft64.lds_kib = c->fft32.lds_kib = (int) value;
+        c->fft64.lds_set = c->fft32.lds_set = true;
         if (c->fft64.plan(c->nx, c->ny, c->nz, c->h) != hipSuccess ||
             (c->fft32.twz && c->fft32.plan(c->nx, c->ny, c->nz, c->h) != hipSuccess))
             return fail(c, FANS_GPU_EINVAL, "FFT plan failed");

@@ -1,4 +1,4 @@
-// Small in-register DFT butterflies (radix 2, 3, 4, 5, 8), forward and inverse.
+// In-register DFTs (2 to 24 points), forward and inverse.
 #pragma once
 #include "common.h"
 
@@ -134,5 +134,141 @@ template <>
 __device__ __forceinline__ void dft<float, 8, false>(cplx<float> (&v)[8]) { dft8<float, false>(v); }
 template <>
 __device__ __forceinline__ void dft<float, 8, true>(cplx<float> (&v)[8]) { dft8<float, true>(v); }
+
+// in-register DFT of length 16 as 4 x 4 with constant internal twiddles
+template <typename T, bool INV>
+__device__ __forceinline__ void dft16(cplx<T> (&v)[16])
+{
+    const T c = (T) 0.92387953251128675613, s = (T) 0.38268343236508977173, r = (T) 0.70710678118654752440;
+    cplx<T> y[4][4];
+#pragma unroll
+    for (int i2 = 0; i2 < 4; ++i2) {
+        cplx<T> a[4] = {v[i2], v[i2 + 4], v[i2 + 8], v[i2 + 12]};
+        dft4<T, INV>(a);
+#pragma unroll
+        for (int k1 = 0; k1 < 4; ++k1)
+            y[i2][k1] = a[k1];
+    }
+    // y[i2][k1] *= W16^(i2 k1); forward W16^p = (cos, -sin)(2 pi p / 16)
+    auto tw = [&](cplx<T> a, T wr, T wi) { return INV ? cplx<T>{a.x * wr + a.y * wi, a.y * wr - a.x * wi}
+                                                       : cplx<T>{a.x * wr - a.y * wi, a.x * wi + a.y * wr}; };
+    // (wr, wi) below are the forward twiddles; the lambda conjugates for INV
+    y[1][1] = tw(y[1][1], c, -s);
+    y[1][2] = tw(y[1][2], r, -r);
+    y[1][3] = tw(y[1][3], s, -c);
+    y[2][1] = tw(y[2][1], r, -r);
+    y[2][2] = tw(y[2][2], (T) 0, (T) -1);
+    y[2][3] = tw(y[2][3], -r, -r);
+    y[3][1] = tw(y[3][1], s, -c);
+    y[3][2] = tw(y[3][2], -r, -r);
+    y[3][3] = tw(y[3][3], -c, s);
+#pragma unroll
+    for (int k1 = 0; k1 < 4; ++k1) {
+        cplx<T> a[4] = {y[0][k1], y[1][k1], y[2][k1], y[3][k1]};
+        dft4<T, INV>(a);
+#pragma unroll
+        for (int k2 = 0; k2 < 4; ++k2)
+            v[k1 + 4 * k2] = a[k2];
+    }
+}
+
+// exp(-2 pi i k / n) for compile-time k, n: the angle reduced to a quadrant
+// and a Taylor series there (terms below 1e-20 of the result)
+constexpr double ct_taylor(double x, bool sine)
+{
+    // sin: x - x^3/3! + ...; cos: 1 - x^2/2! + ...
+    double t = sine ? x : 1.0, s = t;
+    for (int m = 1; m < 14; ++m) {
+        const double a = sine ? 2.0 * m : 2.0 * m - 1.0;
+        t *= -x * x / (a * (a + 1.0));
+        s += t;
+    }
+    return s;
+}
+struct CtW {
+    double re, im;
+};
+constexpr CtW ct_twiddle(int k, int n)
+{
+    k %= n;
+    const int    q  = (4 * k) / n;  // quadrant of 2 pi k / n
+    const double r  = 1.57079632679489661923 * (double) (4 * k - q * n) / (double) n;
+    const double cr = ct_taylor(r, false), sr = ct_taylor(r, true);
+    // angle q pi/2 + r: rotate (cos r, sin r) by q quarter turns
+    const double c = q == 0 ? cr : (q == 1 ? -sr : (q == 2 ? -cr : sr));
+    const double s = q == 0 ? sr : (q == 1 ? cr : (q == 2 ? -sr : -cr));
+    return CtW{c, -s};
+}
+
+template <typename T, int N, bool INV>
+__device__ __forceinline__ void dft_reg(cplx<T> (&v)[N]);
+
+// in-register DFT of length P Q by Cooley-Tukey: P-point DFTs over the
+// stride-Q subsequences, the twiddles W_PQ^(i2 k1), Q-point DFTs; input
+// index i2 + Q m, output k1 + P k2 (dft16's order for P = Q = 4)
+template <typename T, int P, int Q, bool INV>
+__device__ __forceinline__ void dft_pq(cplx<T> (&v)[P * Q])
+{
+    cplx<T> y[Q][P];
+#pragma unroll
+    for (int i2 = 0; i2 < Q; ++i2) {
+        cplx<T> a[P];
+#pragma unroll
+        for (int m = 0; m < P; ++m)
+            a[m] = v[i2 + Q * m];
+        dft_reg<T, P, INV>(a);
+#pragma unroll
+        for (int k1 = 0; k1 < P; ++k1) {
+            if (i2 * k1 == 0) {
+                y[i2][k1] = a[k1];
+            } else {
+                constexpr int n = P * Q;
+                const CtW     w = ct_twiddle(i2 * k1, n);
+                const T       wr = (T) w.re, wi = INV ? (T) -w.im : (T) w.im;
+                y[i2][k1]        = cplx<T>{a[k1].x * wr - a[k1].y * wi, a[k1].x * wi + a[k1].y * wr};
+            }
+        }
+    }
+#pragma unroll
+    for (int k1 = 0; k1 < P; ++k1) {
+        cplx<T> b[Q];
+#pragma unroll
+        for (int i2 = 0; i2 < Q; ++i2)
+            b[i2] = y[i2][k1];
+        dft_reg<T, Q, INV>(b);
+#pragma unroll
+        for (int k2 = 0; k2 < Q; ++k2)
+            v[k1 + P * k2] = b[k2];
+    }
+}
+
+template <typename T, int N, bool INV>
+__device__ __forceinline__ void dft_reg(cplx<T> (&v)[N])
+{
+    if constexpr (N == 2 || N == 3 || N == 5)
+        dft<T, N, INV>(v);
+    else if constexpr (N == 4)
+        dft4<T, INV>(v);
+    else if constexpr (N == 8)
+        dft8<T, INV>(v);
+    else if constexpr (N == 16)
+        dft16<T, INV>(v);
+    else if constexpr (N == 6)
+        dft_pq<T, 3, 2, INV>(v);
+    else if constexpr (N == 9)
+        dft_pq<T, 3, 3, INV>(v);
+    else if constexpr (N == 10)
+        dft_pq<T, 5, 2, INV>(v);
+    else if constexpr (N == 12)
+        dft_pq<T, 3, 4, INV>(v);
+    else if constexpr (N == 15)
+        dft_pq<T, 5, 3, INV>(v);
+    else if constexpr (N == 20)
+        dft_pq<T, 5, 4, INV>(v);
+    else {
+        static_assert(N == 24, "unsupported register DFT length");
+        dft_pq<T, 3, 8, INV>(v);
+    }
+}
 
 }  // namespace fans

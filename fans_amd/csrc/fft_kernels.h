@@ -1,4 +1,4 @@
-// LDS-staged Stockham FFT kernels for 3-D r2c / c2r of nodal fields.
+// LDS-staged FFT kernels for 3-D r2c / c2r of nodal fields.
 //
 // Layouts (all row-major, components fastest):
 //   real field      [x][y][z][h]            (T)
@@ -10,21 +10,26 @@
 // pass carries the Green operator multiply between the forward and inverse
 // transforms, so the spectrum is read and written once for that stage.
 //
-// Every stage runs in place in a single LDS tile: each thread first reads all
-// inputs of its butterflies into registers, the block synchronises, then the
-// outputs are written.  Rows of the tile are padded by one complex value so
-// the power-of-two strides of the first stages do not collide in LDS banks.
+// A transform of n = r1 r2 ... rs runs as s in-place stages: forward by
+// decimation in frequency (natural order in, digit-reversed order out), inverse
+// as its exact reversal.  A butterfly reads and writes the same places, so a
+// stage holds no data across a barrier, and one barrier separates two stages.  The
+// strided passes take their first stage from global memory and give their last
+// one to it; the x pass applies the Green operator to the registers of the last
+// forward stage and starts the inverse from them.
 #pragma once
 #include "common.h"
+#include <type_traits>
 #include "fft_butterflies.h"
 
 namespace fans {
 
+constexpr int kMaxStages = 8;
 struct FftLen {
-    int n;        // transform length
-    int nst;      // number of radix stages
-    int tws;      // stride into the twiddle table (table length n * tws)
-    int rad[14];  // radices in application order
+    int n;                // transform length
+    int nst;              // number of radix stages (0 for n = 1)
+    int tws;              // stride into the twiddle table (table length n * tws)
+    int rad[kMaxStages];  // radices in forward order
 };
 
 // Green operator storage, G[(kxq * gyq + kyq) * Mc + kz][H(H+1)/2] packed
@@ -39,82 +44,176 @@ struct GreenView {
     int      nx, ny, gxq, gyq, Mc;
 };
 
-// stored block of frequency (kx, ky, kz) and the mirror signs sx, sy
-template <typename T, int H>
-__device__ __forceinline__ const T *green_at(const GreenView<T> &gv, int kx, int ky, int kz, T &sx, T &sy)
-{
-    const bool fx = kx >= gv.gxq, fy = ky >= gv.gyq;
-    sx            = fx ? (T) -1 : (T) 1;
-    sy            = fy ? (T) -1 : (T) 1;
-    const int kxq = fx ? gv.nx - kx : kx, kyq = fy ? gv.ny - ky : ky;
-    return gv.G + (((int64_t) kxq * gv.gyq + kyq) * gv.Mc + kz) * (H * (H + 1) / 2);
-}
+// Transform lengths (times the components, along z and x) are at most this.
+constexpr int FFT_MAX_ELEMS = 3840;
 
-// Register budget of the in-place stages: a thread holds at most FFT_MAXV
-// complex values; callers keep n * ncols <= FFT_MAXV * 240 so every radix
-// (including 3 and 5, where MAXV/R rounds down) fits.
-constexpr int FFT_MAXV = 16;
-constexpr int FFT_MAX_ELEMS = FFT_MAXV * 240;
-
-// ---- one in-place Stockham radix-R stage over `ncols` independent columns --
-// element (i, col) lives at buf[i * ld + col]
-template <typename T, int R, bool INV>
-__device__ __forceinline__ void stockham_stage(cplx<T> *__restrict__ buf, int n, int ncols, int ld, int Ns,
-                                               const cplx<T> *__restrict__ tw, int tws)
-{
-    constexpr int MB    = FFT_MAXV / R;
-    const int     nb    = n / R;
-    const int     total = nb * ncols;
-    const int     tstep = (n / (Ns * R)) * tws;
-    cplx<T>       v[MB][R];
-#pragma unroll
-    for (int b = 0; b < MB; ++b) {
-        const int w = threadIdx.x + b * blockDim.x;
-        if (w < total) {
-            const int col = w % ncols, j = w / ncols;
-#pragma unroll
-            for (int t = 0; t < R; ++t)
-                v[b][t] = buf[(j + t * nb) * ld + col];
-        }
+// quotient of 0 <= a < 2^20 by a divisor fixed per launch
+struct FastDiv {
+    int   d;
+    float inv;
+    __device__ __forceinline__ explicit FastDiv(int n) : d(n), inv(1.0f / (float) n) {}
+    __device__ __forceinline__ int operator()(int a, int &rem) const
+    {
+        int q = (int) (((float) a + 0.5f) * inv);
+        rem   = a - q * d;
+        return q;
     }
-    __syncthreads();
-#pragma unroll
-    for (int b = 0; b < MB; ++b) {
-        const int w = threadIdx.x + b * blockDim.x;
-        if (w < total) {
-            const int col = w % ncols, j = w / ncols, k = j % Ns;
-            if (Ns > 1) {
-#pragma unroll
-                for (int t = 1; t < R; ++t) {
-                    const cplx<T> wv = tw[t * k * tstep];
-                    v[b][t]          = INV ? cmulc(v[b][t], wv) : cmul(v[b][t], wv);
-                }
-            }
-            dft<T, R, INV>(v[b]);
-            const int o = (j / Ns) * Ns * R + k;
-#pragma unroll
-            for (int t = 0; t < R; ++t)
-                buf[(o + t * Ns) * ld + col] = v[b][t];
-        }
-    }
-    __syncthreads();
-}
+};
 
-// full in-place transform of the LDS tile (ends synchronised)
-template <typename T, bool INV>
-__device__ void lds_fft(cplx<T> *buf, const FftLen &L, const cplx<T> *__restrict__ tw, int ncols, int ld)
+// f(integral_constant<R>) for the stage radix R <= MAXR
+template <int MAXR = 16, typename F>
+__device__ __forceinline__ void with_radix(int R, F &&f)
 {
-    int Ns = 1;
-    for (int s = 0; s < L.nst; ++s) {
-        const int R = L.rad[s];
+    if constexpr (MAXR < 16) {
+        static_assert(MAXR == 12, "largest radix");
         switch (R) {
-        case 2: stockham_stage<T, 2, INV>(buf, L.n, ncols, ld, Ns, tw, L.tws); break;
-        case 3: stockham_stage<T, 3, INV>(buf, L.n, ncols, ld, Ns, tw, L.tws); break;
-        case 4: stockham_stage<T, 4, INV>(buf, L.n, ncols, ld, Ns, tw, L.tws); break;
-        case 5: stockham_stage<T, 5, INV>(buf, L.n, ncols, ld, Ns, tw, L.tws); break;
-        default: stockham_stage<T, 8, INV>(buf, L.n, ncols, ld, Ns, tw, L.tws); break;
+        case 2: f(std::integral_constant<int, 2>{}); break;
+        case 3: f(std::integral_constant<int, 3>{}); break;
+        case 4: f(std::integral_constant<int, 4>{}); break;
+        case 5: f(std::integral_constant<int, 5>{}); break;
+        case 6: f(std::integral_constant<int, 6>{}); break;
+        case 8: f(std::integral_constant<int, 8>{}); break;
+        case 9: f(std::integral_constant<int, 9>{}); break;
+        case 10: f(std::integral_constant<int, 10>{}); break;
+        default: f(std::integral_constant<int, 12>{}); break;
         }
-        Ns *= R;
+        return;
+    }
+    switch (R) {
+    case 2: f(std::integral_constant<int, 2>{}); break;
+    case 3: f(std::integral_constant<int, 3>{}); break;
+    case 4: f(std::integral_constant<int, 4>{}); break;
+    case 5: f(std::integral_constant<int, 5>{}); break;
+    case 6: f(std::integral_constant<int, 6>{}); break;
+    case 8: f(std::integral_constant<int, 8>{}); break;
+    case 9: f(std::integral_constant<int, 9>{}); break;
+    case 10: f(std::integral_constant<int, 10>{}); break;
+    case 12: f(std::integral_constant<int, 12>{}); break;
+    case 15: f(std::integral_constant<int, 15>{}); break;
+    default: f(std::integral_constant<int, 16>{}); break;
+    }
+}
+
+// the same for a transform of a single stage (n = 2, 3 or 5)
+template <typename F>
+__device__ __forceinline__ void with_prime(int R, F &&f)
+{
+    switch (R) {
+    case 2: f(std::integral_constant<int, 2>{}); break;
+    case 3: f(std::integral_constant<int, 3>{}); break;
+    default: f(std::integral_constant<int, 5>{}); break;
+    }
+}
+
+// v[k] *= W_m^(+-i k) with tw the table of W_n and step = (n / m) tws
+template <typename T, int R, bool CONJ>
+__device__ __forceinline__ void stage_twiddle(cplx<T> (&v)[R], const cplx<T> *__restrict__ tw, int i_step)
+{
+#pragma unroll
+    for (int k = 1; k < R; ++k) {
+        const cplx<T> w = tw[k * i_step];
+        v[k]            = CONJ ? cmulc(v[k], w) : cmul(v[k], w);
+    }
+}
+
+// Decimation-in-frequency stage of radix R on sub-transforms of length m (of a
+// transform of length n): element i + t s, s = m / R, of a sub-transform comes
+// from load(place, column) and output k goes to store(place of k, column, k).
+// `place` counts the n elements, ncols columns each; INV conjugates.
+template <typename T, int R, bool INV, typename Load, typename Store>
+__device__ __forceinline__ void dif_stage(int n, int m, const FastDiv &ncols, const cplx<T> *__restrict__ tw, int tws,
+                                          Load load, Store store)
+{
+    const int     s = m / R, total = (n / R) * ncols.d, step = (n / m) * tws;
+    const FastDiv ds(s);
+    for (int w = threadIdx.x; w < total; w += blockDim.x) {
+        int       col, i;
+        const int bi = ncols(w, col), q = ds(bi, i), p0 = q * m + i;
+        cplx<T>   v[R];
+#pragma unroll
+        for (int t = 0; t < R; ++t)
+            v[t] = load(p0 + t * s, col);
+        dft_reg<T, R, INV>(v);
+        if (s > 1)
+            stage_twiddle<T, R, INV>(v, tw, i * step);
+#pragma unroll
+        for (int k = 0; k < R; ++k)
+            store(p0 + k * s, col, v[k]);
+    }
+}
+
+// The reversal of the forward dif_stage (decimation in time, inverse transform)
+template <typename T, int R, typename Load, typename Store>
+__device__ __forceinline__ void dit_stage(int n, int m, const FastDiv &ncols, const cplx<T> *__restrict__ tw, int tws,
+                                          Load load, Store store)
+{
+    const int     s = m / R, total = (n / R) * ncols.d, step = (n / m) * tws;
+    const FastDiv ds(s);
+    for (int w = threadIdx.x; w < total; w += blockDim.x) {
+        int       col, i;
+        const int bi = ncols(w, col), q = ds(bi, i), p0 = q * m + i;
+        cplx<T>   v[R];
+#pragma unroll
+        for (int k = 0; k < R; ++k)
+            v[k] = load(p0 + k * s, col);
+        if (s > 1)
+            stage_twiddle<T, R, true>(v, tw, i * step);
+        dft_reg<T, R, true>(v);
+#pragma unroll
+        for (int t = 0; t < R; ++t)
+            store(p0 + t * s, col, v[t]);
+    }
+}
+
+// frequency of the first output of block q of the last forward stage (the
+// others follow at a distance of n / r_last)
+__device__ __forceinline__ int block_frequency(const FftLen &L, int q)
+{
+    int f = 0;
+    for (int s = L.nst - 2; s > 0; --s) {
+        const int p = q / L.rad[s];
+        f           = q - p * L.rad[s] + L.rad[s] * f;
+        q           = p;
+    }
+    return q + (L.nst > 1 ? L.rad[0] : 1) * f;
+}
+
+// place of frequency k after the forward stages
+__device__ __forceinline__ int frequency_place(const FftLen &L, int k)
+{
+    int p = 0;
+    for (int s = 0; s < L.nst; ++s) {
+        const int q = k / L.rad[s];
+        p           = p * L.rad[s] + (k - q * L.rad[s]);
+        k           = q;
+    }
+    return p;
+}
+
+// all stages in place in LDS, element (place, column) at buf[place * ld + column]
+// (ends synchronised)
+template <typename T, bool INV>
+__device__ __forceinline__ void lds_fft(cplx<T> *buf, const FftLen &L, const cplx<T> *__restrict__ tw, int ncols,
+                                        int ld)
+{
+    const FastDiv nc(ncols);
+    auto          load  = [&](int p, int c) { return buf[p * ld + c]; };
+    auto          store = [&](int p, int c, const cplx<T> &x) { buf[p * ld + c] = x; };
+    int           m     = INV ? 1 : L.n;
+    for (int j = 0; j < L.nst; ++j) {
+        const int R = L.rad[INV ? L.nst - 1 - j : j];
+        if (INV)
+            m *= R;
+        with_radix(R, [&](auto r) {
+            constexpr int RR = decltype(r)::value;
+            if constexpr (INV)
+                dit_stage<T, RR>(L.n, m, nc, tw, L.tws, load, store);
+            else
+                dif_stage<T, RR, false>(L.n, m, nc, tw, L.tws, load, store);
+        });
+        if (!INV)
+            m /= R;
+        __syncthreads();
     }
 }
 
@@ -181,14 +280,18 @@ __device__ __forceinline__ void z_pro_partials(const ProArgs<T> &pa, double a0, 
 // r2c post-processing of the half-length transform Z (in LDS, column col):
 // X[k] = (Z[k] + conj Z[M-k]) / 2 + W^k (Z[k] - conj Z[M-k]) / (2i)
 template <typename T>
+__device__ __forceinline__ cplx<T> r2c_untangle(cplx<T> zk, cplx<T> zc, cplx<T> w)
+{
+    zc              = conjg(zc);
+    const cplx<T> E = cscale(zk + zc, (T) 0.5);
+    const cplx<T> D = cscale(zk - zc, (T) 0.5);
+    return E + cmul(w, cplx<T>{D.y, -D.x});
+}
+template <typename T>
 __device__ __forceinline__ cplx<T> r2c_untangle(const cplx<T> *A, int ld, int col, int k, int M,
                                                 const cplx<T> *__restrict__ tw)
 {
-    const cplx<T> zk = A[(k == M ? 0 : k) * ld + col];
-    const cplx<T> zc = conjg(A[(k == 0 ? 0 : M - k) * ld + col]);
-    const cplx<T> E  = cscale(zk + zc, (T) 0.5);
-    const cplx<T> D  = cscale(zk - zc, (T) 0.5);
-    return E + cmul(tw[k], cplx<T>{D.y, -D.x});
+    return r2c_untangle(A[(k == M ? 0 : k) * ld + col], A[(k == 0 ? 0 : M - k) * ld + col], tw[k]);
 }
 
 // ---- z pass, forward r2c ----------------------------------------------------
@@ -218,6 +321,11 @@ __global__ __launch_bounds__(256) void k_fft_z_r2c(T *__restrict__ in, cplx<T> *
     const int64_t g0    = line0 * nzh;
     T             alpha = (T) 0;
     double        a0    = 0.0;
+    // places of the frequencies, behind the tile
+    unsigned short *const place = reinterpret_cast<unsigned short *>(A + M * (lpb * H + 1));
+    for (int k = threadIdx.x; k < M; k += blockDim.x)
+        place[k] = (unsigned short) frequency_place(LM, k);
+    const FastDiv dz(nzh);
     if constexpr (PRO == PRO_CG)
         alpha = (T) *pa.alpha;
     if constexpr (PRO == PRO_CG && kZGroupRt > 0) {
@@ -239,7 +347,8 @@ __global__ __launch_bounds__(256) void k_fft_z_r2c(T *__restrict__ in, cplx<T> *
             for (int i = 0; i < CH; ++i) {
                 const int e = e0 + i * stp;
                 if (e < tot) {
-                    const int l = e / nzh, rem = e - l * nzh, z = rem / H, c = rem - z * H;
+                    int       rem;
+                    const int l = dz(e, rem), z = rem / H, c = rem - z * H;
                     const T   r = rv[i] - alpha * qv[i];
                     __builtin_nontemporal_store(r, &in[g0 + e]);
                     acc_norm(a0, r, pa.measure);
@@ -250,18 +359,21 @@ __global__ __launch_bounds__(256) void k_fft_z_r2c(T *__restrict__ in, cplx<T> *
         }
     } else {
         for (int e = threadIdx.x; e < nl * nzh; e += blockDim.x) {
-            const int l = e / nzh, rem = e - l * nzh, z = rem / H, c = rem - z * H;
+            int       rem;
+            const int l = dz(e, rem), z = rem / H, c = rem - z * H;
             T        *d = reinterpret_cast<T *>(&A[(z >> 1) * ld + l * H + c]);
             d[z & 1]    = z_load<T, PRO>(in, g0 + e, pa, alpha, a0);
         }
     }
     __syncthreads();
     lds_fft<T, false>(A, LM, tw, ncols, ld);
-    const int Mc  = M + 1;
-    cplx<T>  *dst = out + line0 * Mc * H;
+    const int     Mc  = M + 1;
+    const FastDiv dl(Mc * H);
+    cplx<T>      *dst = out + line0 * Mc * H;
     for (int e = threadIdx.x; e < nl * Mc * H; e += blockDim.x) {
-        const int l = e / (Mc * H), rem = e - l * (Mc * H), k = rem / H, c = rem - k * H;
-        dst[e]      = r2c_untangle(A, ld, l * H + c, k, M, tw);
+        int       rem;
+        const int l = dl(e, rem), k = rem / H, c = rem - k * H, col = l * H + c;
+        dst[e] = r2c_untangle(A[place[k == M ? 0 : k] * ld + col], A[place[k == 0 ? 0 : M - k] * ld + col], tw[k]);
     }
     z_pro_partials<PRO>(pa, a0, red);
 }
@@ -431,9 +543,16 @@ __global__ __launch_bounds__(256) void k_fft_z_c2r(const cplx<T> *__restrict__ i
     const int         nl    = (int) ((nlines - line0) < lpb ? (nlines - line0) : lpb);
     const int         ncols = nl * H, ld = ncols + 1;
     const cplx<T>    *src   = in + line0 * Mc * H;
+    const FastDiv     dl(M * H);
+    // places of the frequencies, behind the tile
+    unsigned short *const place = reinterpret_cast<unsigned short *>(A + M * (lpb * H + 1));
+    for (int k = threadIdx.x; k < M; k += blockDim.x)
+        place[k] = (unsigned short) frequency_place(LM, k);
+    __syncthreads();
     for (int e = threadIdx.x; e < nl * M * H; e += blockDim.x) {
-        const int l = e / (M * H), rem = e - l * (M * H), k = rem / H, c = rem - k * H;
-        A[k * ld + l * H + c] = c2r_tangle<T, H>(src + l * Mc * H + c, k, M, tw);
+        int       rem;
+        const int l = dl(e, rem), k = rem / H, c = rem - k * H;
+        A[place[k] * ld + l * H + c] = c2r_tangle<T, H>(src + l * Mc * H + c, k, M, tw);
     }
     __syncthreads();
     lds_fft<T, true>(A, LM, tw, ncols, ld);
@@ -443,8 +562,10 @@ __global__ __launch_bounds__(256) void k_fft_z_c2r(const cplx<T> *__restrict__ i
     T             beta = (T) 0;
     if constexpr (EPI == EPI_CGD)
         beta = (T) ep.scal[0];
-    auto val_of = [&](int e) {
-        const int     l = e / nzh, rem = e - l * nzh, z = rem / H, c = rem - z * H;
+    const FastDiv dz(nzh);
+    auto          val_of = [&](int e) {
+        int           rem;
+        const int     l = dz(e, rem), z = rem / H, c = rem - z * H;
         const cplx<T> v = A[(z >> 1) * ld + l * H + c];
         return (z & 1) ? v.y : v.x;
     };
@@ -726,9 +847,9 @@ __global__ __launch_bounds__((zct_threads<H, M>())) void k_fft_z_c2r_ct(const cp
 // data[o*ostride + i*sn + b] for i < L.n, b in [c0, c1); block (bx, o) owns
 // columns [c0 + bx*bc, c0 + bx*bc + bc).
 template <typename T, bool INV>
-__global__ __launch_bounds__(256) void k_fft_strided(cplx<T> *__restrict__ data, FftLen L,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_fft_strided(cplx<T> *__restrict__ data, FftLen L,
                                                      const cplx<T> *__restrict__ tw, int64_t sn, int c0, int c1,
-                                                     int64_t ostride, int bc, Slots sl)
+                                                     int64_t ostride, int bc, int nbx, Slots sl)
 {
     const int sb = slot_of(sl);
     if (sb < 0)
@@ -737,20 +858,38 @@ __global__ __launch_bounds__(256) void k_fft_strided(cplx<T> *__restrict__ data,
         data += sb * sl.spec;
     }
     extern __shared__ char smem_raw[];
-    cplx<T>  *A     = reinterpret_cast<cplx<T> *>(smem_raw);
-    const int b0    = c0 + blockIdx.x * bc;
-    const int ncols = (c1 - b0) < bc ? (c1 - b0) : bc, ld = ncols + 1;
-    cplx<T>  *base  = data + (int64_t) blockIdx.y * ostride + b0;
-    for (int w = threadIdx.x; w < L.n * ncols; w += blockDim.x) {
-        const int i = w / ncols, c = w - i * ncols;
-        A[i * ld + c] = base[i * sn + c];
+    cplx<T>      *A     = reinterpret_cast<cplx<T> *>(smem_raw);
+    const int     lb    = xcd_tile_index(blockIdx.x, gridDim.x), bo = lb / nbx, bx = lb - bo * nbx;
+    const int     b0    = c0 + bx * bc;
+    const int     ncols = (c1 - b0) < bc ? (c1 - b0) : bc, n = L.n;
+    cplx<T>      *base  = data + (int64_t) bo * ostride + b0;
+    const FastDiv nc(ncols);
+    auto          from_mem = [&](int p, int c) { return base[p * sn + c]; };
+    auto          from_lds = [&](int p, int c) { return A[p * ncols + c]; };
+    auto          to_lds   = [&](int p, int c, const cplx<T> &x) { A[p * ncols + c] = x; };
+    // a place's frequency: blocks of r_last places, its digits reversed
+    const int     rl = L.rad[L.nst - 1], ds = n / rl;
+    const FastDiv dr(rl);
+    auto          to_mem = [&](int p, int c, const cplx<T> &x) {
+        int       k;
+        const int q = dr(p, k);
+        base[(int64_t) (block_frequency(L, q) + k * ds) * sn + c] = x;
+    };
+    if (L.nst == 1) {
+        with_prime(rl, [&](auto r) { dif_stage<T, decltype(r)::value, INV>(n, n, nc, tw, L.tws, from_mem, to_mem); });
+        return;
     }
+    int m = n;
+    with_radix(L.rad[0], [&](auto r) { dif_stage<T, decltype(r)::value, INV>(n, m, nc, tw, L.tws, from_mem, to_lds); });
+    m /= L.rad[0];
     __syncthreads();
-    lds_fft<T, INV>(A, L, tw, ncols, ld);
-    for (int w = threadIdx.x; w < L.n * ncols; w += blockDim.x) {
-        const int i     = w / ncols, c = w - i * ncols;
-        base[i * sn + c] = A[i * ld + c];
+    for (int s = 1; s < L.nst - 1; ++s) {
+        with_radix(L.rad[s],
+                   [&](auto r) { dif_stage<T, decltype(r)::value, INV>(n, m, nc, tw, L.tws, from_lds, to_lds); });
+        m /= L.rad[s];
+        __syncthreads();
     }
+    with_radix(rl, [&](auto r) { dif_stage<T, decltype(r)::value, INV>(n, m, nc, tw, L.tws, from_lds, to_mem); });
 }
 
 // ---- spectral <r, s> --------------------------------------------------------
@@ -760,15 +899,61 @@ __global__ __launch_bounds__(256) void k_fft_strided(cplx<T> *__restrict__ data,
 // (their mirrors -kz are the complex conjugates) and kz = 0, nz/2 once.
 __device__ __forceinline__ double kz_weight(int kz, int Mc) { return (kz == 0 || kz == Mc - 1) ? 1.0 : 2.0; }
 
-// ---- x pass with the Green operator between forward and inverse ------------
-// spectrum [x][y][kz][H]; block (bx, y) owns kz in [kz_lo + bx*bk, ... + bk) and all H.
-// G packed per frequency [x][y][kz][H(H+1)/2] = (00 01 02 11 12 22) or (0).
-// partial (nullable): one partial of <r, s> (s = -G r) per block, block index
-// blockIdx.y * gridDim.x + blockIdx.x.
+constexpr int kXGreenGroup = 4;
+// largest radix of the x pass: beyond 12 the FP64 pass of three components takes
+// more than 168 registers (two waves per SIMD)
 template <typename T, int H>
-__global__ __launch_bounds__(256) void k_fft_x_green(cplx<T> *__restrict__ data, FftLen L,
+__host__ __device__ constexpr int kXGreenMaxRadix()
+{
+    return sizeof(T) == 8 && H == 3 ? 12 : 16;
+}
+// lane <- lane (quad base + S) for every lane of a quad (DPP quad_perm broadcast)
+template <int S>
+__device__ __forceinline__ double quad_bcast(double x)
+{
+    constexpr int ctrl = S * 0x55;
+    const int     lo   = __builtin_amdgcn_mov_dpp(__double2loint(x), ctrl, 0xf, 0xf, true);
+    const int     hi   = __builtin_amdgcn_mov_dpp(__double2hiint(x), ctrl, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+template <int S>
+__device__ __forceinline__ float quad_bcast(float x)
+{
+    constexpr int ctrl = S * 0x55;
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), ctrl, 0xf, 0xf, true));
+}
+
+// component c of G r at stored block g with mirror signs sx, sy: for H = 3 the
+// components of a frequency sit in the lanes 0..2 of a quad (lane 3 idle: c = 3
+// computes a value nobody reads)
+template <typename T, int H>
+__device__ __forceinline__ cplx<T> green_row(const T *__restrict__ g, T sx, T sy, int c, const cplx<T> &a)
+{
+    if constexpr (H == 1) {
+        return cscale(a, g[0]);
+    } else {
+        // row c of the packed symmetric 3x3 (00 01 02 11 12 22) with the mirror
+        // signs of the xy (sx sy), xz (sx) and yz (sy) entries
+        const int i1 = c == 0 ? 1 : (c == 1 ? 3 : 4), i2 = c == 0 ? 2 : (c == 1 ? 4 : 5), i0 = c < 2 ? c : 2;
+        const T   s0 = c == 0 ? (T) 1 : (c == 1 ? sx * sy : sx);
+        const T   s1 = c == 0 ? sx * sy : (c == 1 ? (T) 1 : sy);
+        const T   s2 = c == 0 ? sx : (c == 1 ? sy : (T) 1);
+        const T   ga = g[i0] * s0, gb = g[i1] * s1, gc = g[i2] * s2;
+        const T   x0 = quad_bcast<0>(a.x), x1 = quad_bcast<1>(a.x), x2 = quad_bcast<2>(a.x);
+        const T   y0 = quad_bcast<0>(a.y), y1 = quad_bcast<1>(a.y), y2 = quad_bcast<2>(a.y);
+        return cplx<T>{ga * x0 + gb * x1 + gc * x2, ga * y0 + gb * y1 + gc * y2};
+    }
+}
+
+// ---- x pass with the Green operator between forward and inverse ------------
+// spectrum [x][y][kz][H]; logical block (bx, y) of the XCD-mapped 1-D grid (nbk
+// ny blocks) owns kz in [kz_lo + bx*bk, ... + bk) and all H.
+// G packed per frequency [x][y][kz][H(H+1)/2] = (00 01 02 11 12 22) or (0).
+// partial (nullable): one partial of <r, s> (s = -G r) per block.
+template <typename T, int H>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_fft_x_green(cplx<T> *__restrict__ data, FftLen L,
                                                      const cplx<T> *__restrict__ tw, GreenView<T> gv, int kz_lo,
-                                                     int kz_hi, int bk, double *__restrict__ partial, Slots sl)
+                                                     int kz_hi, int bk, int nbk, double *__restrict__ partial, Slots sl)
 {
     const int sb = slot_of(sl);
     if (sb < 0)
@@ -778,55 +963,96 @@ __global__ __launch_bounds__(256) void k_fft_x_green(cplx<T> *__restrict__ data,
         gv.G += sb * sl.green;
         partial = slot_ptr(partial, sb * sl.part);
     }
-    const int ny = gv.ny, Mc = gv.Mc;
+    const int         ny = gv.ny, Mc = gv.Mc;
     __shared__ double red[8];
     double            acc = 0.0;
     extern __shared__ char smem_raw[];
-    cplx<T>      *A     = reinterpret_cast<cplx<T> *>(smem_raw);
-    const int     y     = blockIdx.y;
-    const int     kz0   = kz_lo + blockIdx.x * bk;
+    cplx<T>      *A  = reinterpret_cast<cplx<T> *>(smem_raw);
+    const int     lb = xcd_tile_index(blockIdx.x, gridDim.x), yt = lb / nbk, bx = lb - yt * nbk;
+    // ky and its mirror ny - ky read the same quarter-stored Green values: order
+    // the rows 0, 1, ny-1, 2, ny-2, ... so that both run back to back on one XCD
+    const int     y     = yt == 0 ? 0 : ((yt & 1) ? (yt + 1) >> 1 : ny - (yt >> 1));
+    const int     kz0   = kz_lo + bx * bk;
     const int     nk    = (kz_hi - kz0) < bk ? (kz_hi - kz0) : bk;
-    const int     ncols = nk * H, ld = ncols + 1;
+    const int     ncols = nk * H, n = L.n;
     const int64_t sn    = (int64_t) ny * Mc * H;
     cplx<T>      *base  = data + ((int64_t) y * Mc + kz0) * H;
-    for (int w = threadIdx.x; w < L.n * ncols; w += blockDim.x) {
-        const int i = w / ncols, c = w - i * ncols;
-        A[i * ld + c] = base[i * sn + c];
-    }
-    __syncthreads();
-    lds_fft<T, false>(A, L, tw, ncols, ld);
-    for (int w = threadIdx.x; w < L.n * nk; w += blockDim.x) {
-        const int i = w / nk, kk = w - i * nk;
-        T         sx, sy;
-        const T  *g = green_at<T, H>(gv, i, y, kz0 + kk, sx, sy);
-        cplx<T>  *v = A + i * ld + kk * H;
-        const double wk = kz_weight(kz0 + kk, Mc);
-        if constexpr (H == 1) {
-            const cplx<T> a = v[0];
-            v[0]            = cscale(a, g[0]);
-            acc -= wk * ((double) a.x * v[0].x + (double) a.y * v[0].y);
-        } else {
-            const cplx<T> a = v[0], b = v[1], c = v[2];
-            const T       g00 = g[0], g01 = g[1] * sx * sy, g02 = g[2] * sx, g11 = g[3], g12 = g[4] * sy, g22 = g[5];
-            v[0]                = cplx<T>{g00 * a.x + g01 * b.x + g02 * c.x, g00 * a.y + g01 * b.y + g02 * c.y};
-            v[1]                = cplx<T>{g01 * a.x + g11 * b.x + g12 * c.x, g01 * a.y + g11 * b.y + g12 * c.y};
-            v[2]                = cplx<T>{g02 * a.x + g12 * b.x + g22 * c.x, g02 * a.y + g12 * b.y + g22 * c.y};
-            acc -= wk * ((double) a.x * v[0].x + (double) a.y * v[0].y + (double) b.x * v[1].x +
-                         (double) b.y * v[1].y + (double) c.x * v[2].x + (double) c.y * v[2].y);
+    const FastDiv nc(ncols);
+    auto          from_mem = [&](int p, int c) { return base[p * sn + c]; };
+    auto          to_mem   = [&](int p, int c, const cplx<T> &x) { base[p * sn + c] = x; };
+    auto          from_lds = [&](int p, int c) { return A[p * ncols + c]; };
+    auto          to_lds   = [&](int p, int c, const cplx<T> &x) { A[p * ncols + c] = x; };
+    const bool    fy       = y >= gv.gyq;
+    const T       sy       = fy ? (T) -1 : (T) 1;
+    const int     kyq      = fy ? ny - y : y;
+    // last forward stage, Green operator, first inverse stage on one column
+    auto middle = [&](auto r, auto load, auto store) {
+        constexpr int R = decltype(r)::value, HL = H == 3 ? 4 : 1;  // lanes per frequency
+        const FastDiv dk(nk);
+        const int     total = (n / R) * nk * HL, ds = n / R;
+        for (int w = threadIdx.x; w < total; w += 256) {
+            const int c = H == 3 ? w & 3 : 0;
+            int       kk;
+            const int q = dk(H == 3 ? w >> 2 : w, kk);
+            const int col = kk * H + (c < H ? c : 0), kz = kz0 + kk;
+            cplx<T>   v[R];
+#pragma unroll
+            for (int t = 0; t < R; ++t)
+                v[t] = load(q * R + t, col);
+            dft_reg<T, R, false>(v);
+            const int    f  = block_frequency(L, q);
+            const double wk = c < H ? kz_weight(kz, Mc) : 0.0;
+#pragma unroll
+            for (int k = 0; k < R; ++k) {
+                // Green values of kXGreenGroup frequencies at a time: requested
+                // all together they take the kernel past 256 registers
+                if (k > 0 && k % kXGreenGroup == 0)
+                    __builtin_amdgcn_sched_barrier(0);
+                const int     kx = f + k * ds;
+                const bool    fx = kx >= gv.gxq;
+                const T      *g  = gv.G + (((int64_t) (fx ? gv.nx - kx : kx) * gv.gyq + kyq) * Mc + kz) * (H * (H + 1) / 2);
+                const cplx<T> a  = v[k];
+                v[k]             = green_row<T, H>(g, fx ? (T) -1 : (T) 1, sy, c, a);
+                acc -= wk * ((double) a.x * v[k].x + (double) a.y * v[k].y);
+            }
+            dft_reg<T, R, true>(v);
+            if (c < H)
+#pragma unroll
+                for (int t = 0; t < R; ++t)
+                    store(q * R + t, col, v[t]);
         }
-    }
-    __syncthreads();
-    lds_fft<T, true>(A, L, tw, ncols, ld);
-    for (int w = threadIdx.x; w < L.n * ncols; w += blockDim.x) {
-        const int i     = w / ncols, c = w - i * ncols;
-        base[i * sn + c] = A[i * ld + c];
+    };
+    const int rl = L.rad[L.nst - 1];
+    if (L.nst == 1) {
+        with_prime(rl, [&](auto r) { middle(r, from_mem, to_mem); });
+    } else {
+        int m = n;
+        with_radix<kXGreenMaxRadix<T, H>()>(L.rad[0],
+                   [&](auto r) { dif_stage<T, decltype(r)::value, false>(n, m, nc, tw, L.tws, from_mem, to_lds); });
+        m /= L.rad[0];
+        __syncthreads();
+        for (int s = 1; s < L.nst - 1; ++s) {
+            with_radix<kXGreenMaxRadix<T, H>()>(L.rad[s],
+                       [&](auto r) { dif_stage<T, decltype(r)::value, false>(n, m, nc, tw, L.tws, from_lds, to_lds); });
+            m /= L.rad[s];
+            __syncthreads();
+        }
+        with_radix<kXGreenMaxRadix<T, H>()>(rl, [&](auto r) { middle(r, from_lds, to_lds); });
+        __syncthreads();
+        for (int s = L.nst - 2; s > 0; --s) {
+            m *= L.rad[s];
+            with_radix<kXGreenMaxRadix<T, H>()>(L.rad[s],
+                       [&](auto r) { dit_stage<T, decltype(r)::value>(n, m, nc, tw, L.tws, from_lds, to_lds); });
+            __syncthreads();
+        }
+        with_radix<kXGreenMaxRadix<T, H>()>(L.rad[0], [&](auto r) { dit_stage<T, decltype(r)::value>(n, n, nc, tw, L.tws, from_lds, to_mem); });
     }
     if (partial) {
         double     v1[1] = {acc};
         const bool mx[1] = {false};
         block_reduce<1>(v1, mx, red);
         if (threadIdx.x == 0)
-            partial[blockIdx.y * gridDim.x + blockIdx.x] = v1[0];
+            partial[blockIdx.x] = v1[0];
     }
 }
 

@@ -25,9 +25,6 @@ enum {
     SC_ARING    = 32,  // linear CG: alpha of iteration j at SC_ARING + j % kDirRing
     SC_COUNT    = kScSlot
 };
-// linear CG: search directions kept per iteration before the solution update
-// u -= sum alpha_j d_j is applied in one pass
-constexpr int kDirRing = 8;
 // device integer slots: IS_* (common.h)
 
 enum {

@@ -272,9 +272,9 @@ int fans_gpu_stream_bandwidth(int32_t device, int64_t bytes, int32_t reps, doubl
  * fans_gpu_residual (linear_kd=1) run the FP32 kernels of the mixed form's
  * inner solve (input rounded to FP32, output widened; contexts created with
  * FANS_PREC_MIXED only); FANS_OPT_FFT_LDS_KIB=k sets the LDS budget (8..64
- * KiB, default 40) of one workgroup of the generic FFT passes, i.e. their
- * lines or columns per workgroup (lengths other than the powers of two
- * 16..256, whose kernels have fixed tiles); FANS_OPT_MIXED_RESTART=1 makes a
+ * KiB; unset, each pass has its own) of one workgroup of the generic FFT passes,
+ * i.e. their lines or columns per workgroup (lengths other than the powers of
+ * two 16..256, whose kernels have fixed tiles); FANS_OPT_MIXED_RESTART=1 makes a
  * single-RVE context's mixed form restart its FP32 CG in every outer round
  * (default 0: one FP32 CG whose residual is replaced by the true FP64 one at
  * each outer check, as batched contexts also do). */
