@@ -16,6 +16,7 @@
 #include <vector>
 
 #include "assemble_kernels.h"
+#include "cg_scalars.h"
 #include "common.h"
 #include "element_kernels.h"
 #include "fft_kernels.h"
@@ -23,10 +24,6 @@
 namespace fans {
 
 constexpr int kThreads = 256;
-
-// linear CG: search directions kept per iteration before the solution update
-// u -= sum alpha_j d_j is applied in one pass
-constexpr int kDirRing = 8;
 
 // kernel families for the timing report
 enum {
@@ -383,6 +380,12 @@ inline Slots launch_slots(const fans_gpu_ctx *c, bool gated)
     s.is    = gated ? c->is : nullptr;
     return s;
 }
+
+// partials of one kernel up to which the z passes fold the CG scalars themselves:
+// with 2176 (128^3 elastic FP64) the solve went from 9.26 to 9.12 ms, with 2304
+// (144^3 mixed) 10.61 to 10.43; with 2400 (200 x 192 x 160 conduction) from 4.77 to
+// 4.80 and, mixed, 4.01 to 4.17: every workgroup reads all of them
+constexpr int kFoldMax = 2304;
 
 // ---- launches ----------------------------------------------------------------
 // z passes, strided (y or x) pass, x+Green pass; x+Green returns its block count

@@ -270,31 +270,43 @@ int reduce(fans_gpu_ctx *c, const double *partial, int nblk, int nq, int stage, 
 // ---------------------------------------------------------------------------
 // FFT convolution: out = G * r  with the requested epilogue.  With `pro` the
 // forward z pass first applies the previous CG residual update to r and the
-// RED_ERR_NEXT reduction (error, stop test) follows it.
+// RED_ERR_NEXT reduction (error, stop test) follows it.  EPI_CGDF (pro with
+// PRO_CGF): both z passes fold the scalars themselves; `after_z` (nullable) is
+// launched between the z and y passes.
 // ---------------------------------------------------------------------------
 template <typename T>
 int convolve_dev(fans_gpu_ctx *c, Fft3D<T> &P, T *rin, cplx<T> *spec, const T *Gp, int epi, EpiArgs<T> ep,
-                 const int *done, const ProArgs<T> *pro = nullptr)
+                 const int *done, const ProArgs<T> *pro = nullptr, const std::function<int()> &after_z = nullptr)
 {
-    const int h = c->h, Kc = P.Mc * h;
+    const int  h = c->h, Kc = P.Mc * h;
+    const bool fold = epi == EPI_CGDF;
     {
         Timed            t(c, pro ? KF_CG_FFT_Z_FWD : KF_FFT_Z_FWD);
         const ProArgs<T> pa = pro ? *pro : ProArgs<T>{};
         if (h == 1) {
-            if (pro)
+            if (pro && fold)
+                launch_z_r2c<T, 1, PRO_CGF>(c, P, rin, spec, pa, done);
+            else if (pro)
                 launch_z_r2c<T, 1, PRO_CG>(c, P, rin, spec, pa, done);
             else
                 launch_z_r2c<T, 1, PRO_NONE>(c, P, rin, spec, pa, done);
         } else {
-            if (pro)
+            if (pro && fold)
+                launch_z_r2c<T, 3, PRO_CGF>(c, P, rin, spec, pa, done);
+            else if (pro)
                 launch_z_r2c<T, 3, PRO_CG>(c, P, rin, spec, pa, done);
             else
                 launch_z_r2c<T, 3, PRO_NONE>(c, P, rin, spec, pa, done);
         }
     }
     HIPCHK(c, hipGetLastError());
-    if (pro) {
+    if (pro && !fold) {
         const int rc = reduce(c, pro->partial, (int) P.nblk_z, 1, RED_ERR_NEXT);
+        if (rc)
+            return rc;
+    }
+    if (after_z) {
+        const int rc = after_z();
         if (rc)
             return rc;
     }
@@ -304,7 +316,7 @@ int convolve_dev(fans_gpu_ctx *c, Fft3D<T> &P, T *rin, cplx<T> *spec, const T *G
     const int nch = std::max(1, std::min(c->fft_chunks, P.Mc));
     // EPI_CGD: delta = <r, s> from the spectrum (x+Green partials), then
     // beta (RED_DELTA) before the inverse z pass forms d = s + beta d_prev
-    double *const xg_partial = c->partial;
+    double *const xg_partial = fold ? const_cast<double *>(ep.fold.p1) : c->partial;
     int           xg_blocks  = 0;
     for (int q = 0; q < nch; ++q) {
         const int kz_lo = (int) ((int64_t) P.Mc * q / nch), kz_hi = (int) ((int64_t) P.Mc * (q + 1) / nch);
@@ -316,7 +328,7 @@ int convolve_dev(fans_gpu_ctx *c, Fft3D<T> &P, T *rin, cplx<T> *spec, const T *G
         }
         {
             Timed   t(c, KF_FFT_X_GREEN);
-            double *xp = epi == EPI_CGD ? xg_partial + xg_blocks : nullptr;
+            double *xp = epi_cgd(epi) ? xg_partial + xg_blocks : nullptr;
             xg_blocks += h == 1 ? launch_x_green<T, 1>(c, P, spec, Gp, kz_lo, kz_hi, xp, done)
                                 : launch_x_green<T, 3>(c, P, spec, Gp, kz_lo, kz_hi, xp, done);
         }
@@ -341,6 +353,8 @@ int convolve_dev(fans_gpu_ctx *c, Fft3D<T> &P, T *rin, cplx<T> *spec, const T *G
                 launch_z_c2r<T, 1, EPI_CG>(c, P, spec, ep, done);
             else if (epi == EPI_CGD)
                 launch_z_c2r<T, 1, EPI_CGD>(c, P, spec, ep, done);
+            else if (epi == EPI_CGDF)
+                launch_z_c2r<T, 1, EPI_CGDF>(c, P, spec, ep, done);
             else
                 launch_z_c2r<T, 1, EPI_FP>(c, P, spec, ep, done);
         } else {
@@ -350,6 +364,8 @@ int convolve_dev(fans_gpu_ctx *c, Fft3D<T> &P, T *rin, cplx<T> *spec, const T *G
                 launch_z_c2r<T, 3, EPI_CG>(c, P, spec, ep, done);
             else if (epi == EPI_CGD)
                 launch_z_c2r<T, 3, EPI_CGD>(c, P, spec, ep, done);
+            else if (epi == EPI_CGDF)
+                launch_z_c2r<T, 3, EPI_CGDF>(c, P, spec, ep, done);
             else
                 launch_z_c2r<T, 3, EPI_FP>(c, P, spec, ep, done);
         }
@@ -751,7 +767,11 @@ void host_sym_pinv(int n, const double *A, double *P)
 // one pass reading kDirRing directions instead of a read-modify-write of u per
 // iteration.  After RED_ERR_NEXT sets `done` every later kernel returns at
 // entry; r then holds the final residual and finish() applies the directions
-// left in the ring.  ring[kDirRing - 1] must hold zeros on entry (d_(-1) = 0).
+// left in the ring.  On small grids (kFoldMax) there are no reduction launches:
+// z r2c forms alpha_(j-1), z c2r the error, the stop test and beta, so that the
+// y and x+Green passes of the stopping iteration run to no purpose, and the
+// solution update follows the next iteration's forward z pass.
+// ring[kDirRing - 1] must hold zeros on entry (d_(-1) = 0).
 // integer scalars of every slot of a batched context (fields at slot 0)
 int read_is_all(fans_gpu_ctx *c, std::vector<int> &is)
 {
@@ -780,6 +800,12 @@ int cg_linear_loop(fans_gpu_ctx *c, Fft3D<T> &P, T *r, T *const *ring, T *rnew, 
     int                    is[IS_COUNT];
     std::vector<int>       isall;
     bool                   stop = false;
+    // few enough partials: the z passes fold the scalars (no reduction launches).
+    // The partials of the matvec, the forward z pass and x+Green then lie one
+    // after the other in `partial`, each kept until its consumer has run.
+    const int64_t nz_p = P.nblk_z, nx_p = x_green_blocks(P, c->h, c->ny);
+    const bool    fold = std::max<int64_t>({c->nblk_asm, nz_p, nx_p}) <= kFoldMax && c->fft_chunks <= 1 &&
+                      c->nblk_asm + nz_p + nx_p <= c->partial_len;
     // u -= alpha_m d_m for the ring slots 0 .. count-1 (iterations filled in
     // order); count < 0: each RVE slot's pending count; gated: finished RVE
     // slots skip it
@@ -841,7 +867,8 @@ int cg_linear_loop(fans_gpu_ctx *c, Fft3D<T> &P, T *r, T *const *ring, T *rnew, 
     auto iteration = [&](int j, bool with_pro) -> int {
         T *const         dprev    = ring[(j + kDirRing - 1) % kDirRing];
         T *const         dnext    = ring[j % kDirRing];
-        const ProArgs<T> pa{rnew, c->sc + SC_ALPHA, c->d.measure, c->partial};
+        double *const    err_partial = fold ? c->partial + c->nblk_asm : c->partial;
+        ProArgs<T>       pa{rnew, c->sc + SC_ALPHA, c->d.measure, err_partial, CgFold{}};
         // delta and beta from the spectrum, then d = s + beta d_prev in the
         // inverse z pass, with <d, K d_prev> (read after the matvec); the first
         // iteration has d_prev = 0, and rnew holds no K d_prev yet
@@ -851,8 +878,19 @@ int cg_linear_loop(fans_gpu_ctx *c, Fft3D<T> &P, T *r, T *const *ring, T *rnew, 
         ep.qprev   = j > 0 ? rnew : nullptr;
         ep.dnext   = dnext;
         ep.scal    = c->sc;  // SC_BETA == 0
+        // folded, alpha of the iteration that fills the ring's last slot is known
+        // after the next forward z pass
+        std::function<int()> ring_full;
+        if (fold) {
+            pa.fold = CgFold{c->partial, c->partial_e, c->nblk_asm, (int) nz_p, c->sc, c->is, c->hist, c->d.measure};
+            ep.fold = CgFold{err_partial, err_partial + nz_p, with_pro ? (int) nz_p : 0, (int) nx_p,
+                             c->sc,       c->is,              c->hist,                    c->d.measure};
+            if (with_pro && j % kDirRing == 0)
+                ring_full = [&] { return ring_update(kDirRing, true); };
+        }
         int e;
-        if ((e = convolve_dev<T>(c, P, r, spec, Gp, EPI_CGD, ep, done, with_pro ? &pa : nullptr)))
+        if ((e = convolve_dev<T>(c, P, r, spec, Gp, fold ? EPI_CGDF : EPI_CGD, ep, done, with_pro ? &pa : nullptr,
+                                 ring_full)))
             return e;
         // rnew = K d, <d, rnew>
         AsmArgs<T> a = asm_args<T>(c);
@@ -862,6 +900,8 @@ int cg_linear_loop(fans_gpu_ctx *c, Fft3D<T> &P, T *r, T *const *ring, T *rnew, 
         a.sl         = launch_slots(c, true);
         if ((e = launch_assemble<T, ASM_CGLIN>(c, a)))
             return e;
+        if (fold)
+            return 0;
         // quantity 1, <d, K d_prev>, is zero in the first iteration
         if ((e = reduce(c, c->partial, c->nblk_asm, j > 0 ? 2 : 1, RED_ALPHA, j > 0 ? c->partial_e : nullptr,
                         (int) P.nblk_z)))
@@ -929,9 +969,10 @@ int cg_linear_loop(fans_gpu_ctx *c, Fft3D<T> &P, T *r, T *const *ring, T *rnew, 
                 if ((rc = read_scalars(c, nullptr, is)))
                     return rc;
                 // done was set by this iteration's RED_ERR_NEXT (the fused update
-                // and that reduction did work) or before it (nothing did)
+                // and that reduction did work), by its inverse z pass (every pass
+                // before it did) or before it (nothing did)
                 if (is[IS_DONE])
-                    drop_timing(c, j > j0 ? mark + 2 : mark);
+                    drop_timing(c, j <= j0 ? mark : !fold ? mark + 2 : mark + (j % kDirRing ? 4 : 5));
             }
         }
         if ((rc = poll()))

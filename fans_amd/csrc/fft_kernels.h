@@ -18,6 +18,7 @@
 // one to it; the x pass applies the Green operator to the registers of the last
 // forward stage and starts the inverse from them.
 #pragma once
+#include "cg_scalars.h"
 #include "common.h"
 #include <type_traits>
 #include "fft_butterflies.h"
@@ -225,7 +226,8 @@ __device__ __forceinline__ void lds_fft(cplx<T> *buf, const FftLen &L, const cpl
 // needs no s here: the CG scalars form it from <d, K d> (matvec) and
 // <d, K d_prev> (inverse z pass).  The matching solution update u -= alpha d
 // runs in the inverse z pass of the next iteration, which reads that d anyway.
-enum { PRO_NONE = 0, PRO_CG = 1 };
+// PRO_CGF: alpha, that reduction and the one before it from the partials (CgFold).
+enum { PRO_NONE = 0, PRO_CG = 1, PRO_CGF = 2 };
 
 template <typename T>
 struct ProArgs {
@@ -233,6 +235,7 @@ struct ProArgs {
     const double *alpha;    // device scalar
     int           measure;  // 0 L1, 1 L2, 2 Linf
     double       *partial;  // [gridDim.x]
+    CgFold        fold;     // PRO_CGF
 };
 
 // Loads a thread issues together before the stores that follow them in the
@@ -252,7 +255,7 @@ constexpr int kZGroupRt = FANS_Z_GROUP_RT;
 template <typename T, int PRO>
 __device__ __forceinline__ T z_load(T *__restrict__ in, int64_t gi, const ProArgs<T> &pa, T alpha, double &a0)
 {
-    if constexpr (PRO == PRO_CG) {
+    if constexpr (PRO != PRO_NONE) {
         // r and rnew are not read again before the spectrum passes that
         // follow: streaming (non-temporal) accesses keep them from displacing
         // the freshly written spectrum in the Infinity Cache
@@ -268,7 +271,7 @@ __device__ __forceinline__ T z_load(T *__restrict__ in, int64_t gi, const ProArg
 template <int PRO, typename T>
 __device__ __forceinline__ void z_pro_partials(const ProArgs<T> &pa, double a0, double *red)
 {
-    if constexpr (PRO == PRO_CG) {
+    if constexpr (PRO != PRO_NONE) {
         double     v[1]  = {a0};
         const bool mx[1] = {pa.measure == 2};
         block_reduce<1>(v, mx, red);
@@ -328,7 +331,9 @@ __global__ __launch_bounds__(256) void k_fft_z_r2c(T *__restrict__ in, cplx<T> *
     const FastDiv dz(nzh);
     if constexpr (PRO == PRO_CG)
         alpha = (T) *pa.alpha;
-    if constexpr (PRO == PRO_CG && kZGroupRt > 0) {
+    if constexpr (PRO == PRO_CGF)
+        alpha = (T) fold_alpha<256>(pa.fold, red);
+    if constexpr (PRO != PRO_NONE && kZGroupRt > 0) {
         // r -= alpha K d in groups (same arithmetic and order as z_load)
         constexpr int CH = kZGroupRt;
         const int     tot = nl * nzh, stp = blockDim.x;
@@ -383,8 +388,10 @@ __global__ __launch_bounds__(256) void k_fft_z_r2c(T *__restrict__ in, cplx<T> *
 // d = s + beta d_prev with s = -result (beta from the spectral <r, s> of the x
 // pass); s itself is not stored.  With qprev = K d_prev (the previous matvec's
 // output) it emits per block the partial <d, K d_prev>, from which the CG
-// scalars form the next deltamid.
-enum { EPI_STORE = 0, EPI_CG = 1, EPI_FP = 2, EPI_CGD = 3 };
+// scalars form the next deltamid.  EPI_CGDF: the same with beta, and before it
+// the error and the stop test, from the partials (CgFold).
+enum { EPI_STORE = 0, EPI_CG = 1, EPI_FP = 2, EPI_CGD = 3, EPI_CGDF = 4 };
+constexpr bool epi_cgd(int epi) { return epi == EPI_CGD || epi == EPI_CGDF; }
 
 template <typename T>
 struct EpiArgs {
@@ -396,6 +403,7 @@ struct EpiArgs {
     const T      *qprev;    // EPI_CGD: K d_prev (nullable), partial <d, K d_prev>
     T            *dnext;    // EPI_CGD: new direction (written)
     const double *scal;     // EPI_CGD: device scalars (beta at [0])
+    CgFold        fold;     // EPI_CGDF
 };
 
 // the argument blocks at RVE slot sb
@@ -405,6 +413,7 @@ __device__ __forceinline__ void slot_pro(ProArgs<T> &pa, int sb, const Slots &sl
     pa.rnew    = slot_ptr(pa.rnew, sb * sl.field);
     pa.alpha   = slot_ptr(pa.alpha, (int64_t) sb * kScSlot);
     pa.partial = slot_ptr(pa.partial, sb * sl.part);
+    slot_fold(pa.fold, sb, sl);
 }
 template <typename T>
 __device__ __forceinline__ void slot_epi(EpiArgs<T> &ep, int sb, const Slots &sl)
@@ -417,6 +426,7 @@ __device__ __forceinline__ void slot_epi(EpiArgs<T> &ep, int sb, const Slots &sl
     ep.qprev   = slot_ptr(ep.qprev, sb * sl.field);
     ep.dnext   = slot_ptr(ep.dnext, sb * sl.field);
     ep.scal    = slot_ptr(ep.scal, (int64_t) sb * kScSlot);
+    slot_fold(ep.fold, sb, sl);
 }
 
 // c2r pre-processing of one (line, component): `line` points at kz = 0 of the
@@ -437,7 +447,7 @@ __device__ __forceinline__ void z_epilogue(const EpiArgs<T> &ep, int64_t gi, T v
 {
     if constexpr (EPI == EPI_STORE) {
         ep.out[gi] = val;
-    } else if constexpr (EPI == EPI_CGD) {
+    } else if constexpr (epi_cgd(EPI)) {
         // d_next is read by the very next pass (the matvec) and stays cached;
         // d_prev and u stream past the caches
         const T dp = __builtin_nontemporal_load(&ep.dprev[gi]);
@@ -475,7 +485,7 @@ __device__ __forceinline__ void z_epilogue_grouped(const EpiArgs<T> &ep, int64_t
             pa[i] = pb[i] = (T) 0;
             pu[i]         = 0.0;
             if (e < tot) {
-                if constexpr (EPI == EPI_CGD) {
+                if constexpr (epi_cgd(EPI)) {
                     pa[i] = __builtin_nontemporal_load(&ep.dprev[gi]);
                     if (ep.qprev)
                         pb[i] = __builtin_nontemporal_load(&ep.qprev[gi]);
@@ -494,7 +504,7 @@ __device__ __forceinline__ void z_epilogue_grouped(const EpiArgs<T> &ep, int64_t
                 const T val = val_of(e);
                 if constexpr (EPI == EPI_STORE) {
                     ep.out[gi] = val;
-                } else if constexpr (EPI == EPI_CGD) {
+                } else if constexpr (epi_cgd(EPI)) {
                     const T dn   = beta * pa[i] - val;
                     ep.dnext[gi] = dn;
                     if (ep.qprev)
@@ -514,7 +524,8 @@ __device__ __forceinline__ void z_epilogue_grouped(const EpiArgs<T> &ep, int64_t
 template <int EPI, typename T>
 __device__ __forceinline__ void z_epi_partials(const EpiArgs<T> &ep, double acc, double *red)
 {
-    if (EPI == EPI_CG || (EPI == EPI_CGD && ep.qprev)) {
+    // (EPI_CGDF: also without qprev, a zero, which the next launch folds)
+    if (EPI == EPI_CG || EPI == EPI_CGDF || (EPI == EPI_CGD && ep.qprev)) {
         double     v[1]  = {acc};
         const bool mx[1] = {false};
         block_reduce<1>(v, mx, red);
@@ -544,6 +555,9 @@ __global__ __launch_bounds__(256) void k_fft_z_c2r(const cplx<T> *__restrict__ i
     const int         ncols = nl * H, ld = ncols + 1;
     const cplx<T>    *src   = in + line0 * Mc * H;
     const FastDiv     dl(M * H);
+    FoldBeta          fb;
+    if constexpr (EPI == EPI_CGDF)
+        fb.template load<256>(ep.fold);
     // places of the frequencies, behind the tile
     unsigned short *const place = reinterpret_cast<unsigned short *>(A + M * (lpb * H + 1));
     for (int k = threadIdx.x; k < M; k += blockDim.x)
@@ -562,6 +576,12 @@ __global__ __launch_bounds__(256) void k_fft_z_c2r(const cplx<T> *__restrict__ i
     T             beta = (T) 0;
     if constexpr (EPI == EPI_CGD)
         beta = (T) ep.scal[0];
+    if constexpr (EPI == EPI_CGDF) {
+        double b;
+        if (!fb.template finish<256>(ep.fold, red, b))
+            return;
+        beta = (T) b;
+    }
     const FastDiv dz(nzh);
     auto          val_of = [&](int e) {
         int           rem;
@@ -704,16 +724,18 @@ __global__ __launch_bounds__((zct_threads<H, M>())) void k_fft_z_r2c_ct(T *__res
     constexpr int NT = zct_threads<H, M>(), LPB = zct_lpb<H, M>();
     constexpr int NZH = 2 * M * H, NC = LPB * H, LD = NC + 1, MC = M + 1;
     __shared__ cplx<T> A[M * LD];
-    __shared__ double  red[NT / 64 + 1];
+    __shared__ double  red[2 * ((NT + 63) / 64)];
     const int64_t      line0 = (int64_t) blockIdx.x * LPB;
     const int64_t      g0    = line0 * NZH;
     T                  alpha = (T) 0;
     double             a0    = 0.0;
     if constexpr (PRO == PRO_CG)
         alpha = (T) *pa.alpha;
+    if constexpr (PRO == PRO_CGF)
+        alpha = (T) fold_alpha<NT>(pa.fold, red);
     constexpr int PER = (LPB * NZH) / NT;
     constexpr int CH  = kZGroup < PER ? kZGroup : PER;
-    if constexpr (PRO == PRO_CG && kZGroup > 0 && (LPB * NZH) % NT == 0 && PER % CH == 0) {
+    if constexpr (PRO != PRO_NONE && kZGroup > 0 && (LPB * NZH) % NT == 0 && PER % CH == 0) {
         // r -= alpha K d in groups of CH elements: the loads of a group are in
         // flight together (same arithmetic and accumulation order as z_load)
         for (int i0 = 0; i0 < PER; i0 += CH) {
@@ -769,7 +791,7 @@ __global__ __launch_bounds__((zct_threads<H, M>())) void k_fft_z_c2r_ct(const cp
     constexpr int NT = zct_threads<H, M>(), LPB = zct_lpb<H, M>();
     constexpr int NZH = 2 * M * H, NC = LPB * H, LD = NC + 1, MC = M + 1;
     __shared__ cplx<T> A[M * LD];
-    __shared__ double  red[NT / 64 + 1];
+    __shared__ double  red[2 * ((NT + 63) / 64)];
     const int64_t      line0 = (int64_t) blockIdx.x * LPB;
     const cplx<T>     *src   = in + line0 * MC * H;
     const int64_t      g0    = line0 * NZH;
@@ -778,9 +800,12 @@ __global__ __launch_bounds__((zct_threads<H, M>())) void k_fft_z_c2r_ct(const cp
     // at the cost of registers during it
     constexpr int  PER   = (LPB * NZH) / NT;
     constexpr int  AHEAD = sizeof(T) == 8 ? kC2rAhead64 : kC2rAhead32;
-    constexpr bool PRE   = EPI == EPI_CGD && (LPB * NZH) % NT == 0;
+    constexpr bool PRE   = epi_cgd(EPI) && (LPB * NZH) % NT == 0;
     constexpr bool PRED = PRE && AHEAD >= 1, PREQ = PRE && AHEAD >= 2;
     T              dpv[PRE ? PER : 1], qpv[PRE ? PER : 1];
+    FoldBeta       fb;
+    if constexpr (EPI == EPI_CGDF)
+        fb.template load<NT>(ep.fold);
     if constexpr (PRED) {
         const T *__restrict__ dp = ep.dprev;
         const T *__restrict__ qp = ep.qprev;
@@ -802,6 +827,12 @@ __global__ __launch_bounds__((zct_threads<H, M>())) void k_fft_z_c2r_ct(const cp
     T      beta = (T) 0;
     if constexpr (EPI == EPI_CGD)
         beta = (T) ep.scal[0];
+    if constexpr (EPI == EPI_CGDF) {
+        double b;
+        if (!fb.template finish<NT>(ep.fold, red, b))
+            return;
+        beta = (T) b;
+    }
     if constexpr (PRE) {
         T *__restrict__ dn = ep.dnext;
         // the operands not requested ahead: all of this thread's values are

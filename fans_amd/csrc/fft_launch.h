@@ -201,10 +201,13 @@ void launch_z_c2r(fans_gpu_ctx *c, Fft3D<T> &P, const cplx<T> *spec, const EpiAr
                                                const int *);                                                      \
     template void launch_z_r2c<T, H, PRO_CG>(fans_gpu_ctx *, Fft3D<T> &, T *, cplx<T> *, const ProArgs<T> &,       \
                                              const int *);                                                        \
+    template void launch_z_r2c<T, H, PRO_CGF>(fans_gpu_ctx *, Fft3D<T> &, T *, cplx<T> *, const ProArgs<T> &,      \
+                                              const int *);                                                       \
     FANS_FFT_INSTANCES_C2R(T, H, EPI_STORE)                                                                       \
     FANS_FFT_INSTANCES_C2R(T, H, EPI_CG)                                                                          \
     FANS_FFT_INSTANCES_C2R(T, H, EPI_FP)                                                                          \
-    FANS_FFT_INSTANCES_C2R(T, H, EPI_CGD)
+    FANS_FFT_INSTANCES_C2R(T, H, EPI_CGD)                                                                         \
+    FANS_FFT_INSTANCES_C2R(T, H, EPI_CGDF)
 #define FANS_FFT_INSTANCES_C2R(T, H, EPI)                                                                         \
     template void launch_z_c2r<T, H, EPI>(fans_gpu_ctx *, Fft3D<T> &, const cplx<T> *, const EpiArgs<T> &, const int *);
 

@@ -6,26 +6,10 @@
 // launch geometry of every streaming kernel is fixed per problem size, so all
 // sums are bitwise reproducible from run to run.
 #pragma once
+#include "cg_scalars.h"
 #include "common.h"
 
 namespace fans {
-
-// device scalar slots (double) -- layout shared with the host
-enum {
-    SC_BETA     = 0,
-    SC_ALPHA    = 1,
-    SC_DELTA    = 2,
-    SC_DELTA0   = 3,
-    SC_DELTAMID = 4,
-    SC_ERR      = 5,
-    SC_ERR0     = 6,
-    SC_DN       = 7,
-    SC_TOL      = 8,
-    SC_RES0     = 16,  // generic reduction results [16, 32)
-    SC_ARING    = 32,  // linear CG: alpha of iteration j at SC_ARING + j % kDirRing
-    SC_COUNT    = kScSlot
-};
-// device integer slots: IS_* (common.h)
 
 enum {
     RED_ERR_INIT = 0,  // q0 = norm partials      -> err0, iter = 0, delta = 1, deltamid = 0
@@ -35,35 +19,6 @@ enum {
     RED_SUM      = 5,  // q0..q(nq-1) sums        -> SC_RES0 + q
     RED_ERR_SET  = 6   // q0 = norm partials      -> err, stop test (iteration and CG scalars kept)
 };
-
-__device__ __forceinline__ double finish_norm(double v, int measure) { return measure == 1 ? sqrt(v) : v; }
-
-// The scalars a reduction stage reads, loaded before its first store (the
-// compiler cannot tell the stores to sc / is / hist from those loads, so it
-// would keep each load behind the stores before it: one round trip each).
-struct StageScalars {
-    int    iter, errtype, nit;
-    double delta, deltamid, beta, err0, tol;
-};
-__device__ __forceinline__ StageScalars load_stage_scalars(const double *sc, const int *is)
-{
-    return StageScalars{is[IS_ITER],     is[IS_ERRTYPE], is[IS_NIT], sc[SC_DELTA], sc[SC_DELTAMID],
-                        sc[SC_BETA],     sc[SC_ERR0],    sc[SC_TOL]};
-}
-
-// records the error of iteration it and sets done if the loop condition of
-// solverCG.h:84 / solverFP.h:221 fails
-__device__ __forceinline__ void record_error(double *sc, int *is, double *hist, const StageScalars &S, int it,
-                                             double err)
-{
-    hist[it] = err;
-    if (it == 0)
-        sc[SC_ERR0] = err;
-    sc[SC_ERR]           = err;
-    const double err_rel = it == 0 ? 100.0 : err / S.err0;
-    const double e       = S.errtype == 0 ? err : err_rel;
-    is[IS_DONE]          = !(it < S.nit && e > S.tol);
-}
 
 // one block of kReduceThreads; each thread folds its strided partials into
 // four independent accumulators (fixed order) before the block reduction
@@ -126,21 +81,19 @@ __global__ __launch_bounds__(kReduceThreads) void k_reduce(const double *__restr
                 if (stage == RED_ERR_INIT) {
                     is[IS_ITER]     = 0;
                     sc[SC_DELTA]    = 1.0;
+                    sc[SC_DELTA0]   = 1.0;
                     sc[SC_DELTAMID] = 0.0;
                     record_error(sc, is, hist, S, 0, finish_norm(v[0], measure));
                 } else if (stage == RED_DELTA) {
                     sc[SC_DELTA0] = S.delta;
                     sc[SC_DELTA]  = v[0];
-                    sc[SC_BETA]   = fmax(0.0, (v[0] - S.deltamid) / S.delta);
+                    sc[SC_BETA]   = cg_beta(v[0], S.deltamid, S.delta);
                 } else if (stage == RED_ALPHA) {
-                    const double alpha                = S.delta / v[0];
-                    sc[SC_DN]                         = v[0];
-                    sc[SC_ALPHA]                      = alpha;
+                    const double alpha               = cg_alpha(S.delta, v[0]);
+                    sc[SC_DN]                        = v[0];
+                    sc[SC_ALPHA]                     = alpha;
                     sc[SC_ARING + S.iter % kDirRing] = alpha;
-                    // deltamid of the next iteration, <r - alpha K d, s> with
-                    // s = d - beta d_prev (solverCG.h:87, 91 and 104):
-                    // delta - alpha (<d, K d> - beta <K d_prev, d>), K symmetric
-                    sc[SC_DELTAMID] = S.delta - alpha * (v[0] - S.beta * v[1]);
+                    sc[SC_DELTAMID]                  = cg_deltamid(S.delta, S.beta, alpha, v[0], v[1]);
                 } else if (stage == RED_ERR_NEXT) {
                     is[IS_ITER] = S.iter + 1;
                     record_error(sc, is, hist, S, S.iter + 1, finish_norm(v[0], measure));
