@@ -1,9 +1,6 @@
-// Assembly launches in float.
+// Assembly launches in float, k_assemble.
 #include "assemble_launch.h"
 
 namespace fans {
-template void launch_modal<float, 1, 8, ASM_CGLIN>(fans_gpu_ctx *, const AsmArgs<float> &, dim3);
-template void launch_modal<float, 1, 1, ASM_CGLIN>(fans_gpu_ctx *, const AsmArgs<float> &, dim3);
-template void launch_modal<float, 3, 8, ASM_CGLIN>(fans_gpu_ctx *, const AsmArgs<float> &, dim3);
-template void launch_modal<float, 3, 1, ASM_CGLIN>(fans_gpu_ctx *, const AsmArgs<float> &, dim3);
+template void launch_general<float, ASM_CGLIN>(fans_gpu_ctx *, const AsmArgs<float> &, dim3);
 }

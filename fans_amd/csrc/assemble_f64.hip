@@ -1,14 +1,7 @@
-// Assembly launches in double.
+// Assembly launches in double, k_assemble.
 #include "assemble_launch.h"
 
 namespace fans {
-template void launch_modal<double, 1, 8, ASM_CGLIN>(fans_gpu_ctx *, const AsmArgs<double> &, dim3);
-template void launch_modal<double, 1, 1, ASM_CGLIN>(fans_gpu_ctx *, const AsmArgs<double> &, dim3);
-template void launch_modal<double, 3, 8, ASM_CGLIN>(fans_gpu_ctx *, const AsmArgs<double> &, dim3);
-template void launch_modal<double, 3, 1, ASM_CGLIN>(fans_gpu_ctx *, const AsmArgs<double> &, dim3);
-template void launch_modal<double, 1, 8, ASM_RESID>(fans_gpu_ctx *, const AsmArgs<double> &, dim3);
-template void launch_modal<double, 1, 1, ASM_RESID>(fans_gpu_ctx *, const AsmArgs<double> &, dim3);
-template void launch_modal<double, 3, 8, ASM_RESID>(fans_gpu_ctx *, const AsmArgs<double> &, dim3);
-template void launch_modal<double, 3, 1, ASM_RESID>(fans_gpu_ctx *, const AsmArgs<double> &, dim3);
-template void launch_general<double>(fans_gpu_ctx *, const AsmArgs<double> &, dim3);
+template void launch_general<double, ASM_CGLIN>(fans_gpu_ctx *, const AsmArgs<double> &, dim3);
+template void launch_general<double, ASM_RESID>(fans_gpu_ctx *, const AsmArgs<double> &, dim3);
 }

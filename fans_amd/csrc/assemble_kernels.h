@@ -8,7 +8,7 @@
 // node is produced by exactly one thread in a fixed summation order, so results
 // are deterministic and atomic-free.
 //
-// k_assemble_modal (linear materials): works on Walsh coefficients.  Per x
+// k_assemble_modal (linear materials, FP64 form): works on Walsh coefficients.  Per x
 // plane each thread reads the four nodes of its y-z cell from LDS, takes their
 // 2-D Walsh coefficients, and combines them with the previous plane's, kept in
 // registers, to the element's 3-D coefficients; the element maps these to force
@@ -18,7 +18,8 @@
 // reads (24 -> 9 words per component triple), the z (DPP) and y (shuffle)
 // exchanges, and takes 36 instead of about 56 additions per component.
 //
-// k_assemble (nonlinear models): per-Gauss-point constitutive path.  Per plane:
+// k_assemble (nonlinear models: per-Gauss-point constitutive path; linear ones in
+// the mixed form, see element_forces_iso3_modal).  Per plane:
 //   1. the 17x17 node plane x+1 is staged in LDS;
 //   2. each thread gathers its 8 corners from LDS and computes its element;
 //   3. corner forces are combined along z with DPP row_shr (in registers),
@@ -76,7 +77,7 @@ __device__ __forceinline__ T shfl_up16(T v)
 // k_assemble_modal: ASM_ISO = every phase LinearElasticIsotropic (H=3) or
 // LinearThermalIsotropic (H=1); ASM_ISO_CUBIC = the same on cubic voxels;
 // ASM_ANISO = any linear models, the phase table holding full tensors.
-// k_assemble: ASM_GENERAL = small strain; ASM_LARGE = finite strain (F and P,
+// k_assemble: the isotropic two in the mixed form; ASM_GENERAL = small strain; ASM_LARGE = finite strain (F and P,
 // n_str 9); ASM_GENERAL_PNL = ASM_GENERAL with power-law PseudoPlastic phases
 // present; ASM_GENERAL_VISCO = ASM_GENERAL with J2ViscoPlastic phases present
 // (their per-call psi / psi_bar update, see PointModel).
@@ -85,12 +86,19 @@ enum { ASM_GENERAL = 0, ASM_ISO = 1, ASM_ISO_CUBIC = 2, ASM_LARGE = 3, ASM_GENER
 
 // The per-Gauss-point FP64 residual lands just above 256 registers (one wave
 // per SIMD) unless asked for two waves, which it reaches without spilling; the
-// finite-strain, power-law and visco-plastic residuals would spill there, so
-// they keep one.
-template <typename T, int VAR>
+// finite-strain, power-law and visco-plastic residuals and the FP64
+// per-Gauss-point linear matvec would spill there, so they keep one.  The FP64
+// isotropic matvec takes 132 registers (three waves per SIMD); the FP32 one fits 84
+// (six), with GRP 96 (five: 256^3 184 us; at six it spills, 224; without GRP 163).
+template <typename T, int MODE, int VAR, bool GRP>
 constexpr int kAsmWaves()
 {
-    return VAR == ASM_LARGE || VAR == ASM_GENERAL_PNL || VAR == ASM_GENERAL_VISCO ? 1 : 2;
+    if (VAR == ASM_LARGE || VAR == ASM_GENERAL_PNL || VAR == ASM_GENERAL_VISCO ||
+        (VAR == ASM_GENERAL && MODE == ASM_CGLIN && sizeof(T) == 8))
+        return 1;
+    if ((VAR == ASM_ISO || VAR == ASM_ISO_CUBIC) && MODE == ASM_CGLIN)
+        return sizeof(T) == 8 ? 3 : GRP ? 5 : 6;
+    return 2;
 }
 
 // the workgroup's buffers moved to its RVE slot
@@ -484,9 +492,12 @@ void k_assemble_modal(AsmArgs<T> a)
     }
 }
 
-template <typename T, int H, int NGP, int VAR>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kAsmWaves<T, VAR>()))) void k_assemble(AsmArgs<T> a)
+// GRP (matvec): one partial per a.grp planes instead of one per workgroup, for
+// workgroups of several times a.grp planes
+template <typename T, int H, int NGP, int MODE, int VAR, bool GRP = false>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kAsmWaves<T, MODE, VAR, GRP>()))) void k_assemble(AsmArgs<T> a)
 {
+    constexpr bool ISO = VAR == ASM_ISO || VAR == ASM_ISO_CUBIC, CUBIC = VAR == ASM_ISO_CUBIC;
     const int sb = slot_of(a.sl);
     if (sb < 0)
         return;
@@ -539,9 +550,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kAsmWaves<T
     T g0[NS];
 #pragma unroll
     for (int i = 0; i < NS; ++i)
-        g0[i] = a.g0[i];
-    // small strain: model kind of the first 256 phases, staged once per block
-    constexpr bool PM = VAR != ASM_LARGE;
+        g0[i] = (MODE == ASM_RESID) ? a.g0[i] : (T) 0;
+    const T w = (T) a.geom.w;
+    // isotropic moduli of the first 256 phases, staged once per block (ids
+    // beyond read the phase table)
+    __shared__ T PL[256][2];
+    if constexpr (ISO) {
+        for (int p = t; p < min(a.nphases, 256); p += blockDim.x) {
+            PL[p][0] = a.phases[p].p[0];
+            PL[p][1] = H == 3 ? a.phases[p].p[1] : (T) 0;
+        }
+    }
+    // per-Gauss-point residual: model kind of the first 256 phases, staged once
+    // per block
+    constexpr bool PM = !ISO && VAR != ASM_LARGE && MODE == ASM_RESID;
     __shared__ int PK[PM ? 256 : 1];
     if constexpr (PM)
         for (int p = t; p < min(a.nphases, 256); p += blockDim.x)
@@ -587,6 +609,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kAsmWaves<T
     int                   ph_next = phase_of(X0 - 1);
     PointModel<T, H, NGP, VAR == ASM_GENERAL_PNL || VAR == ASM_GENERAL_VISCO, VAR == ASM_GENERAL_VISCO> pm;
     bool pm_pre = false;  // point 0 of the coming element requested
+    int           left = a.grp;
+    double       *part = GRP ? a.partial + ((int64_t) (X0 / a.grp) * a.nty + ty) * a.ntz + tz : nullptr;
     for (int i = 0; X0 - 1 + i < X1; ++i) {
         const int xe = X0 - 1 + i;
         commit_plane((i + 1) & 1);
@@ -603,14 +627,56 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kAsmWaves<T
             for (int c = 0; c < H; ++c)
                 u[cr][c] = src[c];
         }
-        const int xg = xe < 0 ? xe + nx : xe;
-        T         f[8][H];
-        {
+        T dv[H];  // d at node plane xe (CG mode)
+#pragma unroll
+        for (int c = 0; c < H; ++c)
+            dv[c] = u[0][c];
+        const int     xg = xe < 0 ? xe + nx : xe;
+        const int64_t el = xg * plane + off_own;
+        T             f[8][H];
+        if constexpr (ISO) {
+            if constexpr (H == 3) {
+                T lam = ph < 256 ? PL[ph][0] : a.phases[ph].p[0], mu = ph < 256 ? PL[ph][1] : a.phases[ph].p[1];
+                if (a.vk) {
+                    mu  = a.vg[el];
+                    lam = a.vk[el] - (T) (2.0 / 3.0) * mu;
+                }
+                const T lw = lam * w, mw = mu * w;
+                T       T0[3][3];
+                if constexpr (MODE == ASM_RESID) {
+                    const T r = (T) kSqrtHalf, tr = g0[0] + g0[1] + g0[2];
+                    const T E[3][3] = {{g0[0], r * g0[3], r * g0[4]}, {r * g0[3], g0[1], r * g0[5]},
+                                       {r * g0[4], r * g0[5], g0[2]}};
+#pragma unroll
+                    for (int p = 0; p < 3; ++p)
+#pragma unroll
+                        for (int q = 0; q < 3; ++q)
+                            T0[p][q] = (T) 2 * mw * E[p][q] + (p == q ? lw * tr : (T) 0);
+                } else {
+#pragma unroll
+                    for (int p = 0; p < 3; ++p)
+#pragma unroll
+                        for (int q = 0; q < 3; ++q)
+                            T0[p][q] = (T) 0;
+                }
+                element_forces_iso3_modal<T, NGP, CUBIC>(reinterpret_cast<const T(&)[8][3]>(u), a.geom, lw, mw, T0,
+                                            reinterpret_cast<T(&)[8][3]>(f));
+            } else {
+                const T kw    = (a.vk ? a.vk[el] : (ph < 256 ? PL[ph][0] : a.phases[ph].p[0])) * w;
+                const T T0[3] = {kw * g0[0], kw * g0[1], kw * g0[2]};
+                element_forces_iso1_modal<T, NGP, CUBIC>(reinterpret_cast<const T(&)[8][1]>(u), a.geom, kw, T0,
+                                            reinterpret_cast<T(&)[8][1]>(f));
+            }
+        } else {
             const Phase<T> &P = a.phases[ph];
+            // the linear matvec sees linear models only: no state to prefetch
             if constexpr (NS == 9) {
                 auto mat = [&](int gp, const T(&e)[NS], T(&s)[NS]) {
                     material_point_ns<T, H, NS>(P, e, s);
                 };
+                element_forces<T, H, NGP, NS>(u, a.geom, g0, mat, f);
+            } else if constexpr (MODE == ASM_CGLIN) {
+                auto mat = [&](int gp, const T(&e)[NS], T(&s)[NS]) { linear_point<T, H>(P, e, s); };
                 element_forces<T, H, NGP, NS>(u, a.geom, g0, mat, f);
             } else {
                 // the next element of this thread's row is xe + 1 (phase ph_next),
@@ -665,22 +731,48 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kAsmWaves<T
             for (int c = 0; c < H; ++c) {
                 const T res            = carry[c] + P2[0][0][c] + up[0][c];
                 a.out[off_own * H + po + c] = res;
-                acc_norm(acc0, res, a.measure);
-                if (a.dotv)
-                    acc1 += (double) res * (double) a.dotv[off_own * H + po + c];
+                if constexpr (MODE == ASM_CGLIN) {
+                    acc0 += (double) dv[c] * (double) res;
+                } else {
+                    const double ar = fabs((double) res);
+                    if (a.measure == 2)
+                        acc0 = fmax(acc0, ar);
+                    else if (a.measure == 1)
+                        acc0 += ar * ar;
+                    else
+                        acc0 += ar;
+                    if (a.dotv)
+                        acc1 += (double) res * (double) a.dotv[off_own * H + po + c];
+                }
             }
         }
 #pragma unroll
         for (int c = 0; c < H; ++c)
             carry[c] = P2[1][0][c] + up[1][c];
+        if constexpr (GRP) {
+            if (i >= 1 && (--left == 0 || xe + 1 == X1)) {
+                double     v[1]  = {acc0};
+                const bool mx[1] = {false};
+                block_reduce<1>(v, mx, red);
+                if (t == 0)
+                    *part = v[0];
+                part += a.nty * a.ntz;
+                acc0 = 0.0;
+                left = a.grp;
+            }
+        }
     }
-    if (a.partial) {
+    if (!GRP && a.partial) {
         double     v[2]  = {acc0, acc1};
-        const bool mx[2] = {a.measure == 2, false};
+        const bool mx[2] = {MODE == ASM_RESID && a.measure == 2, false};
         block_reduce<2>(v, mx, red);
         if (t == 0) {
-            a.partial[blockIdx.x]             = v[0];
-            a.partial[gridDim.x + blockIdx.x] = v[1];
+            if (MODE == ASM_CGLIN) {
+                a.partial[((int64_t) bx * a.nty + ty) * a.ntz + tz] = v[0];
+            } else {
+                a.partial[blockIdx.x]             = v[0];
+                a.partial[gridDim.x + blockIdx.x] = v[1];
+            }
         }
     }
 }

@@ -36,26 +36,53 @@ void launch_modal(fans_gpu_ctx *c, const AsmArgs<T> &a, dim3 g)
 #undef MODAL
 }
 
-// the residual of nonlinear materials (thermal models are all linear)
-template <typename T>
-void launch_general(fans_gpu_ctx *c, const AsmArgs<T> &a, dim3 g)
+// k_assemble: nonlinear materials (residual only; thermal models are all linear),
+// linear ones in the mixed form
+template <typename T, int MODE, int H, int NGP>
+void launch_general_hn(fans_gpu_ctx *c, const AsmArgs<T> &a, dim3 g)
 {
-#define ASM(VAR)                                                                                \
-    do {                                                                                        \
-        if (c->ngp == 8)                                                                        \
-            hipLaunchKernelGGL((k_assemble<T, 3, 8, VAR>), g, dim3(kThreads), 0, c->stream, a); \
-        else                                                                                    \
-            hipLaunchKernelGGL((k_assemble<T, 3, 1, VAR>), g, dim3(kThreads), 0, c->stream, a); \
-    } while (0)
-    if (c->nstr == 9)
-        ASM(ASM_LARGE);
-    else if (c->has_visco)
-        ASM(ASM_GENERAL_VISCO);
-    else if (c->has_pnl)
-        ASM(ASM_GENERAL_PNL);
+#define ASM(VAR) hipLaunchKernelGGL((k_assemble<T, H, NGP, MODE, VAR>), g, dim3(kThreads), 0, c->stream, a)
+    if constexpr (MODE == ASM_RESID && H == 3) {
+        if (c->nstr == 9) {
+            ASM(ASM_LARGE);
+            return;
+        }
+        if (c->has_visco) {
+            ASM(ASM_GENERAL_VISCO);
+            return;
+        }
+        if (c->has_pnl) {
+            ASM(ASM_GENERAL_PNL);
+            return;
+        }
+    }
+    if constexpr (MODE == ASM_CGLIN && sizeof(T) == 4)
+        if (a.cx != a.grp) {  // a batch's deeper workgroups
+#define ASMG(VAR) hipLaunchKernelGGL((k_assemble<T, H, NGP, MODE, VAR, true>), g, dim3(kThreads), 0, c->stream, a)
+            if (c->all_iso && c->cubic)
+                ASMG(ASM_ISO_CUBIC);
+            else if (c->all_iso)
+                ASMG(ASM_ISO);
+            else
+                ASMG(ASM_GENERAL);
+#undef ASMG
+            return;
+        }
+    if (c->all_iso && c->cubic)
+        ASM(ASM_ISO_CUBIC);
+    else if (c->all_iso)
+        ASM(ASM_ISO);
     else
         ASM(ASM_GENERAL);
 #undef ASM
+}
+template <typename T, int MODE>
+void launch_general(fans_gpu_ctx *c, const AsmArgs<T> &a, dim3 g)
+{
+    if (c->h == 1)
+        c->ngp == 8 ? launch_general_hn<T, MODE, 1, 8>(c, a, g) : launch_general_hn<T, MODE, 1, 1>(c, a, g);
+    else
+        c->ngp == 8 ? launch_general_hn<T, MODE, 3, 8>(c, a, g) : launch_general_hn<T, MODE, 3, 1>(c, a, g);
 }
 
 }  // namespace fans

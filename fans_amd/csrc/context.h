@@ -91,6 +91,23 @@ inline bool make_len(int n, int tws, FftLen &L, int max_radix = 16)
     return found;
 }
 
+// the FP32 stages (lds_stockham)
+inline bool make_len_stockham(int n, int tws, FftLen &L)
+{
+    L.n   = n;
+    L.tws = tws;
+    L.nst = 0;
+    int m = n;
+    for (int r : {5, 3, 8, 4, 2})
+        while (m % r == 0) {
+            if (L.nst >= kMaxStages)
+                return false;
+            L.rad[L.nst++] = r;
+            m /= r;
+        }
+    return m == 1;
+}
+
 // lines per block of the compile-time z kernels (0: generic kernels)
 inline int zct_lines(int h, int M)
 {
@@ -158,34 +175,48 @@ struct Fft3D {
         nx = nx_, ny = ny_, nz = nz_, h = h_;
         M  = nz / 2;
         Mc = M + 1;
-        if (!make_len(M, 2, Lz) || !make_len(ny, 1, Ly) ||
-            !make_len(nx, 1, Lx, h == 3 ? kXGreenMaxRadix<T, 3>() : kXGreenMaxRadix<T, 1>()))
-            return hipErrorInvalidValue;
         const size_t cb = sizeof(cplx<T>);
+        const int    Kc = Mc * h;
         if ((int64_t) M * h > FFT_MAX_ELEMS || ny > FFT_MAX_ELEMS || (int64_t) nx * h > FFT_MAX_ELEMS)
             return hipErrorInvalidValue;
-        // one LDS tile per workgroup, by default 40 KiB (four workgroups per CU).
-        // The strided passes go to 64 KiB where that gives rows of 16 columns (192
-        // points, FP64, 200 x 192 x 160 conduction: 25.5 us against 27.7 with 8
-        // columns); the FP32 x pass stays within 24 KiB (256^3 132 us against 138
-        // at 40 KiB, 128^3 24.7 against 27.4, 96^3 12.5 against 15.1) and the z passes
-        // within 32 (125 x 120 x 150 FP64 52.5 and 50.0 us against 56.8 and 52.0)
-        const int64_t lim  = (int64_t) lds_kib * 1024 / (int64_t) cb;
-        const int64_t wide = lds_set ? lim : 64 * 1024 / (int64_t) cb;
-        const int64_t xlim = lds_set ? lim : (int64_t) (sizeof(T) == 4 ? 24 : 40) * 1024 / (int64_t) cb;
-        const int64_t zlim = lds_set ? lim : (int64_t) 32 * 1024 / (int64_t) cb;
-        lpb                = (int) std::max<int64_t>(1, std::min<int64_t>(16, zlim / (M * h)));
-        smz                = cb * M * (lpb * h + 1) + sizeof(unsigned short) * M;
-        const int Kc       = Mc * h;
-        bc                 = pow2_cols((int) (wide / ny), std::min(Kc, 16));
-        smy                = cb * ny * bc;
-        // frequencies per x+Green workgroup: the budget, less where that leaves
-        // fewer than 256 workgroups
-        const int64_t nbk = std::max<int64_t>({1, (Mc * (int64_t) nx * h + xlim - 1) / xlim, lds_set ? 1 : 256 / ny});
-        bk                = (int) std::max<int64_t>(1, std::min<int64_t>(xlim / (nx * h), (Mc + nbk - 1) / nbk));
-        smx               = cb * nx * bk * h;
-        bcx               = pow2_cols((int) (wide / nx), 16);
-        smx_plain         = cb * nx * bcx;
+        const int64_t lim = (int64_t) lds_kib * 1024 / (int64_t) cb;
+        if constexpr (sizeof(T) == 4) {
+            // one padded LDS tile per workgroup, n * columns <= FFT_MAX_ELEMS so the
+            // in-place stages keep every butterfly input in registers
+            if (!make_len_stockham(M, 2, Lz) || !make_len_stockham(ny, 1, Ly) || !make_len_stockham(nx, 1, Lx))
+                return hipErrorInvalidValue;
+            const int le = (int) std::min<int64_t>(FFT_MAX_ELEMS, lim);
+            lpb          = std::max(1, std::min(16, le / (M * h)));
+            smz          = cb * M * (lpb * h + 1);
+            bc           = pow2_cols(le / ny, std::min(Kc, 16));
+            smy          = cb * ny * (bc + 1);
+            bk           = std::max(1, std::min(Mc, le / (nx * h)));
+            smx          = cb * nx * (bk * h + 1);
+            bcx          = pow2_cols(le / nx, 16);
+            smx_plain    = cb * nx * (bcx + 1);
+        } else {
+            if (!make_len(M, 2, Lz) || !make_len(ny, 1, Ly) ||
+                !make_len(nx, 1, Lx, h == 3 ? kXGreenMaxRadix<3>() : kXGreenMaxRadix<1>()))
+                return hipErrorInvalidValue;
+            // one LDS tile per workgroup, by default 40 KiB (four workgroups per CU).
+            // The strided passes go to 64 KiB where that gives rows of 16 columns (192
+            // points, 200 x 192 x 160 conduction: 25.5 us against 27.7 with 8
+            // columns); the z passes stay within 32 (125 x 120 x 150 52.5 and 50.0 us
+            // against 56.8 and 52.0)
+            const int64_t wide = lds_set ? lim : 64 * 1024 / (int64_t) cb;
+            const int64_t zlim = lds_set ? lim : (int64_t) 32 * 1024 / (int64_t) cb;
+            lpb                = (int) std::max<int64_t>(1, std::min<int64_t>(16, zlim / (M * h)));
+            smz                = cb * M * (lpb * h + 1) + sizeof(unsigned short) * M;
+            bc                 = pow2_cols((int) (wide / ny), std::min(Kc, 16));
+            smy                = cb * ny * bc;
+            // frequencies per x+Green workgroup: the budget, less where that leaves
+            // fewer than 256 workgroups
+            const int64_t nbk = std::max<int64_t>({1, (Mc * (int64_t) nx * h + lim - 1) / lim, lds_set ? 1 : 256 / ny});
+            bk                = (int) std::max<int64_t>(1, std::min<int64_t>(lim / (nx * h), (Mc + nbk - 1) / nbk));
+            smx               = cb * nx * bk * h;
+            bcx               = pow2_cols((int) (wide / nx), 16);
+            smx_plain         = cb * nx * bcx;
+        }
         nblk_z       = ((int64_t) nx * ny + lpb - 1) / lpb;
         const int lct = zct_lines(h, M);
         zct           = lct > 0 && ((int64_t) nx * ny) % lct == 0;
@@ -406,7 +437,7 @@ int64_t x_green_blocks(const Fft3D<T> &P, int h, int ny);
 // linear and nonlinear assembly
 template <typename T, int H, int NGP, int MODE>
 void launch_modal(fans_gpu_ctx *c, const AsmArgs<T> &a, dim3 g);
-template <typename T>
+template <typename T, int MODE>
 void launch_general(fans_gpu_ctx *c, const AsmArgs<T> &a, dim3 g);
 
 }  // namespace fans

@@ -1502,4 +1502,265 @@ __global__ __launch_bounds__(256) void k_element_pass(ElemArgs<T> a)
     }
 }
 
+// ---------------------------------------------------------------------------
+// linear elements of the mixed form (k_assemble), all eight corners at a time.
+// Its operation order is kept: a mixed displacement is FP32 rounding below about
+// 1e-8 of its size, and another order moves it by up to 5e-9.
+// ---------------------------------------------------------------------------
+
+// sigma of the linear models only (the linear matvec K d never sees another
+// kind; anything else gives NaN)
+template <typename T, int H>
+__device__ __forceinline__ void linear_point(const Phase<T> &P, const T (&e)[H == 1 ? 3 : 6],
+                                             T (&s)[H == 1 ? 3 : 6])
+{
+    constexpr int n = H == 1 ? 3 : 6;
+    if (P.kind == MODEL_THERMAL_ISO || P.kind == MODEL_ELASTIC_ISO) {
+        if constexpr (H == 1) {
+#pragma unroll
+            for (int i = 0; i < 3; ++i)
+                s[i] = P.p[0] * e[i];
+        } else {
+            const T b1 = P.p[0] * (e[0] + e[1] + e[2]), b2 = (T) 2 * P.p[1];
+#pragma unroll
+            for (int i = 0; i < 3; ++i)
+                s[i] = b1 + b2 * e[i];
+#pragma unroll
+            for (int i = 3; i < 6; ++i)
+                s[i] = b2 * e[i];
+        }
+    } else if (P.kind == MODEL_THERMAL_TRI || P.kind == MODEL_ELASTIC_TRI) {
+#pragma unroll
+        for (int i = 0; i < n; ++i) {
+            T a = 0;
+#pragma unroll
+            for (int j = 0; j < n; ++j)
+                a += P.p[n * i + j] * e[j];
+            s[i] = a;
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < n; ++i)
+            s[i] = (T) NAN;
+    }
+}
+
+// unnormalised 3-D Walsh-Hadamard transform of the 8 corner values (corner /
+// coefficient index i + 2j + 4k): W[ijk] = sum_xyz (-1)^(ix+jy+kz) v[xyz].
+// The Hadamard modes of the edge differences are Walsh coefficients:
+//   d/dx: A0..A3 = -W100, W110, W101, -W111   (d/dy: -W010, W110, W011, -W111;
+//   d/dz: -W001, W101, W011, -W111)
+// so one transform of 24 additions replaces the 3 x (4 differences + 8-addition
+// Hadamard) per component, and the transposed maps are one transform of the
+// mode sums.  The transform is symmetric (its own transpose).
+template <typename T>
+__device__ __forceinline__ void walsh8(T (&v)[8])
+{
+#pragma unroll
+    for (int s = 1; s < 8; s <<= 1)
+#pragma unroll
+        for (int a = 0; a < 8; ++a)
+            if ((a & s) == 0) {
+                const T x = v[a], y = v[a + s];
+                v[a]      = x + y;
+                v[a + s]  = x - y;
+            }
+}
+
+template <typename T, int d>
+__device__ __forceinline__ void modal_single(T (&a)[3], T L, T M)
+{
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+        a[c] *= (c == d) ? (L + M + M) : M;
+}
+
+// f = Ke(lambda, mu) u (+ the forces of the traction T0 = w sigma(g0)).  CUBIC (hx = hy = hz): the 1/h of the edge
+// differences and of their transpose fold into the modal constants (k^2) and
+// the traction term (k), which saves 72 multiplications per element.
+template <typename T, int NGP, bool CUBIC = false>
+__device__ __forceinline__ void element_forces_iso3_modal(const T (&u)[8][3], const Geom &g, T lw, T mw,
+                                                          const T (&T0)[3][3], T (&f)[8][3])
+{
+    const T kc   = (T) g.ilx;
+    const T k[3] = {CUBIC ? (T) 1 : (T) g.ilx, CUBIC ? (T) 1 : (T) g.ily, CUBIC ? (T) 1 : (T) g.ilz};
+    // A[d][mode][c]: Hadamard modes of the edge differences along d, scaled by 1/h_d
+    T A[3][4][3];
+    if constexpr (NGP == 8) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            T w[8];
+#pragma unroll
+            for (int n = 0; n < 8; ++n)
+                w[n] = u[n][c];
+            walsh8(w);
+            A[0][0][c] = -w[1] * k[0], A[0][1][c] = w[3] * k[0], A[0][2][c] = w[5] * k[0], A[0][3][c] = -w[7] * k[0];
+            A[1][0][c] = -w[2] * k[1], A[1][1][c] = w[3] * k[1], A[1][2][c] = w[6] * k[1], A[1][3][c] = -w[7] * k[1];
+            A[2][0][c] = -w[4] * k[2], A[2][1][c] = w[5] * k[2], A[2][2][c] = w[6] * k[2], A[2][3][c] = -w[7] * k[2];
+        }
+    } else {
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+#pragma unroll
+            for (int p = 0; p < 2; ++p)
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    A[0][p + 2 * q][c] = (u[1 + 2 * p + 4 * q][c] - u[2 * p + 4 * q][c]) * k[0];
+                    A[1][p + 2 * q][c] = (u[p + 2 + 4 * q][c] - u[p + 4 * q][c]) * k[1];
+                    A[2][p + 2 * q][c] = (u[p + 2 * q + 4][c] - u[p + 2 * q][c]) * k[2];
+                }
+    }
+    // Gauss weight w = V / NGP; mode weights NGP / 3^deg; 1/16 from the two
+    // factors 1/4 of the bilinear expansion
+    const T s  = CUBIC ? (T) NGP / (T) 16 * kc * kc : (T) NGP / (T) 16;
+    const T L0 = s * lw, M0 = s * mw;
+    if constexpr (NGP == 1) {
+#pragma unroll
+        for (int d = 0; d < 3; ++d)
+#pragma unroll
+            for (int c = 0; c < 3; ++c)
+                A[d][0][c] = (A[d][0][c] + A[d][2][c]) + (A[d][1][c] + A[d][3][c]);
+    }
+    // mode 1: all nine entries
+    {
+        const T t  = L0 * (A[0][0][0] + A[1][0][1] + A[2][0][2]);
+        const T m2 = M0 + M0;
+        const T t0 = CUBIC ? (T) NGP * (T) 0.25 * kc : (T) NGP * (T) 0.25;
+#pragma unroll
+        for (int d = 0; d < 3; ++d)
+            A[d][0][d] = t + m2 * A[d][0][d] + t0 * T0[d][d];
+#pragma unroll
+        for (int d = 0; d < 3; ++d)
+#pragma unroll
+            for (int c = d + 1; c < 3; ++c) {
+                // entry (c, d) holds du_c/dx_d, entry (d, c) du_d/dx_c
+                const T v  = M0 * (A[d][0][c] + A[c][0][d]);
+                A[d][0][c] = v + t0 * T0[c][d];
+                A[c][0][d] = v + t0 * T0[d][c];
+            }
+    }
+    if constexpr (NGP == 8) {
+        // B-bar keeps only the element-mean trace: the trace energy of the
+        // higher modes drops by K, which leaves lambda - K = -2 mu / 3
+        const T third = (T) (1.0 / 3.0);
+        const T Lh = g.bbar ? (T) (-2.0 / 3.0) * M0 : L0;
+        const T L1 = Lh * third, M1 = M0 * third, L2 = L1 * third, M2 = M1 * third;
+        // xi: d/dy mode 1, d/dz mode 1; eta: d/dx mode 1, d/dz mode 2; zeta: d/dx mode 2, d/dy mode 2
+        modal_pair<T, 1, 2>(A[1][1], A[2][1], L1, M1);
+        modal_pair<T, 0, 2>(A[0][1], A[2][2], L1, M1);
+        modal_pair<T, 0, 1>(A[0][2], A[1][2], L1, M1);
+        modal_single<T, 0>(A[0][3], L2, M2);  // eta zeta
+        modal_single<T, 1>(A[1][3], L2, M2);  // xi zeta
+        modal_single<T, 2>(A[2][3], L2, M2);  // xi eta
+        // transposed maps: the Walsh transform of the mode sums
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            T b[8];
+            b[0] = (T) 0;
+            b[1] = -A[0][0][c] * k[0];
+            b[2] = -A[1][0][c] * k[1];
+            b[4] = -A[2][0][c] * k[2];
+            b[3] = A[0][1][c] * k[0] + A[1][1][c] * k[1];
+            b[5] = A[0][2][c] * k[0] + A[2][1][c] * k[2];
+            b[6] = A[1][2][c] * k[1] + A[2][2][c] * k[2];
+            b[7] = -(A[0][3][c] * k[0] + A[1][3][c] * k[1] + A[2][3][c] * k[2]);
+            walsh8(b);
+#pragma unroll
+            for (int n = 0; n < 8; ++n)
+                f[n][c] = b[n];
+        }
+        return;
+    } else {
+#pragma unroll
+        for (int d = 0; d < 3; ++d)
+#pragma unroll
+            for (int c = 0; c < 3; ++c)
+                A[d][1][c] = A[d][2][c] = A[d][3][c] = A[d][0][c];
+    }
+    // transposed edge differences (one Gauss point)
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+#pragma unroll
+        for (int n = 0; n < 8; ++n)
+            f[n][c] = (T) 0;
+#pragma unroll
+        for (int p = 0; p < 2; ++p)
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                const T dx = A[0][p + 2 * q][c] * k[0], dy = A[1][p + 2 * q][c] * k[1],
+                        dz = A[2][p + 2 * q][c] * k[2];
+                f[1 + 2 * p + 4 * q][c] += dx;
+                f[2 * p + 4 * q][c] -= dx;
+                f[p + 2 + 4 * q][c] += dy;
+                f[p + 4 * q][c] -= dy;
+                f[p + 2 * q + 4][c] += dz;
+                f[p + 2 * q][c] -= dz;
+            }
+    }
+}
+
+// isotropic conduction in modal form: every mode of every derivative is its
+// own block, weighted by NGP / 3^deg
+template <typename T, int NGP, bool CUBIC = false>
+__device__ __forceinline__ void element_forces_iso1_modal(const T (&u)[8][1], const Geom &g, T kw, const T (&T0)[3],
+                                                          T (&f)[8][1])
+{
+    const T kc   = (T) g.ilx;
+    const T k[3] = {CUBIC ? (T) 1 : (T) g.ilx, CUBIC ? (T) 1 : (T) g.ily, CUBIC ? (T) 1 : (T) g.ilz};
+    const T c0   = CUBIC ? (T) NGP / (T) 16 * kw * kc * kc : (T) NGP / (T) 16 * kw;
+    const T t0   = CUBIC ? (T) NGP * (T) 0.25 * kc : (T) NGP * (T) 0.25;
+    if constexpr (NGP == 8) {
+        // Walsh coefficients -> modes (see walsh8), modal scaling, mode sums -> Walsh
+        T w[8];
+#pragma unroll
+        for (int n = 0; n < 8; ++n)
+            w[n] = u[n][0];
+        walsh8(w);
+        const T c1 = c0 * (T) (1.0 / 3.0), c2 = c1 * (T) (1.0 / 3.0);
+        T       b[8];
+        b[0]        = (T) 0;
+        b[1]        = -(c0 * (-w[1] * k[0]) + t0 * T0[0]) * k[0];
+        b[2]        = -(c0 * (-w[2] * k[1]) + t0 * T0[1]) * k[1];
+        b[4]        = -(c0 * (-w[4] * k[2]) + t0 * T0[2]) * k[2];
+        b[3]        = c1 * w[3] * (k[0] * k[0] + k[1] * k[1]);
+        b[5]        = c1 * w[5] * (k[0] * k[0] + k[2] * k[2]);
+        b[6]        = c1 * w[6] * (k[1] * k[1] + k[2] * k[2]);
+        b[7]        = c2 * w[7] * (k[0] * k[0] + k[1] * k[1] + k[2] * k[2]);
+        walsh8(b);
+#pragma unroll
+        for (int n = 0; n < 8; ++n)
+            f[n][0] = b[n];
+        return;
+    }
+    T A[3][4];
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            A[0][p + 2 * q] = (u[1 + 2 * p + 4 * q][0] - u[2 * p + 4 * q][0]) * k[0];
+            A[1][p + 2 * q] = (u[p + 2 + 4 * q][0] - u[p + 4 * q][0]) * k[1];
+            A[2][p + 2 * q] = (u[p + 2 * q + 4][0] - u[p + 2 * q][0]) * k[2];
+        }
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        const T a = c0 * ((A[d][0] + A[d][2]) + (A[d][1] + A[d][3])) + t0 * T0[d];
+        A[d][0] = A[d][1] = A[d][2] = A[d][3] = a;
+    }
+#pragma unroll
+    for (int n = 0; n < 8; ++n)
+        f[n][0] = (T) 0;
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const T dx = A[0][p + 2 * q] * k[0], dy = A[1][p + 2 * q] * k[1], dz = A[2][p + 2 * q] * k[2];
+            f[1 + 2 * p + 4 * q][0] += dx;
+            f[2 * p + 4 * q][0] -= dx;
+            f[p + 2 + 4 * q][0] += dy;
+            f[p + 4 * q][0] -= dy;
+            f[p + 2 * q + 4][0] += dz;
+            f[p + 2 * q][0] -= dz;
+        }
+}
+
 }  // namespace fans

@@ -434,8 +434,12 @@ int asm_planes_rule(int nx, int64_t tiles, bool modal, int grp = 1)
 
 int ensure_partials(fans_gpu_ctx *c);
 
-// every phase linear, small strain: the modal kernel
-bool asm_modal(const fans_gpu_ctx *c) { return c->all_linear && c->nstr != 9; }
+// every phase linear, small strain: the modal kernel, except in the mixed form,
+// whose operation order is kept (element_forces_iso3_modal)
+bool asm_modal(const fans_gpu_ctx *c)
+{
+    return c->all_linear && c->nstr != 9 && c->d.precision != FANS_PREC_MIXED;
+}
 
 void set_planes(fans_gpu_ctx *c, int cx)
 {
@@ -458,24 +462,25 @@ template <typename T, int MODE>
 int launch_assemble(fans_gpu_ctx *c, AsmArgs<T> a)
 {
     Timed t(c, MODE == ASM_CGLIN ? KF_ASSEMBLE_LIN : KF_ASSEMBLE_RES);
-    if (asm_modal(c)) {
-        // partials come per c->cx planes whatever depth runs: a batch of many
-        // slots takes deeper workgroups without moving any slot's sums
-        int nblk = c->nblk_asm;
-        a.grp    = c->cx;
-        if (MODE == ASM_CGLIN && c->gz > 1 && !c->cx_set) {
-            a.cx = asm_planes_rule(c->nx, (int64_t) c->nty * c->ntz * c->gz, true, c->cx);
-            nblk = (c->nx + a.cx - 1) / a.cx * c->nty * c->ntz;
-        }
-        const dim3 g(nblk, 1, c->gz);
+    if (MODE == ASM_CGLIN && !c->all_linear)
+        return fail(c, FANS_GPU_EINVAL, "linear matvec needs linear materials");
+    // matvec partials come per c->cx planes whatever depth runs: a batch of many
+    // slots takes deeper workgroups without moving any slot's sums
+    const bool modal = asm_modal(c);
+    int        nblk  = c->nblk_asm;
+    a.grp            = c->cx;
+    if (MODE == ASM_CGLIN && c->gz > 1 && !c->cx_set && (modal || sizeof(T) == 4)) {
+        a.cx = asm_planes_rule(c->nx, (int64_t) c->nty * c->ntz * c->gz, modal, c->cx);
+        nblk = (c->nx + a.cx - 1) / a.cx * c->nty * c->ntz;
+    }
+    const dim3 g(nblk, 1, c->gz);
+    if (!modal) {
+        launch_general<T, MODE>(c, a, g);
+    } else if constexpr (sizeof(T) == 8) {
         if (c->h == 1)
             c->ngp == 8 ? launch_modal<T, 1, 8, MODE>(c, a, g) : launch_modal<T, 1, 1, MODE>(c, a, g);
         else
             c->ngp == 8 ? launch_modal<T, 3, 8, MODE>(c, a, g) : launch_modal<T, 3, 1, MODE>(c, a, g);
-    } else if constexpr (MODE == ASM_RESID) {
-        launch_general<T>(c, a, dim3(c->nblk_asm, 1, c->gz));
-    } else {
-        return fail(c, FANS_GPU_EINVAL, "linear matvec needs linear materials");
     }
     HIPCHK(c, hipGetLastError());
     return 0;
@@ -1996,7 +2001,7 @@ static int create_ctx(fans_gpu_ctx **out, const fans_gpu_desc *d, int slots)
     // launch geometry
     c->nty      = (c->ny + NOUT - 1) / NOUT;
     c->ntz      = (c->nz + NOUT - 1) / NOUT;
-    set_planes(c, asm_planes_rule(c->nx, (int64_t) c->nty * c->ntz, c->nstr != 9));
+    set_planes(c, asm_planes_rule(c->nx, (int64_t) c->nty * c->ntz, c->nstr != 9 && d->precision != FANS_PREC_MIXED));
     c->nblk_vec = grid_vec(c->Nh);
     c->nblk_el  = (int) ((c->N + kThreads - 1) / kThreads);
     // J2 state slots (J2State); the state commit walks them
@@ -2336,7 +2341,7 @@ int fans_gpu_set_materials(fans_gpu_ctx *c, int32_t ng, const int32_t *kind, con
     for (int p = 0; p < c->nphases; ++p)
         if (c->phase_kind[p] != (c->h == 1 ? FANS_MODEL_THERMAL_ISO : FANS_MODEL_ELASTIC_ISO))
             c->all_iso = false;
-    const bool aniso = c->all_linear && !c->all_iso;
+    const bool aniso = asm_modal(c) && !c->all_iso;
     c->ph64.assign(c->nphases, Phase<double>{});
     c->ph32.assign(c->nphases, Phase<float>{});
     for (int p = 0; p < c->nphases; ++p) {

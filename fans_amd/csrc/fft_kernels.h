@@ -10,13 +10,13 @@
 // pass carries the Green operator multiply between the forward and inverse
 // transforms, so the spectrum is read and written once for that stage.
 //
-// A transform of n = r1 r2 ... rs runs as s in-place stages: forward by
+// An FP64 transform of n = r1 r2 ... rs runs as s in-place stages: forward by
 // decimation in frequency (natural order in, digit-reversed order out), inverse
 // as its exact reversal.  A butterfly reads and writes the same places, so a
 // stage holds no data across a barrier, and one barrier separates two stages.  The
 // strided passes take their first stage from global memory and give their last
 // one to it; the x pass applies the Green operator to the registers of the last
-// forward stage and starts the inverse from them.
+// forward stage and starts the inverse from them.  FP32: see lds_stockham.
 #pragma once
 #include "cg_scalars.h"
 #include "common.h"
@@ -218,6 +218,80 @@ __device__ __forceinline__ void lds_fft(cplx<T> *buf, const FftLen &L, const cpl
     }
 }
 
+// ---- FP32 stages ----------------------------------------------------------------
+// The FP32 transforms (the inner solve of the mixed form) are Stockham stages of
+// radices 5, 3, 8, 4 and 2, in this order of operations: a mixed displacement is
+// FP32 rounding below about 1e-8 of its size (several outer rounds of FP32
+// directions), so that another order moves it by up to 5e-9, more than the form's
+// results are compared to.  (The larger radices of the FP64 stages took the 128^3
+// mixed solve from 11.6 to 11.0 ms.)
+// Register budget of the in-place stages: a thread holds at most FFT_MAXV
+// complex values; callers keep n * ncols <= FFT_MAXV * 240 so every radix
+// (including 3 and 5, where MAXV/R rounds down) fits.
+constexpr int FFT_MAXV = 16;
+
+// ---- one in-place Stockham radix-R stage over `ncols` independent columns --
+// element (i, col) lives at buf[i * ld + col]
+template <typename T, int R, bool INV>
+__device__ __forceinline__ void stockham_stage(cplx<T> *__restrict__ buf, int n, int ncols, int ld, int Ns,
+                                               const cplx<T> *__restrict__ tw, int tws)
+{
+    constexpr int MB    = FFT_MAXV / R;
+    const int     nb    = n / R;
+    const int     total = nb * ncols;
+    const int     tstep = (n / (Ns * R)) * tws;
+    cplx<T>       v[MB][R];
+#pragma unroll
+    for (int b = 0; b < MB; ++b) {
+        const int w = threadIdx.x + b * blockDim.x;
+        if (w < total) {
+            const int col = w % ncols, j = w / ncols;
+#pragma unroll
+            for (int t = 0; t < R; ++t)
+                v[b][t] = buf[(j + t * nb) * ld + col];
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int b = 0; b < MB; ++b) {
+        const int w = threadIdx.x + b * blockDim.x;
+        if (w < total) {
+            const int col = w % ncols, j = w / ncols, k = j % Ns;
+            if (Ns > 1) {
+#pragma unroll
+                for (int t = 1; t < R; ++t) {
+                    const cplx<T> wv = tw[t * k * tstep];
+                    v[b][t]          = INV ? cmulc(v[b][t], wv) : cmul(v[b][t], wv);
+                }
+            }
+            dft<T, R, INV>(v[b]);
+            const int o = (j / Ns) * Ns * R + k;
+#pragma unroll
+            for (int t = 0; t < R; ++t)
+                buf[(o + t * Ns) * ld + col] = v[b][t];
+        }
+    }
+    __syncthreads();
+}
+
+// full in-place transform of the LDS tile (ends synchronised)
+template <typename T, bool INV>
+__device__ void lds_stockham(cplx<T> *buf, const FftLen &L, const cplx<T> *__restrict__ tw, int ncols, int ld)
+{
+    int Ns = 1;
+    for (int s = 0; s < L.nst; ++s) {
+        const int R = L.rad[s];
+        switch (R) {
+        case 2: stockham_stage<T, 2, INV>(buf, L.n, ncols, ld, Ns, tw, L.tws); break;
+        case 3: stockham_stage<T, 3, INV>(buf, L.n, ncols, ld, Ns, tw, L.tws); break;
+        case 4: stockham_stage<T, 4, INV>(buf, L.n, ncols, ld, Ns, tw, L.tws); break;
+        case 5: stockham_stage<T, 5, INV>(buf, L.n, ncols, ld, Ns, tw, L.tws); break;
+        default: stockham_stage<T, 8, INV>(buf, L.n, ncols, ld, Ns, tw, L.tws); break;
+        }
+        Ns *= R;
+    }
+}
+
 // ---- CG update fused into the forward z pass --------------------------------
 // PRO_CG: the forward z pass of CG iteration i first finishes the residual
 // update of iteration i-1 (solverCG.h:106-117): r -= alpha rnew, and emits per
@@ -324,10 +398,12 @@ __global__ __launch_bounds__(256) void k_fft_z_r2c(T *__restrict__ in, cplx<T> *
     const int64_t g0    = line0 * nzh;
     T             alpha = (T) 0;
     double        a0    = 0.0;
-    // places of the frequencies, behind the tile
+    // places of the frequencies, behind the tile (FP64)
     unsigned short *const place = reinterpret_cast<unsigned short *>(A + M * (lpb * H + 1));
-    for (int k = threadIdx.x; k < M; k += blockDim.x)
-        place[k] = (unsigned short) frequency_place(LM, k);
+    if constexpr (sizeof(T) == 8)
+        for (int k = threadIdx.x; k < M; k += blockDim.x)
+            place[k] = (unsigned short) frequency_place(LM, k);
+    auto place_of = [&](int k) { return sizeof(T) == 8 ? (int) place[k] : k; };
     const FastDiv dz(nzh);
     if constexpr (PRO == PRO_CG)
         alpha = (T) *pa.alpha;
@@ -371,14 +447,17 @@ __global__ __launch_bounds__(256) void k_fft_z_r2c(T *__restrict__ in, cplx<T> *
         }
     }
     __syncthreads();
-    lds_fft<T, false>(A, LM, tw, ncols, ld);
+    if constexpr (sizeof(T) == 8)
+        lds_fft<T, false>(A, LM, tw, ncols, ld);
+    else
+        lds_stockham<T, false>(A, LM, tw, ncols, ld);
     const int     Mc  = M + 1;
     const FastDiv dl(Mc * H);
     cplx<T>      *dst = out + line0 * Mc * H;
     for (int e = threadIdx.x; e < nl * Mc * H; e += blockDim.x) {
         int       rem;
         const int l = dl(e, rem), k = rem / H, c = rem - k * H, col = l * H + c;
-        dst[e] = r2c_untangle(A[place[k == M ? 0 : k] * ld + col], A[place[k == 0 ? 0 : M - k] * ld + col], tw[k]);
+        dst[e] = r2c_untangle(A[place_of(k == M ? 0 : k) * ld + col], A[place_of(k == 0 ? 0 : M - k) * ld + col], tw[k]);
     }
     z_pro_partials<PRO>(pa, a0, red);
 }
@@ -558,18 +637,23 @@ __global__ __launch_bounds__(256) void k_fft_z_c2r(const cplx<T> *__restrict__ i
     FoldBeta          fb;
     if constexpr (EPI == EPI_CGDF)
         fb.template load<256>(ep.fold);
-    // places of the frequencies, behind the tile
+    // places of the frequencies, behind the tile (FP64)
     unsigned short *const place = reinterpret_cast<unsigned short *>(A + M * (lpb * H + 1));
-    for (int k = threadIdx.x; k < M; k += blockDim.x)
-        place[k] = (unsigned short) frequency_place(LM, k);
+    if constexpr (sizeof(T) == 8)
+        for (int k = threadIdx.x; k < M; k += blockDim.x)
+            place[k] = (unsigned short) frequency_place(LM, k);
+    auto place_of = [&](int k) { return sizeof(T) == 8 ? (int) place[k] : k; };
     __syncthreads();
     for (int e = threadIdx.x; e < nl * M * H; e += blockDim.x) {
         int       rem;
         const int l = dl(e, rem), k = rem / H, c = rem - k * H;
-        A[place[k] * ld + l * H + c] = c2r_tangle<T, H>(src + l * Mc * H + c, k, M, tw);
+        A[place_of(k) * ld + l * H + c] = c2r_tangle<T, H>(src + l * Mc * H + c, k, M, tw);
     }
     __syncthreads();
-    lds_fft<T, true>(A, LM, tw, ncols, ld);
+    if constexpr (sizeof(T) == 8)
+        lds_fft<T, true>(A, LM, tw, ncols, ld);
+    else
+        lds_stockham<T, true>(A, LM, tw, ncols, ld);
     const int     nzh = nz * H;
     const int64_t g0  = line0 * nzh;
     double        acc = 0.0;
@@ -923,6 +1007,35 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     with_radix(rl, [&](auto r) { dif_stage<T, decltype(r)::value, INV>(n, m, nc, tw, L.tws, from_lds, to_mem); });
 }
 
+// the same, FP32: the whole tile through LDS; block (bx, o) = blockIdx.x, y
+template <typename T, bool INV>
+__global__ __launch_bounds__(256) void k_fft_strided_stockham(cplx<T> *__restrict__ data, FftLen L,
+                                                     const cplx<T> *__restrict__ tw, int64_t sn, int c0, int c1,
+                                                     int64_t ostride, int bc, Slots sl)
+{
+    const int sb = slot_of(sl);
+    if (sb < 0)
+        return;
+    if (sl.map) {  // batched launch: this slot's buffers
+        data += sb * sl.spec;
+    }
+    extern __shared__ char smem_raw[];
+    cplx<T>  *A     = reinterpret_cast<cplx<T> *>(smem_raw);
+    const int b0    = c0 + blockIdx.x * bc;
+    const int ncols = (c1 - b0) < bc ? (c1 - b0) : bc, ld = ncols + 1;
+    cplx<T>  *base  = data + (int64_t) blockIdx.y * ostride + b0;
+    for (int w = threadIdx.x; w < L.n * ncols; w += blockDim.x) {
+        const int i = w / ncols, c = w - i * ncols;
+        A[i * ld + c] = base[i * sn + c];
+    }
+    __syncthreads();
+    lds_stockham<T, INV>(A, L, tw, ncols, ld);
+    for (int w = threadIdx.x; w < L.n * ncols; w += blockDim.x) {
+        const int i     = w / ncols, c = w - i * ncols;
+        base[i * sn + c] = A[i * ld + c];
+    }
+}
+
 // ---- spectral <r, s> --------------------------------------------------------
 // With s = -G * r, the unnormalised r2c / c2r pair and G holding 1/N,
 // sum_x r(x) s(x) = sum over the full spectrum of conj(r^) s^ (Parseval); the
@@ -931,12 +1044,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
 __device__ __forceinline__ double kz_weight(int kz, int Mc) { return (kz == 0 || kz == Mc - 1) ? 1.0 : 2.0; }
 
 constexpr int kXGreenGroup = 4;
-// largest radix of the x pass: beyond 12 the FP64 pass of three components takes
+// largest radix of the x pass: beyond 12 the pass of three components takes
 // more than 168 registers (two waves per SIMD)
-template <typename T, int H>
+template <int H>
 __host__ __device__ constexpr int kXGreenMaxRadix()
 {
-    return sizeof(T) == 8 && H == 3 ? 12 : 16;
+    return H == 3 ? 12 : 16;
 }
 // lane <- lane (quad base + S) for every lane of a quad (DPP quad_perm broadcast)
 template <int S>
@@ -1058,25 +1171,25 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
         with_prime(rl, [&](auto r) { middle(r, from_mem, to_mem); });
     } else {
         int m = n;
-        with_radix<kXGreenMaxRadix<T, H>()>(L.rad[0],
+        with_radix<kXGreenMaxRadix<H>()>(L.rad[0],
                    [&](auto r) { dif_stage<T, decltype(r)::value, false>(n, m, nc, tw, L.tws, from_mem, to_lds); });
         m /= L.rad[0];
         __syncthreads();
         for (int s = 1; s < L.nst - 1; ++s) {
-            with_radix<kXGreenMaxRadix<T, H>()>(L.rad[s],
+            with_radix<kXGreenMaxRadix<H>()>(L.rad[s],
                        [&](auto r) { dif_stage<T, decltype(r)::value, false>(n, m, nc, tw, L.tws, from_lds, to_lds); });
             m /= L.rad[s];
             __syncthreads();
         }
-        with_radix<kXGreenMaxRadix<T, H>()>(rl, [&](auto r) { middle(r, from_lds, to_lds); });
+        with_radix<kXGreenMaxRadix<H>()>(rl, [&](auto r) { middle(r, from_lds, to_lds); });
         __syncthreads();
         for (int s = L.nst - 2; s > 0; --s) {
             m *= L.rad[s];
-            with_radix<kXGreenMaxRadix<T, H>()>(L.rad[s],
+            with_radix<kXGreenMaxRadix<H>()>(L.rad[s],
                        [&](auto r) { dit_stage<T, decltype(r)::value>(n, m, nc, tw, L.tws, from_lds, to_lds); });
             __syncthreads();
         }
-        with_radix<kXGreenMaxRadix<T, H>()>(L.rad[0], [&](auto r) { dit_stage<T, decltype(r)::value>(n, n, nc, tw, L.tws, from_lds, to_mem); });
+        with_radix<kXGreenMaxRadix<H>()>(L.rad[0], [&](auto r) { dit_stage<T, decltype(r)::value>(n, n, nc, tw, L.tws, from_lds, to_mem); });
     }
     if (partial) {
         double     v1[1] = {acc};
@@ -1084,6 +1197,84 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
         block_reduce<1>(v1, mx, red);
         if (threadIdx.x == 0)
             partial[blockIdx.x] = v1[0];
+    }
+}
+
+// stored block of frequency (kx, ky, kz) and the mirror signs sx, sy
+template <typename T, int H>
+__device__ __forceinline__ const T *green_at(const GreenView<T> &gv, int kx, int ky, int kz, T &sx, T &sy)
+{
+    const bool fx = kx >= gv.gxq, fy = ky >= gv.gyq;
+    sx            = fx ? (T) -1 : (T) 1;
+    sy            = fy ? (T) -1 : (T) 1;
+    const int kxq = fx ? gv.nx - kx : kx, kyq = fy ? gv.ny - ky : ky;
+    return gv.G + (((int64_t) kxq * gv.gyq + kyq) * gv.Mc + kz) * (H * (H + 1) / 2);
+}
+
+// FP32 x+Green pass, the whole tile through LDS; block (bx, y) = blockIdx.x, y;
+// partial index blockIdx.y * gridDim.x + blockIdx.x
+template <typename T, int H>
+__global__ __launch_bounds__(256) void k_fft_x_green_stockham(cplx<T> *__restrict__ data, FftLen L,
+                                                     const cplx<T> *__restrict__ tw, GreenView<T> gv, int kz_lo,
+                                                     int kz_hi, int bk, double *__restrict__ partial, Slots sl)
+{
+    const int sb = slot_of(sl);
+    if (sb < 0)
+        return;
+    if (sl.map) {  // batched launch: this slot's buffers
+        data += sb * sl.spec;
+        gv.G += sb * sl.green;
+        partial = slot_ptr(partial, sb * sl.part);
+    }
+    const int ny = gv.ny, Mc = gv.Mc;
+    __shared__ double red[8];
+    double            acc = 0.0;
+    extern __shared__ char smem_raw[];
+    cplx<T>      *A     = reinterpret_cast<cplx<T> *>(smem_raw);
+    const int     y     = blockIdx.y;
+    const int     kz0   = kz_lo + blockIdx.x * bk;
+    const int     nk    = (kz_hi - kz0) < bk ? (kz_hi - kz0) : bk;
+    const int     ncols = nk * H, ld = ncols + 1;
+    const int64_t sn    = (int64_t) ny * Mc * H;
+    cplx<T>      *base  = data + ((int64_t) y * Mc + kz0) * H;
+    for (int w = threadIdx.x; w < L.n * ncols; w += blockDim.x) {
+        const int i = w / ncols, c = w - i * ncols;
+        A[i * ld + c] = base[i * sn + c];
+    }
+    __syncthreads();
+    lds_stockham<T, false>(A, L, tw, ncols, ld);
+    for (int w = threadIdx.x; w < L.n * nk; w += blockDim.x) {
+        const int i = w / nk, kk = w - i * nk;
+        T         sx, sy;
+        const T  *g = green_at<T, H>(gv, i, y, kz0 + kk, sx, sy);
+        cplx<T>  *v = A + i * ld + kk * H;
+        const double wk = kz_weight(kz0 + kk, Mc);
+        if constexpr (H == 1) {
+            const cplx<T> a = v[0];
+            v[0]            = cscale(a, g[0]);
+            acc -= wk * ((double) a.x * v[0].x + (double) a.y * v[0].y);
+        } else {
+            const cplx<T> a = v[0], b = v[1], c = v[2];
+            const T       g00 = g[0], g01 = g[1] * sx * sy, g02 = g[2] * sx, g11 = g[3], g12 = g[4] * sy, g22 = g[5];
+            v[0]                = cplx<T>{g00 * a.x + g01 * b.x + g02 * c.x, g00 * a.y + g01 * b.y + g02 * c.y};
+            v[1]                = cplx<T>{g01 * a.x + g11 * b.x + g12 * c.x, g01 * a.y + g11 * b.y + g12 * c.y};
+            v[2]                = cplx<T>{g02 * a.x + g12 * b.x + g22 * c.x, g02 * a.y + g12 * b.y + g22 * c.y};
+            acc -= wk * ((double) a.x * v[0].x + (double) a.y * v[0].y + (double) b.x * v[1].x +
+                         (double) b.y * v[1].y + (double) c.x * v[2].x + (double) c.y * v[2].y);
+        }
+    }
+    __syncthreads();
+    lds_stockham<T, true>(A, L, tw, ncols, ld);
+    for (int w = threadIdx.x; w < L.n * ncols; w += blockDim.x) {
+        const int i     = w / ncols, c = w - i * ncols;
+        base[i * sn + c] = A[i * ld + c];
+    }
+    if (partial) {
+        double     v1[1] = {acc};
+        const bool mx[1] = {false};
+        block_reduce<1>(v1, mx, red);
+        if (threadIdx.x == 0)
+            partial[blockIdx.y * gridDim.x + blockIdx.x] = v1[0];
     }
 }
 

@@ -11,14 +11,12 @@ namespace fans {
 // ---------------------------------------------------------------------------
 inline bool reg_len(int n) { return n == 16 || n == 32 || n == 64 || n == 128 || n == 256; }
 inline bool reg_len_y(int n) { return reg_len(n) || n == 96 || n == 80 || n == 48; }
-// the x+Green pass: the powers of two in FP64 (256^3 260 us against 377 with the
-// staged kernel, 128^3 35 against 48), 16 and 32 in FP32 (32^3 conduction 5.3
-// against 5.8; from 64 on the staged kernel is the faster: 128^3 25 against 33,
-// 256^3 133 against 138)
+// the x+Green pass: the powers of two; FP32 also 48, 80 and 96, whose FP64 forms
+// would spill (one wave)
 template <typename T>
 bool x_green_reg(int n)
 {
-    return reg_len(n) && (sizeof(T) == 8 || n <= 32);
+    return sizeof(T) == 8 ? reg_len(n) : reg_len_y(n);
 }
 
 // columns per block: a power of two (>= 4) within ~72 KiB of LDS (two
@@ -69,8 +67,12 @@ void launch_strided(fans_gpu_ctx *c, const FftLen &L, const cplx<T> *tw, int bc,
     case 1: break;
     default: {
         const int nbx = (c1 - c0 + bc - 1) / bc;
-        hipLaunchKernelGGL((k_fft_strided<T, INV>), dim3(nbx * nouter, 1, c->gz), dim3(kThreads), smem, c->stream, spec,
-                           L, tw, sn, c0, c1, ostride, bc, nbx, launch_slots(c, done != nullptr));
+        if constexpr (sizeof(T) == 4)
+            hipLaunchKernelGGL((k_fft_strided_stockham<T, INV>), dim3(nbx, nouter, c->gz), dim3(kThreads), smem, c->stream,
+                               spec, L, tw, sn, c0, c1, ostride, bc, launch_slots(c, done != nullptr));
+        else
+            hipLaunchKernelGGL((k_fft_strided<T, INV>), dim3(nbx * nouter, 1, c->gz), dim3(kThreads), smem, c->stream,
+                               spec, L, tw, sn, c0, c1, ostride, bc, nbx, launch_slots(c, done != nullptr));
     }
     }
 }
@@ -100,22 +102,28 @@ int launch_x_green(fans_gpu_ctx *c, Fft3D<T> &P, cplx<T> *spec, const T *G, int 
                    const int *done)
 {
     const GreenView<T> gv{G, c->nx, c->ny, c->gxq, c->gyq, P.Mc};
-    switch (x_green_reg<T>(P.Lx.n) ? P.Lx.n : 0) {
-    case 256:
-        if constexpr (sizeof(T) == 8)
-            return launch_x_green_reg<T, H, 16, 16>(c, spec, P.twx, gv, kz_lo, kz_hi, partial, done);
-    case 128:
-        if constexpr (sizeof(T) == 8)
-            return launch_x_green_reg<T, H, 16, 8>(c, spec, P.twx, gv, kz_lo, kz_hi, partial, done);
-    case 64:
-        if constexpr (sizeof(T) == 8)
-            return launch_x_green_reg<T, H, 8, 8>(c, spec, P.twx, gv, kz_lo, kz_hi, partial, done);
+    if constexpr (sizeof(T) == 4) {
+        switch (P.Lx.n) {
+        case 96: return launch_x_green_reg<T, H, 24, 4>(c, spec, P.twx, gv, kz_lo, kz_hi, partial, done);
+        case 80: return launch_x_green_reg<T, H, 20, 4>(c, spec, P.twx, gv, kz_lo, kz_hi, partial, done);
+        case 48: return launch_x_green_reg<T, H, 12, 4>(c, spec, P.twx, gv, kz_lo, kz_hi, partial, done);
+        default: break;
+        }
+    }
+    switch (P.Lx.n) {
+    case 256: return launch_x_green_reg<T, H, 16, 16>(c, spec, P.twx, gv, kz_lo, kz_hi, partial, done);
+    case 128: return launch_x_green_reg<T, H, 16, 8>(c, spec, P.twx, gv, kz_lo, kz_hi, partial, done);
+    case 64: return launch_x_green_reg<T, H, 8, 8>(c, spec, P.twx, gv, kz_lo, kz_hi, partial, done);
     case 32: return launch_x_green_reg<T, H, 8, 4>(c, spec, P.twx, gv, kz_lo, kz_hi, partial, done);
     case 16: return launch_x_green_reg<T, H, 4, 4>(c, spec, P.twx, gv, kz_lo, kz_hi, partial, done);
     default: {
         const int nbk = (kz_hi - kz_lo + P.bk - 1) / P.bk;
-        hipLaunchKernelGGL((k_fft_x_green<T, H>), dim3(nbk * c->ny, 1, c->gz), dim3(kThreads), P.smx, c->stream, spec,
-                           P.Lx, P.twx, gv, kz_lo, kz_hi, P.bk, nbk, partial, launch_slots(c, done != nullptr));
+        if constexpr (sizeof(T) == 4)
+            hipLaunchKernelGGL((k_fft_x_green_stockham<T, H>), dim3(nbk, c->ny, c->gz), dim3(kThreads), P.smx, c->stream,
+                               spec, P.Lx, P.twx, gv, kz_lo, kz_hi, P.bk, partial, launch_slots(c, done != nullptr));
+        else
+            hipLaunchKernelGGL((k_fft_x_green<T, H>), dim3(nbk * c->ny, 1, c->gz), dim3(kThreads), P.smx, c->stream, spec,
+                               P.Lx, P.twx, gv, kz_lo, kz_hi, P.bk, nbk, partial, launch_slots(c, done != nullptr));
         return nbk * c->ny;
     }
     }
@@ -126,6 +134,9 @@ int64_t x_green_blocks(const Fft3D<T> &P, int h, int ny)
 {
     int kb = 0;
     switch (x_green_reg<T>(P.Lx.n) ? P.Lx.n : 0) {
+    case 96: kb = reg_cols<T, 24, 4>(); break;
+    case 80: kb = reg_cols<T, 20, 4>(); break;
+    case 48: kb = reg_cols<T, 12, 4>(); break;
     case 256: kb = reg_cols<T, 16, 16>(); break;
     case 128: kb = reg_cols<T, 16, 8>(); break;
     case 64: kb = reg_cols<T, 8, 8>(); break;

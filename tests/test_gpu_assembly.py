@@ -1,4 +1,4 @@
-"""The linear assembly kernel (residual and CG matvec of linear materials) at the
+"""The linear assembly kernels (residual and CG matvec of linear materials) at the
 sizes where its tiling can go wrong, against the oracle: grids below, at and one
 past the 15-node tile in y and z and odd in x, tensors beside isotropic phases
 (staged table, and more phases than it holds), 16-bit ids, per-voxel moduli,
@@ -63,20 +63,23 @@ def test_linear_assembly_against_oracle(model, nph, dims, fe, L):
     p = Problem(dims=dims, howmany=h, ms=ms, groups=groups, fe_type=fe, method="cg", L=L, tol=1e-10, n_it=10)
     u = rng.standard_normal(dims + (h,)) * 0.01
     g0 = rng.uniform(-0.01, 0.01, 3 if h == 1 else 6)
-    o, g = oracle.Oracle(p), gpu.GpuSolver(p, precision="mixed")
-    try:
-        o.set_gradient(g0)
-        g.set_gradient(g0)
-        r_o, k_o = o.residual(u), o.residual(u, linear_kd=True)
-        for planes in (None, 1, 2, 3, dims[0]):
-            if planes:
-                g.set_asm_planes(planes)
-            assert relerr(g.residual(u), r_o) < 1e-12, planes
-            assert relerr(g.residual(u, linear_kd=True), k_o) < 1e-12, planes
-        g.set_operator_fp32(True)
-        assert relerr(g.residual(u, linear_kd=True), k_o) < 1e-5
-    finally:
-        g.close()
+    o = oracle.Oracle(p)
+    o.set_gradient(g0)
+    r_o, k_o = o.residual(u), o.residual(u, linear_kd=True)
+    for precision in ("fp64", "mixed"):  # each form has its own kernel
+        g = gpu.GpuSolver(p, precision=precision)
+        try:
+            g.set_gradient(g0)
+            for planes in (None, 1, 2, 3, dims[0]):
+                if planes:
+                    g.set_asm_planes(planes)
+                assert relerr(g.residual(u), r_o) < 1e-12, (precision, planes)
+                assert relerr(g.residual(u, linear_kd=True), k_o) < 1e-12, (precision, planes)
+            if precision == "mixed":
+                g.set_operator_fp32(True)
+                assert relerr(g.residual(u, linear_kd=True), k_o) < 1e-5
+        finally:
+            g.close()
 
 
 @pytest.mark.parametrize("h,dims,L", [(3, (6, 16, 12), (6.0, 16.0, 12.0)), (3, (5, 9, 18), (1.0, 1.0, 2.0)),
@@ -92,12 +95,14 @@ def test_voxel_moduli_match_phases(h, dims, L):
     p = Problem(dims=dims, howmany=h, ms=ms, groups=groups, fe_type="HEX8", method="cg", L=L, tol=1e-10, n_it=10)
     u = rng.standard_normal(dims + (h,)) * 0.01
     k_o = oracle.Oracle(p).residual(u, linear_kd=True)
-    g = gpu.GpuSolver(p, precision="mixed")
-    try:
-        pr = groups[0].param_matrix()
-        g.set_voxel_moduli(pr[ms, 0], None if h == 1 else pr[ms, 1])
-        assert relerr(g.residual(u, linear_kd=True), k_o) < 1e-12
-        g.set_operator_fp32(True)
-        assert relerr(g.residual(u, linear_kd=True), k_o) < 1e-5
-    finally:
-        g.close()
+    for precision in ("fp64", "mixed"):
+        g = gpu.GpuSolver(p, precision=precision)
+        try:
+            pr = groups[0].param_matrix()
+            g.set_voxel_moduli(pr[ms, 0], None if h == 1 else pr[ms, 1])
+            assert relerr(g.residual(u, linear_kd=True), k_o) < 1e-12
+            if precision == "mixed":
+                g.set_operator_fp32(True)
+                assert relerr(g.residual(u, linear_kd=True), k_o) < 1e-5
+        finally:
+            g.close()
