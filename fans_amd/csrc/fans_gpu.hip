@@ -2144,12 +2144,12 @@ int rebuild_green(fans_gpu_ctx *c)
     c->gxq            = quarter ? c->nx / 2 + 1 : c->nx;
     c->gyq            = quarter ? c->ny / 2 + 1 : c->ny;
     const int64_t ngs = (int64_t) c->gxq * c->gyq * (c->nz / 2 + 1);  // stored frequencies
-    const int     gb  = (int) ((ngs + kThreads - 1) / kThreads);
+    const int     gb  = (int) ((ngs + kGreenThreads - 1) / kGreenThreads);
     if (c->h == 1)
-        hipLaunchKernelGGL((k_build_green<1>), dim3(gb), dim3(kThreads), 0, c->stream, c->keref_d, c->G64, c->nx,
+        hipLaunchKernelGGL((k_build_green<1>), dim3(gb), dim3(kGreenThreads), 0, c->stream, c->keref_d, c->G64, c->nx,
                            c->ny, c->nz, c->gxq, c->gyq);
     else
-        hipLaunchKernelGGL((k_build_green<3>), dim3(gb), dim3(kThreads), 0, c->stream, c->keref_d, c->G64, c->nx,
+        hipLaunchKernelGGL((k_build_green<3>), dim3(gb), dim3(kGreenThreads), 0, c->stream, c->keref_d, c->G64, c->nx,
                            c->ny, c->nz, c->gxq, c->gyq);
     HIPCHK(c, hipGetLastError());
     if (c->d.precision == FANS_PREC_MIXED) {

@@ -19,6 +19,10 @@ __device__ __forceinline__ void jacobi_eig(double (&a)[N][N], double (&V)[N][N])
 #pragma unroll
         for (int j = 0; j < N; ++j)
             V[i][j] = (i == j) ? 1.0 : 0.0;
+    // the off-diagonal falls quadratically; near equal eigenvalues it can settle at
+    // rounding just above the threshold, so a sweep that no longer lowered it ends
+    // the loop (3 to 6 sweeps; one such frequency in 16 took its wave through all 50)
+    double last = HUGE_VAL;
     for (int sweep = 0; sweep < 50; ++sweep) {
         double off = 0.0, tot = 0.0;
 #pragma unroll
@@ -29,8 +33,9 @@ __device__ __forceinline__ void jacobi_eig(double (&a)[N][N], double (&V)[N][N])
                 if (i != j)
                     off += a[i][j] * a[i][j];
             }
-        if (off <= 1e-32 * tot || off == 0.0)
+        if (off <= 1e-32 * tot || off == 0.0 || !(off < last))
             break;
+        last = off;
 #pragma unroll
         for (int p = 0; p < N; ++p)
 #pragma unroll
@@ -63,11 +68,16 @@ __device__ __forceinline__ void jacobi_eig(double (&a)[N][N], double (&V)[N][N])
     }
 }
 
+constexpr int kGreenThreads = 64;
+
 // keref: component-major (8H)x(8H) reference element stiffness (matmodel.h:237-253)
 // G: [gxq][gyq][nz/2+1][H(H+1)/2] packed (00 01 02 11 12 22) for the stored
 // frequencies kx < gxq, ky < gyq (see GreenView)
+// One-wave workgroups: the 36k stored frequencies of 64^3 spread over the chip
+// (18.5 us; 139 with A in scratch memory, four-wave workgroups and the sweeps that
+// jacobi_eig now ends).  Bound by the chains of divisions and square roots.
 template <int H>
-__global__ __launch_bounds__(256) void k_build_green(const double *__restrict__ keref, double *__restrict__ G, int nx,
+__global__ __launch_bounds__(kGreenThreads) void k_build_green(const double *__restrict__ keref, double *__restrict__ G, int nx,
                                                      int ny, int nz, int gxq, int gyq)
 {
     constexpr int NP = H * (H + 1) / 2, NE = 8 * H;
@@ -99,18 +109,34 @@ __global__ __launch_bounds__(256) void k_build_green(const double *__restrict__ 
     A[5] = cmul(ex, ez);
     A[6] = cmul(ez, ey);
     A[7] = cmul(cmul(ex, ey), ez);
-    double blk[H][H];
+    // corner pairs outermost and unrolled: A stays in registers (indexed at run time
+    // it lived in scratch memory), each product serves all blocks; every block still
+    // sums its 64 terms in the order of (a, b)
+    double acc[NP];
 #pragma unroll
-    for (int i = 0; i < H; ++i)
+    for (int k = 0; k < NP; ++k)
+        acc[k] = 0.0;
 #pragma unroll
-        for (int j = i; j < H; ++j) {
-            double acc = 0.0;
-            for (int a = 0; a < 8; ++a)
-                for (int b = 0; b < 8; ++b)
-                    acc += keref[(8 * i + a) * NE + 8 * j + b] * (A[a].x * A[b].x + A[a].y * A[b].y);
-            blk[i][j] = acc;
-            blk[j][i] = acc;
+    for (int a = 0; a < 8; ++a)
+#pragma unroll
+        for (int b = 0; b < 8; ++b) {
+            const double AA = A[a].x * A[b].x + A[a].y * A[b].y;
+            int          k  = 0;
+#pragma unroll
+            for (int i = 0; i < H; ++i)
+#pragma unroll
+                for (int j = i; j < H; ++j)
+                    acc[k++] += keref[(8 * i + a) * NE + 8 * j + b] * AA;
         }
+    double blk[H][H];
+    {
+        int k = 0;
+#pragma unroll
+        for (int i = 0; i < H; ++i)
+#pragma unroll
+            for (int j = i; j < H; ++j)
+                blk[i][j] = blk[j][i] = acc[k++];
+    }
     double V[H][H];
     jacobi_eig<H>(blk, V);
     const double Nd = (double) ((int64_t) nx * ny * nz);  // solver.h:198 divides by N
