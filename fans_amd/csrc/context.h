@@ -23,6 +23,9 @@
 
 namespace fans {
 
+struct HostScalars;  // vec_kernels.h
+struct MixedCtl;
+
 constexpr int kThreads = 256;
 
 // kernel families for the timing report
@@ -329,6 +332,9 @@ struct fans_gpu_ctx {
     int64_t       partial_len = 0;
     double       *partial_e   = nullptr;  // [nblk_z] of the linear CG's inverse z pass
     int64_t       partial_e_len = 0;
+    // nonlinear CG: scalars in pinned host memory, mixed-control state
+    HostScalars  *nl_host     = nullptr;
+    MixedCtl     *nl_ctl      = nullptr;
     double       *sc = nullptr;
     int          *is = nullptr;
     double       *hist = nullptr;

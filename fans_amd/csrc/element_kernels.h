@@ -1257,7 +1257,7 @@ __global__ __launch_bounds__(256) void k_element_pass(ElemArgs<T> a)
 {
     __shared__ double red[NS * 4];
     {
-        const int sb = slot_of(a.sl, false);
+        const int sb = slot_of(a.sl);
         if (sb < 0)
             return;
         if (a.sl.map) {  // batched launch: this slot's buffers

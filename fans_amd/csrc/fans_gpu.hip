@@ -265,7 +265,7 @@ void clear_map(fans_gpu_ctx *c)
 }
 
 int reduce(fans_gpu_ctx *c, const double *partial, int nblk, int nq, int stage, const double *partial_b = nullptr,
-           int nblk_b = 0);
+           int nblk_b = 0, const ReduceSide &side = {});
 
 // ---------------------------------------------------------------------------
 // FFT convolution: out = G * r  with the requested epilogue.  With `pro` the
@@ -487,7 +487,7 @@ int launch_assemble(fans_gpu_ctx *c, AsmArgs<T> a)
 }
 
 // r = R(u) (material path with g0); partial slot 0 = norm(r), slot 1 = <r, dotv>
-int residual64(fans_gpu_ctx *c, const double *uin, double *rout, const double *dotv)
+int residual64(fans_gpu_ctx *c, const double *uin, double *rout, const double *dotv, bool gated = false)
 {
     AsmArgs<double> a = asm_args<double>(c);
     a.phases          = c->dph64;
@@ -495,15 +495,16 @@ int residual64(fans_gpu_ctx *c, const double *uin, double *rout, const double *d
     a.out             = rout;
     a.dotv            = dotv;
     a.g0              = c->g0d;
+    a.sl              = launch_slots(c, gated);
     return launch_assemble<double, ASM_RESID>(c, a);
 }
 
 int reduce(fans_gpu_ctx *c, const double *partial, int nblk, int nq, int stage, const double *partial_b,
-           int nblk_b)
+           int nblk_b, const ReduceSide &side)
 {
     Timed t(c, KF_REDUCE);
     hipLaunchKernelGGL(k_reduce, dim3(1, 1, c->gz), dim3(kReduceThreads), 0, c->stream, partial, nblk, nq, stage, c->sc,
-                       c->is, c->hist, partial_b, nblk_b, launch_slots(c, false));
+                       c->is, c->hist, partial_b, nblk_b, launch_slots(c, false), side);
     HIPCHK(c, hipGetLastError());
     return 0;
 }
@@ -550,8 +551,8 @@ int upload_g0(fans_gpu_ctx *c)
     return 0;
 }
 
-// Solver::get_homogenized_stress (solver.h:707-737)
-int homog_stress(fans_gpu_ctx *c, double *out)
+// partial sums of the stress over the elements (n_str quantities, nblk_el blocks)
+int stress_partials(fans_gpu_ctx *c, bool gated = false)
 {
     ElemArgs<double> a{};
     a.nx      = c->nx;
@@ -568,7 +569,7 @@ int homog_stress(fans_gpu_ctx *c, double *out)
     a.vk      = c->voxel_moduli ? c->vk64 : nullptr;
     a.vg      = c->voxel_moduli ? c->vg64 : nullptr;
     a.partial = c->partial;
-    a.sl      = launch_slots(c, false);
+    a.sl      = launch_slots(c, gated);
     {
         Timed t(c, KF_ELEMENT);
 #define EP(HH, GG)                                                                                              \
@@ -595,8 +596,14 @@ int homog_stress(fans_gpu_ctx *c, double *out)
 #undef EP
     }
     HIPCHK(c, hipGetLastError());
-    int rc = reduce(c, c->partial, c->nblk_el, c->nstr, RED_SUM);
-    if (rc || !out)
+    return 0;
+}
+
+// Solver::get_homogenized_stress (solver.h:707-737)
+int homog_stress(fans_gpu_ctx *c, double *out)
+{
+    int rc;
+    if ((rc = stress_partials(c)) || (rc = reduce(c, c->partial, c->nblk_el, c->nstr, RED_SUM)) || !out)
         return rc;
     double sc[SC_COUNT];
     if ((rc = read_scalars(c, sc, nullptr)))
@@ -658,6 +665,51 @@ int mixed_update(fans_gpu_ctx *c)
         for (int i = 0; i < nF; ++i)
             c->gvec[c->idxF[i]] += dE[i];
     }
+    for (int i = 0; i < c->nstr; ++i)
+        c->g0[i] = c->gvec[i];
+    return upload_g0(c);
+}
+
+// the nonlinear CG's scalars for the host and its mixed controller's state at the
+// start of a solve
+int start_nonlinear(fans_gpu_ctx *c, ReduceSide &side)
+{
+    if (!c->nl_host)
+        HIPCHK(c, hipHostMalloc(reinterpret_cast<void **>(&c->nl_host), sizeof(HostScalars), hipHostMallocCoherent));
+    if (!c->nl_ctl)
+        HIPCHK(c, hipMalloc(&c->nl_ctl, sizeof(MixedCtl)));
+    side = ReduceSide{c->nl_host, c->nl_ctl, c->g0d};
+    if (!c->mixed_active)
+        return 0;
+    MixedCtl m{};
+    m.nF   = (int) c->idxF.size();
+    m.nstr = c->nstr;
+    m.N    = (double) c->N;
+    std::copy(c->idxF.begin(), c->idxF.end(), m.idx);
+    std::copy(c->M.begin(), c->M.end(), m.M);
+    for (int i = 0; i < m.nF; ++i)
+        m.PF[i] = c->PF[(size_t) c->step * m.nF + i];
+    std::copy(c->gvec, c->gvec + 9, m.g);
+    HIPCHK(c, copy_on(c, c->nl_ctl, &m, sizeof(m), hipMemcpyHostToDevice));
+    return 0;
+}
+// mixed_update() of the nonlinear CG: nothing for the host (gated: nothing at all
+// once the stop test holds)
+int mixed_update_dev(fans_gpu_ctx *c, const ReduceSide &side)
+{
+    if (!c->mixed_active)
+        return 0;
+    const int rc = stress_partials(c, true);
+    return rc ? rc : reduce(c, c->partial, c->nblk_el, c->nstr, RED_MIXED, nullptr, 0, side);
+}
+// the controller's gradient back on the host
+int finish_nonlinear(fans_gpu_ctx *c)
+{
+    if (!c->mixed_active)
+        return 0;
+    MixedCtl m;
+    HIPCHK(c, copy_on(c, &m, c->nl_ctl, sizeof(m), hipMemcpyDeviceToHost));
+    std::copy(m.g, m.g + 9, c->gvec);
     for (int i = 0; i < c->nstr; ++i)
         c->g0[i] = c->gvec[i];
     return upload_g0(c);
@@ -1035,22 +1087,32 @@ int solve_cg_fp64(fans_gpu_ctx *c)
         c->iter = it;
         return fetch_history(c, it);
     }
-    // nonlinear CG with the secant line search (solverCG.h:84-160)
-    int    is[IS_COUNT];
-    double sc[SC_COUNT];
+    // nonlinear CG with the secant line search (solverCG.h:84-160).  The host
+    // waits once per evaluation, for <r, d>: every other scalar stays on the device,
+    // and the launches of an iteration up to its first evaluation are queued before
+    // its stop test is known, gated by the done flag.
+    int is[IS_COUNT];
     if ((rc = read_scalars(c, nullptr, is)))
         return rc;
-    double *d = c->dA;
-    while (!is[IS_DONE]) {
+    ReduceSide side;
+    if ((rc = start_nonlinear(c, side)))
+        return rc;
+    const int *const done = c->is + IS_DONE;
+    auto             wait = [&]() -> int {
+        HIPCHK(c, hipStreamSynchronize(c->stream));
+        return 0;
+    };
+    HostScalars &hs = *c->nl_host;
+    hs.done         = is[IS_DONE];
+    hs.iter         = is[IS_ITER];
+    double *d       = c->dA;
+    while (!hs.done) {
+        const size_t mark = c->ev_used.size();
         // deltamid = <r, s>
         hipLaunchKernelGGL((k_dot<double>), dim3(c->nblk_vec), dim3(kThreads), 0, c->stream, c->r, c->s, c->Nh,
                            c->d.measure, c->partial);
-        if ((rc = reduce(c, c->partial, c->nblk_vec, 1, RED_SUM)))
+        if ((rc = reduce(c, c->partial, c->nblk_vec, 1, RED_DELTAMID)))
             return rc;
-        if ((rc = read_scalars(c, sc, nullptr)))
-            return rc;
-        HIPCHK(c, hipMemcpyAsync(c->sc + SC_DELTAMID, &sc[SC_RES0], sizeof(double), hipMemcpyHostToDevice,
-                                 c->stream));
         if (c->d.precision == FANS_PREC_MIXED) {
             // mixed form of the nonlinear solve: the Green preconditioner s = -G r
             // in FP32 (FFTs and Green multiply); residuals, the J2 return map,
@@ -1061,7 +1123,7 @@ int solve_cg_fp64(fans_gpu_ctx *c)
             ep.out     = c->s32;
             ep.r       = c->r32;
             ep.partial = c->partial;
-            if ((rc = convolve_dev<float>(c, c->fft32, c->r32, c->spec32, c->G32, EPI_CG, ep, nullptr)))
+            if ((rc = convolve_dev<float>(c, c->fft32, c->r32, c->spec32, c->G32, EPI_CG, ep, done)))
                 return rc;
             hipLaunchKernelGGL((k_convert<double, float>), dim3(c->nblk_vec), dim3(kThreads), 0, c->stream, c->s,
                                c->s32, c->Nh);
@@ -1074,7 +1136,7 @@ int solve_cg_fp64(fans_gpu_ctx *c)
             ep.out     = c->s;
             ep.r       = c->r;
             ep.partial = c->partial;
-            if ((rc = convolve_dev<double>(c, c->fft64, c->r, c->spec64, c->G64, EPI_CG, ep, nullptr)))
+            if ((rc = convolve_dev<double>(c, c->fft64, c->r, c->spec64, c->G64, EPI_CG, ep, done)))
                 return rc;
             if ((rc = reduce(c, c->partial, (int) c->fft64.nblk_z, 1, RED_DELTA)))
                 return rc;
@@ -1088,17 +1150,17 @@ int solve_cg_fp64(fans_gpu_ctx *c)
         {
             Timed tv(c, KF_VECTOR);
             hipLaunchKernelGGL((k_ls_start<double>), dim3(c->nblk_vec), dim3(kThreads), 0, c->stream, d, c->s, c->r,
-                               c->u, c->sc, ac, c->Nh, c->partial);
+                               c->u, c->sc, ac, c->Nh, c->partial, done);
         }
-        if ((rc = reduce(c, c->partial, c->nblk_vec, 1, RED_SUM)) || (rc = read_scalars(c, sc, nullptr)))
+        if ((rc = reduce(c, c->partial, c->nblk_vec, 1, RED_RPD, nullptr, 0, side)) ||
+            (rc = mixed_update_dev(c, side)) || (rc = residual64(c, c->u, c->rnew, d, true)) ||
+            (rc = reduce(c, c->partial + c->nblk_asm, c->nblk_asm, 1, RED_SUM, nullptr, 0, side)) || (rc = wait()))
             return rc;
-        double rpd = sc[SC_RES0];
-        if ((rc = mixed_update(c)) || (rc = residual64(c, c->u, c->rnew, d)))
-            return rc;
-        if ((rc = reduce(c, c->partial + c->nblk_asm, c->nblk_asm, 1, RED_SUM)) ||
-            (rc = read_scalars(c, sc, nullptr)))
-            return rc;
-        double r1pd = sc[SC_RES0];
+        if (hs.done) {
+            drop_timing(c, mark);
+            break;
+        }
+        double rpd = hs.rpd, r1pd = hs.sum;
         while (lit < MaxIt && lerr > ltol) {
             double denom = r1pd - rpd;
             if (std::fabs(denom) < 1e-14 * (std::fabs(r1pd) + std::fabs(rpd)))
@@ -1113,20 +1175,20 @@ int solve_cg_fp64(fans_gpu_ctx *c)
             rpd = r1pd;
             ac  = an;
             lit++;
-            if ((rc = mixed_update(c)) || (rc = residual64(c, c->u, c->rnew, d)))
+            if ((rc = mixed_update_dev(c, side)) || (rc = residual64(c, c->u, c->rnew, d)) ||
+                (rc = reduce(c, c->partial + c->nblk_asm, c->nblk_asm, 1, RED_SUM, nullptr, 0, side)) || (rc = wait()))
                 return rc;
-            if ((rc = reduce(c, c->partial + c->nblk_asm, c->nblk_asm, 1, RED_SUM)) ||
-                (rc = read_scalars(c, sc, nullptr)))
-                return rc;
-            r1pd = sc[SC_RES0];
+            r1pd = hs.sum;
         }
         c->alpha_warm = (lit == MaxIt && lerr > ltol) ? 0.1 : ac;
         std::swap(c->r, c->rnew);
         // the last residual evaluation left norm(rnew) partials in slot 0
-        if ((rc = reduce(c, c->partial, c->nblk_asm, 1, RED_ERR_NEXT)) || (rc = read_scalars(c, nullptr, is)))
+        if ((rc = reduce(c, c->partial, c->nblk_asm, 1, RED_ERR_NEXT, nullptr, 0, side)))
             return rc;
     }
-    c->iter = is[IS_ITER];
+    c->iter = hs.iter;
+    if ((rc = finish_nonlinear(c)))
+        return rc;
     return fetch_history(c, c->iter);
 }
 
@@ -1764,13 +1826,15 @@ void free_all(fans_gpu_ctx *c)
         set_views(c, 0);  // the fields hold the allocations again
     if (c->slot_map)
         (void) hipFree(c->slot_map);
+    if (c->nl_host)
+        (void) hipHostFree(c->nl_host);
     for (void *p : {(void *) c->ms, (void *) c->dph64, (void *) c->dph32, (void *) c->u, (void *) c->u_prev,
                     (void *) c->r, (void *) c->s, (void *) c->dA, (void *) c->dB, (void *) c->rnew,
                     (void *) c->spec64, (void *) c->G64, (void *) c->keref_d, (void *) c->G32, (void *) c->js,
                     (void *) c->g0d, (void *) c->g0f, (void *) c->partial, (void *) c->partial_e, (void *) c->sc, (void *) c->is,
                     (void *) c->hist, (void *) c->r32, (void *) c->s32, (void *) c->dA32, (void *) c->dB32,
                     (void *) c->rnew32, (void *) c->x32, (void *) c->spec32, (void *) c->vk64, (void *) c->vg64,
-                    (void *) c->vk32, (void *) c->vg32, (void *) c->ub_d, (void *) c->sens_d})
+                    (void *) c->vk32, (void *) c->vg32, (void *) c->ub_d, (void *) c->sens_d, (void *) c->nl_ctl})
         if (p)
             (void) hipFree(p);
     for (int m = 2; m < kDirRing; ++m) {

@@ -17,8 +17,53 @@ enum {
     RED_ALPHA    = 2,  // q0 = <d,rnew>, q1 = <d,rnew_prev> (nq 1: zero) -> alpha, deltamid
     RED_ERR_NEXT = 4,  // q0 = norm partials      -> err, iter++
     RED_SUM      = 5,  // q0..q(nq-1) sums        -> SC_RES0 + q
-    RED_ERR_SET  = 6   // q0 = norm partials      -> err, stop test (iteration and CG scalars kept)
+    RED_ERR_SET  = 6,  // q0 = norm partials      -> err, stop test (iteration and CG scalars kept)
+    RED_DELTAMID = 7,  // q0 = <r,s> partials     -> deltamid
+    RED_RPD      = 8,  // q0 = <r,d> partials     -> the host's rpd
+    RED_MIXED    = 9   // q0..q(nstr-1) = stress sums -> mixed strain / stress controller (MixedCtl)
 };
+
+// What the host reads of the nonlinear CG, in pinned host memory: the reductions
+// store it there, so that the host only waits for the stream (a copy to the host
+// cost a launch of 3.5 us and its own gap, each time; with MixedCtl and the waits
+// that fall away, a 5-step J2 ramp at 64^3 went from 116 to 84.5 ms)
+struct HostScalars {
+    double sum, rpd;  // RED_SUM of one quantity, RED_RPD
+    int    done, iter;
+};
+// Mixed strain / stress controller (mixedBCs.h:150-227) on the device: the
+// macroscopic gradient g follows g_F += M (PF - Pbar_F) with Pbar the mean stress.
+// On the host it took a copy to it, two from it and a synchronisation in every
+// line-search evaluation.
+struct MixedCtl {
+    int    nF, nstr, idx[9];
+    double N, M[81], PF[9], g[9];
+};
+struct ReduceSide {
+    HostScalars *host = nullptr;
+    MixedCtl    *ctl  = nullptr;
+    double      *g0   = nullptr;  // the macroscopic gradient of the kernels
+};
+// the operations of the host's controller, in its order and without contraction
+__device__ __forceinline__ void mixed_step(MixedCtl &m, const double (&sum)[10], double *g0)
+{
+#pragma clang fp contract(off)
+    double rhs[9];
+    for (int i = 0; i < m.nF; ++i) {
+        double P = 0.0;
+        for (int k = 0; k < 9; ++k)
+            P = k == m.idx[i] ? sum[k] : P;
+        rhs[i] = m.PF[i] - P / m.N;
+    }
+    for (int i = 0; i < m.nF; ++i) {
+        double dE = 0.0;
+        for (int j = 0; j < m.nF; ++j)
+            dE += m.M[i * m.nF + j] * rhs[j];
+        m.g[m.idx[i]] += dE;
+    }
+    for (int i = 0; i < m.nstr; ++i)
+        g0[i] = m.g[i];
+}
 
 // one block of kReduceThreads; each thread folds its strided partials into
 // four independent accumulators (fixed order) before the block reduction
@@ -30,7 +75,7 @@ constexpr int kReduceThreads = 1024;
 __global__ __launch_bounds__(kReduceThreads) void k_reduce(const double *__restrict__ partial, int nblk, int nq,
                                                            int stage, double *sc, int *is, double *hist,
                                                            const double *__restrict__ partial_b, int nblk_b,
-                                                           Slots sl)
+                                                           Slots sl, ReduceSide side)
 {
     __shared__ double sm[2 * (kReduceThreads / 64)];
     const int         sb = slot_of(sl, false);
@@ -46,7 +91,7 @@ __global__ __launch_bounds__(kReduceThreads) void k_reduce(const double *__restr
     const int measure = is[IS_MEASURE];
     if (stage != RED_ERR_INIT && stage != RED_SUM && stage != RED_ERR_SET && is[IS_DONE])
         return;
-    double v[2] = {0.0, 0.0};
+    double v[2] = {0.0, 0.0}, sums[10] = {};
     bool   mx[2];
     for (int q = 0; q < nq; q += 2) {
         const int nqq = (nq - q) < 2 ? 1 : 2;
@@ -76,6 +121,19 @@ __global__ __launch_bounds__(kReduceThreads) void k_reduce(const double *__restr
                 sc[SC_RES0 + q] = v[0];
                 if (nqq == 2)
                     sc[SC_RES0 + q + 1] = v[1];
+                if (side.host)
+                    side.host->sum = v[0];
+            } else if (stage == RED_MIXED) {
+#pragma unroll
+                for (int k = 0; k < 10; k += 2)
+                    if (k == q)
+                        sums[k] = v[0], sums[k + 1] = v[1];
+                if (q + 2 >= nq)
+                    mixed_step(*side.ctl, sums, side.g0);
+            } else if (stage == RED_DELTAMID) {
+                sc[SC_DELTAMID] = v[0];
+            } else if (stage == RED_RPD) {
+                side.host->rpd = v[0];
             } else {
                 const StageScalars S = load_stage_scalars(sc, is);
                 if (stage == RED_ERR_INIT) {
@@ -97,6 +155,10 @@ __global__ __launch_bounds__(kReduceThreads) void k_reduce(const double *__restr
                 } else if (stage == RED_ERR_NEXT) {
                     is[IS_ITER] = S.iter + 1;
                     record_error(sc, is, hist, S, S.iter + 1, finish_norm(v[0], measure));
+                    if (side.host) {
+                        side.host->done = is[IS_DONE];
+                        side.host->iter = S.iter + 1;
+                    }
                 } else if (stage == RED_ERR_SET) {
                     record_error(sc, is, hist, S, S.iter, finish_norm(v[0], measure));
                 }
@@ -301,8 +363,10 @@ template <typename T>
 __global__ __launch_bounds__(256) void k_ls_start(T *__restrict__ d, const T *__restrict__ s,
                                                   const T *__restrict__ r, T *__restrict__ u,
                                                   const double *__restrict__ sc, double alpha0, int64_t n,
-                                                  double *__restrict__ partial)
+                                                  double *__restrict__ partial, const int *__restrict__ done)
 {
+    if (*done)
+        return;
     __shared__ double sm[8];
     const T           beta = (T) sc[SC_BETA];
     double            a0   = 0.0;
