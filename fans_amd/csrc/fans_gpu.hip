@@ -265,7 +265,7 @@ void clear_map(fans_gpu_ctx *c)
 }
 
 int reduce(fans_gpu_ctx *c, const double *partial, int nblk, int nq, int stage, const double *partial_b = nullptr,
-           int nblk_b = 0, const ReduceSide &side = {});
+           int nblk_b = 0, HostScalars *host = nullptr);
 
 // ---------------------------------------------------------------------------
 // FFT convolution: out = G * r  with the requested epilogue.  With `pro` the
@@ -500,11 +500,11 @@ int residual64(fans_gpu_ctx *c, const double *uin, double *rout, const double *d
 }
 
 int reduce(fans_gpu_ctx *c, const double *partial, int nblk, int nq, int stage, const double *partial_b,
-           int nblk_b, const ReduceSide &side)
+           int nblk_b, HostScalars *host)
 {
     Timed t(c, KF_REDUCE);
     hipLaunchKernelGGL(k_reduce, dim3(1, 1, c->gz), dim3(kReduceThreads), 0, c->stream, partial, nblk, nq, stage, c->sc,
-                       c->is, c->hist, partial_b, nblk_b, launch_slots(c, false), side);
+                       c->is, c->hist, partial_b, nblk_b, launch_slots(c, false), host);
     HIPCHK(c, hipGetLastError());
     return 0;
 }
@@ -672,13 +672,12 @@ int mixed_update(fans_gpu_ctx *c)
 
 // the nonlinear CG's scalars for the host and its mixed controller's state at the
 // start of a solve
-int start_nonlinear(fans_gpu_ctx *c, ReduceSide &side)
+int start_nonlinear(fans_gpu_ctx *c)
 {
     if (!c->nl_host)
         HIPCHK(c, hipHostMalloc(reinterpret_cast<void **>(&c->nl_host), sizeof(HostScalars), hipHostMallocCoherent));
     if (!c->nl_ctl)
         HIPCHK(c, hipMalloc(&c->nl_ctl, sizeof(MixedCtl)));
-    side = ReduceSide{c->nl_host, c->nl_ctl, c->g0d};
     if (!c->mixed_active)
         return 0;
     MixedCtl m{};
@@ -695,12 +694,17 @@ int start_nonlinear(fans_gpu_ctx *c, ReduceSide &side)
 }
 // mixed_update() of the nonlinear CG: nothing for the host (gated: nothing at all
 // once the stop test holds)
-int mixed_update_dev(fans_gpu_ctx *c, const ReduceSide &side)
+int mixed_update_dev(fans_gpu_ctx *c)
 {
     if (!c->mixed_active)
         return 0;
-    const int rc = stress_partials(c, true);
-    return rc ? rc : reduce(c, c->partial, c->nblk_el, c->nstr, RED_MIXED, nullptr, 0, side);
+    if (const int rc = stress_partials(c, true))
+        return rc;
+    Timed t(c, KF_REDUCE);
+    hipLaunchKernelGGL(k_mixed_control, dim3(1), dim3(kReduceThreads), 0, c->stream, c->partial, c->nblk_el, c->nl_ctl,
+                       c->g0d, c->is);
+    HIPCHK(c, hipGetLastError());
+    return 0;
 }
 // the controller's gradient back on the host
 int finish_nonlinear(fans_gpu_ctx *c)
@@ -1094,8 +1098,7 @@ int solve_cg_fp64(fans_gpu_ctx *c)
     int is[IS_COUNT];
     if ((rc = read_scalars(c, nullptr, is)))
         return rc;
-    ReduceSide side;
-    if ((rc = start_nonlinear(c, side)))
+    if ((rc = start_nonlinear(c)))
         return rc;
     const int *const done = c->is + IS_DONE;
     auto             wait = [&]() -> int {
@@ -1152,9 +1155,9 @@ int solve_cg_fp64(fans_gpu_ctx *c)
             hipLaunchKernelGGL((k_ls_start<double>), dim3(c->nblk_vec), dim3(kThreads), 0, c->stream, d, c->s, c->r,
                                c->u, c->sc, ac, c->Nh, c->partial, done);
         }
-        if ((rc = reduce(c, c->partial, c->nblk_vec, 1, RED_RPD, nullptr, 0, side)) ||
-            (rc = mixed_update_dev(c, side)) || (rc = residual64(c, c->u, c->rnew, d, true)) ||
-            (rc = reduce(c, c->partial + c->nblk_asm, c->nblk_asm, 1, RED_SUM, nullptr, 0, side)) || (rc = wait()))
+        if ((rc = reduce(c, c->partial, c->nblk_vec, 1, RED_RPD, nullptr, 0, &hs)) ||
+            (rc = mixed_update_dev(c)) || (rc = residual64(c, c->u, c->rnew, d, true)) ||
+            (rc = reduce(c, c->partial + c->nblk_asm, c->nblk_asm, 1, RED_SUM, nullptr, 0, &hs)) || (rc = wait()))
             return rc;
         if (hs.done) {
             drop_timing(c, mark);
@@ -1175,15 +1178,15 @@ int solve_cg_fp64(fans_gpu_ctx *c)
             rpd = r1pd;
             ac  = an;
             lit++;
-            if ((rc = mixed_update_dev(c, side)) || (rc = residual64(c, c->u, c->rnew, d)) ||
-                (rc = reduce(c, c->partial + c->nblk_asm, c->nblk_asm, 1, RED_SUM, nullptr, 0, side)) || (rc = wait()))
+            if ((rc = mixed_update_dev(c)) || (rc = residual64(c, c->u, c->rnew, d)) ||
+                (rc = reduce(c, c->partial + c->nblk_asm, c->nblk_asm, 1, RED_SUM, nullptr, 0, &hs)) || (rc = wait()))
                 return rc;
             r1pd = hs.sum;
         }
         c->alpha_warm = (lit == MaxIt && lerr > ltol) ? 0.1 : ac;
         std::swap(c->r, c->rnew);
         // the last residual evaluation left norm(rnew) partials in slot 0
-        if ((rc = reduce(c, c->partial, c->nblk_asm, 1, RED_ERR_NEXT, nullptr, 0, side)))
+        if ((rc = reduce(c, c->partial, c->nblk_asm, 1, RED_ERR_NEXT, nullptr, 0, &hs)))
             return rc;
     }
     c->iter = hs.iter;

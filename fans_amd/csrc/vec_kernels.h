@@ -19,8 +19,7 @@ enum {
     RED_SUM      = 5,  // q0..q(nq-1) sums        -> SC_RES0 + q
     RED_ERR_SET  = 6,  // q0 = norm partials      -> err, stop test (iteration and CG scalars kept)
     RED_DELTAMID = 7,  // q0 = <r,s> partials     -> deltamid
-    RED_RPD      = 8,  // q0 = <r,d> partials     -> the host's rpd
-    RED_MIXED    = 9   // q0..q(nstr-1) = stress sums -> mixed strain / stress controller (MixedCtl)
+    RED_RPD      = 8   // q0 = <r,d> partials     -> the host's rpd
 };
 
 // What the host reads of the nonlinear CG, in pinned host memory: the reductions
@@ -39,32 +38,6 @@ struct MixedCtl {
     int    nF, nstr, idx[9];
     double N, M[81], PF[9], g[9];
 };
-struct ReduceSide {
-    HostScalars *host = nullptr;
-    MixedCtl    *ctl  = nullptr;
-    double      *g0   = nullptr;  // the macroscopic gradient of the kernels
-};
-// the operations of the host's controller, in its order and without contraction
-__device__ __forceinline__ void mixed_step(MixedCtl &m, const double (&sum)[10], double *g0)
-{
-#pragma clang fp contract(off)
-    double rhs[9];
-    for (int i = 0; i < m.nF; ++i) {
-        double P = 0.0;
-        for (int k = 0; k < 9; ++k)
-            P = k == m.idx[i] ? sum[k] : P;
-        rhs[i] = m.PF[i] - P / m.N;
-    }
-    for (int i = 0; i < m.nF; ++i) {
-        double dE = 0.0;
-        for (int j = 0; j < m.nF; ++j)
-            dE += m.M[i * m.nF + j] * rhs[j];
-        m.g[m.idx[i]] += dE;
-    }
-    for (int i = 0; i < m.nstr; ++i)
-        g0[i] = m.g[i];
-}
-
 // one block of kReduceThreads; each thread folds its strided partials into
 // four independent accumulators (fixed order) before the block reduction
 constexpr int kReduceThreads = 1024;
@@ -75,7 +48,7 @@ constexpr int kReduceThreads = 1024;
 __global__ __launch_bounds__(kReduceThreads) void k_reduce(const double *__restrict__ partial, int nblk, int nq,
                                                            int stage, double *sc, int *is, double *hist,
                                                            const double *__restrict__ partial_b, int nblk_b,
-                                                           Slots sl, ReduceSide side)
+                                                           Slots sl, HostScalars *host)
 {
     __shared__ double sm[2 * (kReduceThreads / 64)];
     const int         sb = slot_of(sl, false);
@@ -91,7 +64,7 @@ __global__ __launch_bounds__(kReduceThreads) void k_reduce(const double *__restr
     const int measure = is[IS_MEASURE];
     if (stage != RED_ERR_INIT && stage != RED_SUM && stage != RED_ERR_SET && is[IS_DONE])
         return;
-    double v[2] = {0.0, 0.0}, sums[10] = {};
+    double v[2] = {0.0, 0.0};
     bool   mx[2];
     for (int q = 0; q < nq; q += 2) {
         const int nqq = (nq - q) < 2 ? 1 : 2;
@@ -121,19 +94,12 @@ __global__ __launch_bounds__(kReduceThreads) void k_reduce(const double *__restr
                 sc[SC_RES0 + q] = v[0];
                 if (nqq == 2)
                     sc[SC_RES0 + q + 1] = v[1];
-                if (side.host)
-                    side.host->sum = v[0];
-            } else if (stage == RED_MIXED) {
-#pragma unroll
-                for (int k = 0; k < 10; k += 2)
-                    if (k == q)
-                        sums[k] = v[0], sums[k + 1] = v[1];
-                if (q + 2 >= nq)
-                    mixed_step(*side.ctl, sums, side.g0);
+                if (host)
+                    host->sum = v[0];
             } else if (stage == RED_DELTAMID) {
                 sc[SC_DELTAMID] = v[0];
             } else if (stage == RED_RPD) {
-                side.host->rpd = v[0];
+                host->rpd = v[0];
             } else {
                 const StageScalars S = load_stage_scalars(sc, is);
                 if (stage == RED_ERR_INIT) {
@@ -155,9 +121,9 @@ __global__ __launch_bounds__(kReduceThreads) void k_reduce(const double *__restr
                 } else if (stage == RED_ERR_NEXT) {
                     is[IS_ITER] = S.iter + 1;
                     record_error(sc, is, hist, S, S.iter + 1, finish_norm(v[0], measure));
-                    if (side.host) {
-                        side.host->done = is[IS_DONE];
-                        side.host->iter = S.iter + 1;
+                    if (host) {
+                        host->done = is[IS_DONE];
+                        host->iter = S.iter + 1;
                     }
                 } else if (stage == RED_ERR_SET) {
                     record_error(sc, is, hist, S, S.iter, finish_norm(v[0], measure));
@@ -166,6 +132,71 @@ __global__ __launch_bounds__(kReduceThreads) void k_reduce(const double *__restr
         }
         __syncthreads();
     }
+}
+
+// The controller's step from the stress partials [nstr][nblk] (1024 threads; the
+// sums in k_reduce's order, the step with the host's operations in its order and
+// without contraction, a thread per row).  All quantities are loaded and reduced
+// together and the state is copied to LDS first: one thread following it through
+// global memory, and the sums two at a time, took 13 us per evaluation at 64^3;
+// this kernel 8.3 (64^3 J2 ramp 84.2 -> 80.1 ms).
+__global__ __launch_bounds__(kReduceThreads) void k_mixed_control(const double *__restrict__ partial, int nblk,
+                                                                  MixedCtl *ctl, double *g0, const int *is)
+{
+#pragma clang fp contract(off)
+    constexpr int     NW = kReduceThreads / 64, NQ = 9;
+    __shared__ MixedCtl m;
+    __shared__ double   sm[NQ][NW], sum[NQ], rhs[NQ];
+    if (is[IS_DONE])
+        return;
+    static_assert(sizeof(MixedCtl) % 8 == 0 && sizeof(MixedCtl) / 8 <= kReduceThreads, "one word per thread");
+    const int t = threadIdx.x;
+    if (t < (int) (sizeof(MixedCtl) / 8))
+        reinterpret_cast<double *>(&m)[t] = reinterpret_cast<const double *>(ctl)[t];
+    const int nq = ctl->nstr;
+    double    v[NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+        double a[4] = {0.0, 0.0, 0.0, 0.0};
+        if (q < nq) {
+            const double *src = partial + (int64_t) q * nblk;
+            int           b   = t;
+            for (; b + 3 * kReduceThreads < nblk; b += 4 * kReduceThreads)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    a[j] += src[b + j * kReduceThreads];
+            for (; b < nblk; b += kReduceThreads)
+                a[0] += src[b];
+        }
+        v[q] = (a[0] + a[1]) + (a[2] + a[3]);
+    }
+#pragma unroll
+    for (int q = 0; q < NQ; ++q)
+        if (q < nq) {
+            v[q] = wave_sum(v[q]);
+            if ((t & 63) == 0)
+                sm[q][t >> 6] = v[q];
+        }
+    __syncthreads();
+    if (t < nq) {
+        double a = sm[t][0];
+        for (int w = 1; w < NW; ++w)
+            a += sm[t][w];
+        sum[t] = a;
+    }
+    __syncthreads();
+    if (t < m.nF)
+        rhs[t] = m.PF[t] - sum[m.idx[t]] / m.N;
+    __syncthreads();
+    if (t < m.nF) {
+        double dE = 0.0;
+        for (int j = 0; j < m.nF; ++j)
+            dE += m.M[t * m.nF + j] * rhs[j];
+        m.g[m.idx[t]] += dE;
+    }
+    __syncthreads();
+    if (t < nq)
+        ctl->g[t] = g0[t] = m.g[t];
 }
 
 // Statistics of per-voxel isotropic moduli for the reference stiffness and the
