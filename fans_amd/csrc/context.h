@@ -126,6 +126,9 @@ inline int zct_lines(int h, int M)
     }
 }
 
+// threads of the z kernels
+inline int zct_nt(int h, int M) { return M / (M >= 32 ? 8 : 4) * zct_lines(h, M) * h; }
+
 template <typename T>
 struct Fft3D {
     int           nx = 0, ny = 0, nz = 0, h = 0, M = 0, Mc = 0;
@@ -423,6 +426,12 @@ inline Slots launch_slots(const fans_gpu_ctx *c, bool gated)
 // (144^3 mixed) 10.61 to 10.43; with 2400 (200 x 192 x 160 conduction) from 4.77 to
 // 4.80 and, mixed, 4.01 to 4.17: every workgroup reads all of them
 constexpr int kFoldMax = 2304;
+// and, in a batch, the partials that all workgroups of the two z passes read in one
+// iteration: the reduction launches are shared by the slots there.  Folded, 32 RVEs
+// of 64^3 conduction (3 million) solve in 7.5 ms against 7.8, 11 of 96^3 (4 million)
+// in 7.1 against 7.2, but 40 of 48^3 elasticity (12 million) in 13.0 against 12.7
+// and 11 of 96^3 (24 million and more) in 18.8 against 17.8
+constexpr int64_t kFoldBatch = 8'000'000;
 
 // ---- launches ----------------------------------------------------------------
 // z passes, strided (y or x) pass, x+Green pass; x+Green returns its block count

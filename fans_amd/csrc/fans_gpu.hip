@@ -265,7 +265,7 @@ void clear_map(fans_gpu_ctx *c)
 }
 
 int reduce(fans_gpu_ctx *c, const double *partial, int nblk, int nq, int stage, const double *partial_b = nullptr,
-           int nblk_b = 0, HostScalars *host = nullptr);
+           int nblk_b = 0, HostScalars *host = nullptr, int nt = 0);
 
 // ---------------------------------------------------------------------------
 // FFT convolution: out = G * r  with the requested epilogue.  With `pro` the
@@ -276,7 +276,8 @@ int reduce(fans_gpu_ctx *c, const double *partial, int nblk, int nq, int stage, 
 // ---------------------------------------------------------------------------
 template <typename T>
 int convolve_dev(fans_gpu_ctx *c, Fft3D<T> &P, T *rin, cplx<T> *spec, const T *Gp, int epi, EpiArgs<T> ep,
-                 const int *done, const ProArgs<T> *pro = nullptr, const std::function<int()> &after_z = nullptr)
+                 const int *done, const ProArgs<T> *pro = nullptr, const std::function<int()> &after_z = nullptr,
+                 int red_nt = 0)
 {
     const int  h = c->h, Kc = P.Mc * h;
     const bool fold = epi == EPI_CGDF;
@@ -301,7 +302,7 @@ int convolve_dev(fans_gpu_ctx *c, Fft3D<T> &P, T *rin, cplx<T> *spec, const T *G
     }
     HIPCHK(c, hipGetLastError());
     if (pro && !fold) {
-        const int rc = reduce(c, pro->partial, (int) P.nblk_z, 1, RED_ERR_NEXT);
+        const int rc = reduce(c, pro->partial, (int) P.nblk_z, 1, RED_ERR_NEXT, nullptr, 0, nullptr, red_nt);
         if (rc)
             return rc;
     }
@@ -340,7 +341,7 @@ int convolve_dev(fans_gpu_ctx *c, Fft3D<T> &P, T *rin, cplx<T> *spec, const T *G
     }
     if (epi == EPI_CGD) {
         HIPCHK(c, hipGetLastError());
-        const int rc = reduce(c, xg_partial, xg_blocks, 1, RED_DELTA);
+        const int rc = reduce(c, xg_partial, xg_blocks, 1, RED_DELTA, nullptr, 0, nullptr, red_nt);
         if (rc)
             return rc;
     }
@@ -500,11 +501,11 @@ int residual64(fans_gpu_ctx *c, const double *uin, double *rout, const double *d
 }
 
 int reduce(fans_gpu_ctx *c, const double *partial, int nblk, int nq, int stage, const double *partial_b,
-           int nblk_b, HostScalars *host)
+           int nblk_b, HostScalars *host, int nt)
 {
     Timed t(c, KF_REDUCE);
     hipLaunchKernelGGL(k_reduce, dim3(1, 1, c->gz), dim3(kReduceThreads), 0, c->stream, partial, nblk, nq, stage, c->sc,
-                       c->is, c->hist, partial_b, nblk_b, launch_slots(c, false), host);
+                       c->is, c->hist, partial_b, nblk_b, launch_slots(c, false), host, nt);
     HIPCHK(c, hipGetLastError());
     return 0;
 }
@@ -865,8 +866,11 @@ int cg_linear_loop(fans_gpu_ctx *c, Fft3D<T> &P, T *r, T *const *ring, T *rnew, 
     // The partials of the matvec, the forward z pass and x+Green then lie one
     // after the other in `partial`, each kept until its consumer has run.
     const int64_t nz_p = P.nblk_z, nx_p = x_green_blocks(P, c->h, c->ny);
-    const bool    fold = std::max<int64_t>({c->nblk_asm, nz_p, nx_p}) <= kFoldMax && c->fft_chunks <= 1 &&
-                      c->nblk_asm + nz_p + nx_p <= c->partial_len;
+    const bool    few  = std::max<int64_t>({c->nblk_asm, nz_p, nx_p}) <= kFoldMax && c->fft_chunks <= 1 &&
+                     c->nblk_asm + nz_p + nx_p <= c->partial_len;
+    const bool    fold = few && (c->gz == 1 || c->gz * nz_p * (c->nblk_asm + 2 * nz_p + nx_p) <= kFoldBatch);
+    // a batch past that keeps the folded sums' order
+    const int red_nt = few && !fold ? (P.zct ? zct_nt(c->h, P.M) : kThreads) : 0;
     // u -= alpha_m d_m for the ring slots 0 .. count-1 (iterations filled in
     // order); count < 0: each RVE slot's pending count; gated: finished RVE
     // slots skip it
@@ -951,7 +955,7 @@ int cg_linear_loop(fans_gpu_ctx *c, Fft3D<T> &P, T *r, T *const *ring, T *rnew, 
         }
         int e;
         if ((e = convolve_dev<T>(c, P, r, spec, Gp, fold ? EPI_CGDF : EPI_CGD, ep, done, with_pro ? &pa : nullptr,
-                                 ring_full)))
+                                 ring_full, red_nt)))
             return e;
         // rnew = K d, <d, rnew>
         AsmArgs<T> a = asm_args<T>(c);
@@ -965,7 +969,7 @@ int cg_linear_loop(fans_gpu_ctx *c, Fft3D<T> &P, T *r, T *const *ring, T *rnew, 
             return 0;
         // quantity 1, <d, K d_prev>, is zero in the first iteration
         if ((e = reduce(c, c->partial, c->nblk_asm, j > 0 ? 2 : 1, RED_ALPHA, j > 0 ? c->partial_e : nullptr,
-                        (int) P.nblk_z)))
+                        (int) P.nblk_z, nullptr, red_nt)))
             return e;
         if (j % kDirRing == kDirRing - 1 && (e = ring_update(kDirRing, true)))
             return e;

@@ -45,10 +45,13 @@ constexpr int kReduceThreads = 1024;
 // partial_b (nullable): quantity 1 comes from partial_b[0, nblk_b) instead of
 // partial[nblk, 2 nblk) (two producing kernels of different grids)
 // One block per slot of the launch (grid z); every buffer at its slot's offset.
+// nt > 0: the sums are taken as nt threads of a folding z pass take them, bit for
+// bit, so that a batch that launches reductions gives each slot the scalars of its
+// single solve.
 __global__ __launch_bounds__(kReduceThreads) void k_reduce(const double *__restrict__ partial, int nblk, int nq,
                                                            int stage, double *sc, int *is, double *hist,
                                                            const double *__restrict__ partial_b, int nblk_b,
-                                                           Slots sl, HostScalars *host)
+                                                           Slots sl, HostScalars *host, int nt)
 {
     __shared__ double sm[2 * (kReduceThreads / 64)];
     const int         sb = slot_of(sl, false);
@@ -77,6 +80,21 @@ __global__ __launch_bounds__(kReduceThreads) void k_reduce(const double *__restr
                 const double *src = alt ? partial_b : partial + (int64_t) (q + k) * nblk;
                 const int     nb  = alt ? nblk_b : nblk;
                 int           b   = threadIdx.x;
+                if (nt) {
+                    // threads < nt, in the order of fold_partials<nt>
+                    for (; b < nb && (int) threadIdx.x < nt; b += kFoldLoads * nt) {
+                        double x[kFoldLoads];
+#pragma unroll
+                        for (int j = 0; j < kFoldLoads; ++j)
+                            x[j] = src[min(b + j * nt, nb - 1)];
+#pragma unroll
+                        for (int j = 0; j < kFoldLoads; ++j) {
+                            const double y = b + j * nt < nb ? x[j] : 0.0;
+                            a[0]           = mx[k] ? fmax(a[0], y) : a[0] + y;
+                        }
+                    }
+                    b = nb;
+                }
                 for (; b + 3 * kReduceThreads < nb; b += 4 * kReduceThreads)
 #pragma unroll
                     for (int j = 0; j < 4; ++j) {

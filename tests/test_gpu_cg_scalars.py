@@ -68,3 +68,41 @@ def test_folded_scalars_in_mixed_solves(kind, dims):
     for (ka, ha, ua), (kb, hb, ub) in zip(_run(p, "mixed", 1), _run(p, "mixed", 2)):
         assert abs(ka - kb) <= 2
         assert relerr(ua, ub) < 1e-7
+
+
+@pytest.mark.parametrize("kind,precision", [("elastic", "fp64"), ("elastic", "mixed"), ("thermal", "fp64")])
+def test_batch_past_the_fold_limit_matches_single_solves(kind, precision):
+    """A batch whose workgroups would read more partials than folding pays for
+    launches reductions in the folded order: bit for bit the single solves, which
+    fold (144-, 192-thread and generic z passes)."""
+    dims, n = {"elastic": ((96, 96, 48), 4), "thermal": ((160, 160, 10), 3)}[kind]
+    print(f"[gpu-case] batch past the fold limit {kind} {precision} {dims} x {n}", flush=True)
+    ps = []
+    for s in range(n):
+        p = _problem(kind, dims, "Linfinity", "absolute", 1e-300, 9)
+        p.ms = np.random.default_rng(s).integers(0, 2, size=dims).astype(np.uint16)
+        ps.append(p)
+    g0 = [0.01] + [0.0] * (ps[0].n_str - 1)
+    single = []
+    for p in ps:
+        g = gpu.GpuSolver(p, precision=precision)
+        try:
+            g.set_gradient(g0)
+            g.solve()
+            single.append((int(g.stats.inner_iterations), g.homogenized_stress().copy(), g.get_u().copy()))
+        finally:
+            g.close()
+    b = gpu.GpuBatch(ps, precision=precision)
+    try:
+        for k, p in enumerate(ps):
+            b.load_slot(k, p, g0)
+        b.solve()
+        its = b.results()[0]
+        st = b.stresses()
+        for k in range(n):
+            assert its[k] == single[k][0]
+            assert np.array_equal(st[k], single[k][1])
+            b.select(k)
+            assert np.array_equal(b.get_u(), single[k][2])
+    finally:
+        b.close()
