@@ -32,12 +32,6 @@
 namespace fans {
 
 enum { ASM_RESID = 0, ASM_CGLIN = 1 };
-#ifndef FANS_MODAL_WAVES64
-#define FANS_MODAL_WAVES64 3
-#endif
-#ifndef FANS_MODAL_WAVES32
-#define FANS_MODAL_WAVES32 5
-#endif
 constexpr int TILE = 16;  // element tile edge (y and z)
 constexpr int NOUT = TILE - 1;
 
@@ -117,14 +111,10 @@ __device__ __forceinline__ void slot_asm(AsmArgs<T> &a, int sb)
 }
 
 // waves per SIMD asked of k_assemble_modal
-template <typename T, int H, int MODE, int VAR>
+template <int H, int VAR>
 constexpr int kModalWaves()
 {
-    if (VAR == ASM_ANISO)
-        return sizeof(T) == 8 ? 2 : 4;
-    if (H == 1)
-        return sizeof(T) == 8 ? 5 : 8;
-    return sizeof(T) == 8 ? FANS_MODAL_WAVES64 : FANS_MODAL_WAVES32;
+    return VAR == ASM_ANISO ? 2 : H == 1 ? 5 : 3;
 }
 
 // phases whose moduli (ASM_ANISO: tensors, in dynamic LDS) are staged per
@@ -137,21 +127,19 @@ constexpr int kTensorLen()
 }
 
 // one wave's request of SIZE bytes per lane from global memory straight to LDS:
-// lane l writes at lds + 4 l (SIZE <= 4) or lds + 16 l (SIZE 12).  Tracked by vmcnt like a load, in issue order.
+// lane l writes a word at lds + 4 l.  Tracked by vmcnt like a load, in issue order.
 template <int SIZE>
 __device__ __forceinline__ void load_to_lds(const void *src, void *lds)
 {
-    static_assert(SIZE == 1 || SIZE == 2 || SIZE == 4 || SIZE == 12, "sizes of the instruction used here");
+    static_assert(SIZE == 1 || SIZE == 2 || SIZE == 4, "sizes of the instruction used here");
     const auto s = (const __attribute__((address_space(1))) void *) src;
     const auto d = (__attribute__((address_space(3))) void *) lds;
     if constexpr (SIZE == 1)  // one byte (two) per lane, a zero-extended word in LDS
         __builtin_amdgcn_global_load_lds(s, d, 1, 0, 0);
     else if constexpr (SIZE == 2)
         __builtin_amdgcn_global_load_lds(s, d, 2, 0, 0);
-    else if constexpr (SIZE == 4)
-        __builtin_amdgcn_global_load_lds(s, d, 4, 0, 0);
     else
-        __builtin_amdgcn_global_load_lds(s, d, 12, 0, 0);
+        __builtin_amdgcn_global_load_lds(s, d, 4, 0, 0);
 }
 
 // workgroup barrier that leaves up to N of the wave's own latest requests (and
@@ -163,17 +151,14 @@ __device__ __forceinline__ void barrier_keep()
 }
 
 // the H values of a node in as few stores as their alignment allows (one store
-// per value cost 20 us more at 256^3 in FP64 and in FP32)
+// per value cost 20 us more at 256^3)
 template <typename T, int H>
 __device__ __forceinline__ void store_node(T *p, const T (&v)[H])
 {
-    if constexpr (H == 3 && sizeof(T) == 8) {
+    if constexpr (H == 3) {
         typedef double d2 __attribute__((ext_vector_type(2), aligned(8)));
         *reinterpret_cast<d2 *>(p) = d2{v[0], v[1]};
         p[2]                       = v[2];
-    } else if constexpr (H == 3) {
-        typedef float f3 __attribute__((ext_vector_type(3), aligned(4)));
-        *reinterpret_cast<f3 *>(p) = f3{v[0], v[1], v[2]};
     } else {
         p[0] = v[0];
     }
@@ -183,18 +168,15 @@ __device__ __forceinline__ void store_node(T *p, const T (&v)[H])
 // ids), the phase table in memory, or the voxel's own moduli (isotropic only)
 enum { MAT_STAGED = 0, MAT_TABLE = 1, MAT_VOXEL = 2 };
 
-// A staged node plane of k_assemble_modal: NL x NL nodes in units of UB bytes, UL
-// bytes apart in LDS (a 12-byte request leaves a gap of 4), requested by FULL
+// A staged node plane of k_assemble_modal: NL x NL nodes in words, requested by FULL
 // instructions of the four waves and one of REST lanes each.
 template <typename T, int H>
 struct ModalPlane {
     static constexpr int NL = TILE + 1, NBUF = 4;
-    static constexpr int UB = H == 3 && sizeof(T) == 4 ? 12 : 4, UL = UB == 12 ? 16 : 4;
-    static constexpr int UPN = H * (int) sizeof(T) / UB, UNITS = NL * NL * UPN;
+    static constexpr int UPN = H * (int) sizeof(T) / 4, UNITS = NL * NL * UPN;
     static constexpr int FULL = UNITS / 256, REST = (UNITS - 256 * FULL + 3) / 4, NREQ = FULL + 1;
     static_assert(REST > 0 && REST <= 64, "units of the last request");
-    static constexpr int ND    = UPN * UL / (int) sizeof(T);  // node stride in LDS
-    static constexpr int PLANE = (256 * FULL + 4 * REST) * UL / (int) sizeof(T);
+    static constexpr int PLANE = (256 * FULL + 4 * REST) * 4 / (int) sizeof(T);
 };
 // a bound on the static LDS of the kernel's ASM_ANISO variants: planes, ids, y
 // exchange and the small arrays
@@ -213,13 +195,13 @@ constexpr size_t modal_static_lds()
 // What bounds it: a wave issues 185 VALU instructions per plane (156 of them
 // FP64 arithmetic); without its stores and requests the 256^3 FP64 matvec takes
 // 0.17 ms, with them 0.26 (0.34 before: eight-corner transforms, two barriers,
-// register prefetch by one plane), FP32 0.11 and 0.15 (0.18).  FP64 keeps three
-// waves per SIMD at 156 registers, FP32 five at 87.  At 48^3 and 64^3 a plane of
+// register prefetch by one plane).  Three waves per SIMD at 156 registers.  At 48^3 and 64^3 a plane of
 // a workgroup alone on its CU takes 0.8 us (1.4 before).
 template <typename T, int H, int NGP, int MODE, int VAR, int MAT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kModalWaves<T, H, MODE, VAR>())))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kModalWaves<H, VAR>())))
 void k_assemble_modal(AsmArgs<T> a)
 {
+    static_assert(sizeof(T) == 8, "the FP64 form's kernel");
     constexpr bool CUBIC = VAR == ASM_ISO_CUBIC, ANISO = VAR == ASM_ANISO, RES = MODE == ASM_RESID;
     static_assert(!(ANISO && MAT == MAT_VOXEL), "per-voxel moduli are isotropic");
     const int sb = slot_of(a.sl);
@@ -228,8 +210,8 @@ void k_assemble_modal(AsmArgs<T> a)
     if (a.sl.map)  // batched launch: this slot's buffers
         slot_asm<T, H>(a, sb);
     using MP         = ModalPlane<T, H>;
-    constexpr int NS = H == 1 ? 3 : 6, NL = MP::NL, NBUF = MP::NBUF, UB = MP::UB, UL = MP::UL, UPN = MP::UPN;
-    constexpr int FULL = MP::FULL, REST = MP::REST, NREQ = MP::NREQ, ND = MP::ND;
+    constexpr int NS = H == 1 ? 3 : 6, NL = MP::NL, NBUF = MP::NBUF, UPN = MP::UPN;
+    constexpr int FULL = MP::FULL, REST = MP::REST, NREQ = MP::NREQ;
     // words of an element plane's material request
     constexpr int WPT  = (int) sizeof(T) / 4, NMOD = MAT == MAT_VOXEL ? (H == 3 ? 2 : 1) * WPT : 1;
     constexpr int KEEP = NREQ + NMOD;  // requests of one plane
@@ -263,7 +245,7 @@ void k_assemble_modal(AsmArgs<T> a)
 #pragma unroll
     for (int q = 0; q < NREQ; ++q) {
         const int u = min(q < FULL ? 256 * q + t : 256 * FULL + wave * REST + lane, MP::UNITS - 1), n = u / UPN;
-        off_req[q]  = ((unsigned) (wrapy(n / NL) * nz + wrapz(n % NL)) * UPN + u % UPN) * UB;
+        off_req[q]  = ((unsigned) (wrapy(n / NL) * nz + wrapz(n % NL)) * UPN + u % UPN) * 4;
     }
 
     const T w = (T) a.geom.w;
@@ -301,10 +283,10 @@ void k_assemble_modal(AsmArgs<T> a)
         constexpr int BUF = decltype(bufc)::value;
 #pragma unroll
         for (int q = 0; q < FULL; ++q)
-            load_to_lds<UB>(nsrc + off_req[q], reinterpret_cast<char *>(Un[BUF]) + (256 * q + 64 * wave) * UL);
+            load_to_lds<4>(nsrc + off_req[q], reinterpret_cast<char *>(Un[BUF]) + (256 * q + 64 * wave) * 4);
         if (lane < REST)
-            load_to_lds<UB>(nsrc + off_req[FULL],
-                                       reinterpret_cast<char *>(Un[BUF]) + (256 * FULL + wave * REST) * UL);
+            load_to_lds<4>(nsrc + off_req[FULL],
+                           reinterpret_cast<char *>(Un[BUF]) + (256 * FULL + wave * REST) * 4);
         if constexpr (decltype(matc)::value) {
             constexpr int MB = (BUF + NBUF - 1) % NBUF;
             if constexpr (MAT == MAT_VOXEL) {
@@ -331,7 +313,7 @@ void k_assemble_modal(AsmArgs<T> a)
     auto cell_walsh = [&](const T *src, T(&q)[4][H]) {
 #pragma unroll
         for (int c = 0; c < H; ++c) {
-            const T u0 = src[c], u1 = src[NL * ND + c], u2 = src[ND + c], u3 = src[(NL + 1) * ND + c];
+            const T u0 = src[c], u1 = src[NL * H + c], u2 = src[H + c], u3 = src[(NL + 1) * H + c];
             const T s0 = u0 + u1, d0 = u0 - u1, s1 = u2 + u3, d1 = u2 - u3;
             q[0][c] = s0 + s1;
             q[1][c] = d0 + d1;
@@ -342,7 +324,7 @@ void k_assemble_modal(AsmArgs<T> a)
 
     // node plane X0 - 1 + i sits in buffer i % NBUF, the material of the element
     // plane above it likewise
-    const int own = (ey * NL + ez) * ND;
+    const int own = (ey * NL + ez) * H;
     T         qp[4][H], carry[4][H];
     double    acc0 = 0.0, acc1 = 0.0;
     request(std::integral_constant<int, 0>{}, std::false_type{});

@@ -1174,10 +1174,8 @@ __device__ __forceinline__ void modal_aniso(const T (&w)[8][H], const Geom &g, c
 template <typename T>
 __device__ __forceinline__ T staged_value(const int *p)
 {
-    if constexpr (sizeof(T) == 8)
-        return __hiloint2double(p[256], p[0]);
-    else
-        return __int_as_float(p[0]);
+    static_assert(sizeof(T) == 8, "two words");
+    return __hiloint2double(p[256], p[0]);
 }
 
 // lane l <- lane l-1 inside each row of 16 lanes (DPP row_shr:1); row starts get 0
