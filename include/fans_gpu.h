@@ -267,7 +267,7 @@ int fans_gpu_stream_bandwidth(int32_t device, int64_t bytes, int32_t reps, doubl
  * of the convolution on k kz-chunks in turn (k >= 1); FANS_OPT_GRAPHS=0/1
  * launches the linear CG iterations eagerly / replays them from a captured
  * hipGraph (default 1); FANS_OPT_ASM_PLANES=p sets the x planes each assembly
- * workgroup marches through (default 16, or n_x/4 below 64);
+ * workgroup marches through (default: by grid size, at most 16);
  * FANS_OPT_OPERATOR_FP32=1 makes fans_gpu_convolve and the linear matvec of
  * fans_gpu_residual (linear_kd=1) run the FP32 kernels of the mixed form's
  * inner solve (input rounded to FP32, output widened; contexts created with
