@@ -414,8 +414,10 @@ AsmArgs<T> asm_args(fans_gpu_ctx *c)
 // a workgroup alone on its CU takes 1.75 units per plane in the modal kernel
 // (latency; three fit) and 1 in the per-Gauss-point one, so too few workgroups
 // cost more than the extra plane of thin ones: the 48^3 elastic matvec (16 tiles)
-// took 24 us at 12 planes (64 workgroups), the 64^3 J2 residual (25 tiles) 118 us
-// at 16 (100 workgroups).
+// took 24 us at 12 planes (64 workgroups) and 8.4 at the rule's depth, the 64^3 J2
+// residual (25 tiles) 118 us at 16 (100 workgroups) and 58 at 7; over five J2 grids
+// from 36^3 to 96^3 the rule is within 5 % of the best depth.  k_assemble in the mixed
+// form takes the per-Gauss-point line (64^3 elastic solve 3.87 -> 2.84 ms).
 int asm_planes_rule(int nx, int64_t tiles, bool modal, int grp = 1)
 {
     constexpr int kCus = 256, kMaxPlanes = 16;

@@ -960,7 +960,10 @@ __global__ __launch_bounds__((zct_threads<H, M>())) void k_fft_z_c2r_ct(const cp
 
 // ---- batched strided complex pass (y or x axis) ----------------------------
 // data[o*ostride + i*sn + b] for i < L.n, b in [c0, c1); block (bx, o) owns
-// columns [c0 + bx*bc, c0 + bx*bc + bc).
+// columns [c0 + bx*bc, c0 + bx*bc + bc).  FP64, lengths without a register kernel.
+// Bound by memory where the tile is 16 columns wide (125 x 120 x 150, y of 120 points:
+// 24 us, 4.6 TB/s; radix 2 to 8 Stockham stages through the whole tile took 34), four
+// waves per SIMD.
 template <typename T, bool INV>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_fft_strided(cplx<T> *__restrict__ data, FftLen L,
                                                      const cplx<T> *__restrict__ tw, int64_t sn, int c0, int c1,
@@ -1094,6 +1097,11 @@ __device__ __forceinline__ cplx<T> green_row(const T *__restrict__ g, T sx, T sy
 // ny blocks) owns kz in [kz_lo + bx*bk, ... + bk) and all H.
 // G packed per frequency [x][y][kz][H(H+1)/2] = (00 01 02 11 12 22) or (0).
 // partial (nullable): one partial of <r, s> (s = -G r) per block.
+// FP64, lengths without a register kernel.  Bound by issue and latency: 240 VALU
+// instructions per value at 125 points (half of them indices), 49 % of the issue slots
+// at three waves per SIMD (a fourth would spill).  48^3 elastic 8.3 us (20.7 with
+// Stockham stages and the Green product read back from LDS), 200 x 192 x 160
+// conduction 44 (64), 96^3 elastic 18.5 (29).
 template <typename T, int H>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_fft_x_green(cplx<T> *__restrict__ data, FftLen L,
                                                      const cplx<T> *__restrict__ tw, GreenView<T> gv, int kz_lo,
