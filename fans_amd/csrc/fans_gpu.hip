@@ -417,7 +417,8 @@ AsmArgs<T> asm_args(fans_gpu_ctx *c)
 // took 24 us at 12 planes (64 workgroups) and 8.4 at the rule's depth, the 64^3 J2
 // residual (25 tiles) 118 us at 16 (100 workgroups) and 58 at 7; over five J2 grids
 // from 36^3 to 96^3 the rule is within 5 % of the best depth.  k_assemble in the mixed
-// form takes the per-Gauss-point line (64^3 elastic solve 3.87 -> 2.84 ms).
+// form takes the per-Gauss-point line (with the folded scalars 64^3 elastic 3.87 ->
+// 2.84 ms).
 int asm_planes_rule(int nx, int64_t tiles, bool modal, int grp = 1)
 {
     constexpr int kCus = 256, kMaxPlanes = 16;
