@@ -12,6 +12,7 @@
 #include <cmath>
 #include <functional>
 #include <string>
+#include <tuple>
 #include <utility>
 #include <vector>
 
@@ -283,6 +284,11 @@ struct SlotHost {
     double                     kref[81]{}, keref[576]{}, g0[9]{}, gvec[9]{}, gvec_prev[9]{};
 };
 
+// what the launches of a captured CG iteration depend on beside the context's
+// settings (drop_graphs): the first direction buffer (with it the precision), the
+// slots per launch (gz) and whether the z passes fold the scalars
+using GraphKey = std::tuple<const void *, int, bool>;
+
 }  // namespace fans
 
 using namespace fans;  // the context is the C ABI's type, at global scope
@@ -396,11 +402,9 @@ struct fans_gpu_ctx {
     bool                                                op_fp32 = false;
     // single-RVE mixed form with restarted inner solves (as batched contexts)
     bool                                                mixed_restart = false;
-    // captured CG iterations (hipGraph), keyed by precision and the direction
-    // buffer current at the first captured iteration
+    // captured CG iterations (hipGraph)
     bool                                                use_graphs = true;
-    // key: the direction buffer and the slots per launch (gz)
-    std::vector<std::pair<std::pair<const void *, int>, hipGraphExec_t>> graphs;
+    std::vector<std::pair<GraphKey, hipGraphExec_t>>    graphs;
     std::array<int, 7>                                  graph_sig{};
     std::vector<std::pair<int, std::pair<hipEvent_t, hipEvent_t>>> ev_used;
     std::vector<hipEvent_t>                             ev_pool;
@@ -427,10 +431,12 @@ inline Slots launch_slots(const fans_gpu_ctx *c, bool gated)
 // 4.80 and, mixed, 4.01 to 4.17: every workgroup reads all of them
 constexpr int kFoldMax = 2304;
 // and, in a batch, the partials that all workgroups of the two z passes read in one
-// iteration: the reduction launches are shared by the slots there.  Folded, 32 RVEs
-// of 64^3 conduction (3 million) solve in 7.5 ms against 7.8, 11 of 96^3 (4 million)
-// in 7.1 against 7.2, but 40 of 48^3 elasticity (12 million) in 13.0 against 12.7
-// and 11 of 96^3 (24 million and more) in 18.8 against 17.8
+// iteration with every slot running: the reduction launches are shared by the slots
+// there.  Folded, 32 RVEs of 64^3 conduction (3 million) solve in 7.5 ms against 7.8,
+// 11 of 96^3 (4 million) in 7.1 against 7.2, but 40 of 48^3 elasticity (12 million)
+// in 13.0 against 12.7 and 11 of 96^3 (24 million and more) in 18.8 against 17.8.
+// Decided per phase instead, from the slots still running, a mixed solve takes the
+// same time (40 of 48^3 12.8 ms either way, 32 of 64^3 16.9).
 constexpr int64_t kFoldBatch = 8'000'000;
 
 // ---- launches ----------------------------------------------------------------

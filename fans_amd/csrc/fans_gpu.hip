@@ -851,9 +851,9 @@ int read_is_all(fans_gpu_ctx *c, std::vector<int> &is)
 // loop runs its slots in lockstep, each stopping on its own test (its
 // launches return at entry from then on); the finished slots leave the map
 // once at most half of its slots still run.
-// j0 > 0 (single RVE): continue a stopped loop at iteration j0 with a
-// replaced residual r (the residual after iteration j0 - 1's update; the
-// directions, K d_(j0-1) in rnew and the CG scalars are kept).
+// j0 > 0: continue a stopped loop at iteration j0 with a replaced residual r
+// (the residual after iteration j0 - 1's update; the directions, K d_(j0-1) in
+// rnew and the CG scalars are kept).
 template <typename T>
 int cg_linear_loop(fans_gpu_ctx *c, Fft3D<T> &P, T *r, T *const *ring, T *rnew, T *u, cplx<T> *spec, const T *Gp,
                    const Phase<T> *ph, int *iters_out, int j0 = 0)
@@ -871,8 +871,11 @@ int cg_linear_loop(fans_gpu_ctx *c, Fft3D<T> &P, T *r, T *const *ring, T *rnew, 
     const int64_t nz_p = P.nblk_z, nx_p = x_green_blocks(P, c->h, c->ny);
     const bool    few  = std::max<int64_t>({c->nblk_asm, nz_p, nx_p}) <= kFoldMax && c->fft_chunks <= 1 &&
                      c->nblk_asm + nz_p + nx_p <= c->partial_len;
-    const bool    fold = few && (c->gz == 1 || c->gz * nz_p * (c->nblk_asm + 2 * nz_p + nx_p) <= kFoldBatch);
-    // a batch past that keeps the folded sums' order
+    // A batch takes one form whatever number of its slots runs: the two keep alpha and
+    // the previous delta in different places between iterations, so neither a later
+    // phase of a mixed solve nor a replayed graph may belong to the other.  Past the
+    // limit it keeps the folded sums' order.
+    const bool fold = few && (c->nb == 1 || c->nb * nz_p * (c->nblk_asm + 2 * nz_p + nx_p) <= kFoldBatch);
     const int red_nt = few && !fold ? (P.zct ? zct_nt(c->h, P.M) : kThreads) : 0;
     // u -= alpha_m d_m for the ring slots 0 .. count-1 (iterations filled in
     // order); count < 0: each RVE slot's pending count; gated: finished RVE
@@ -980,8 +983,8 @@ int cg_linear_loop(fans_gpu_ctx *c, Fft3D<T> &P, T *r, T *const *ring, T *rnew, 
     };
     // After iteration 0 the launches of iteration j depend on j % kDirRing
     // only, so kDirRing iterations are captured once into a hipGraph (per
-    // direction buffer and grid depth) and replayed (one launch per replay
-    // instead of ~10 per iteration).  Timing mode stays eager.
+    // direction buffer, grid depth and form of the scalars) and replayed (one
+    // launch per replay instead of ~10 per iteration).  Timing mode stays eager.
     static_assert(kDirRing == 8, "one captured graph holds one turn of the direction ring");
     if (c->use_graphs && !c->timing) {
         // eager up to the first iteration of a ring turn's graph (j = 1 mod 8)
@@ -998,8 +1001,8 @@ int cg_linear_loop(fans_gpu_ctx *c, Fft3D<T> &P, T *r, T *const *ring, T *rnew, 
                 return finish();
         }
         for (;;) {
-            const std::pair<const void *, int> key{(const void *) ring[0], c->gz};
-            hipGraphExec_t                     exec = nullptr;
+            const GraphKey key{(const void *) ring[0], c->gz, fold};
+            hipGraphExec_t exec = nullptr;
             for (auto &g : c->graphs)
                 if (g.first == key)
                     exec = g.second;

@@ -106,3 +106,55 @@ def test_batch_past_the_fold_limit_matches_single_solves(kind, precision):
             assert np.array_equal(b.get_u(), single[k][2])
     finally:
         b.close()
+
+
+def test_mixed_batch_that_falls_below_the_fold_limit_matches_single_solves():
+    """Five slots of 128 x 128 x 10 elasticity launch reductions, three or fewer of
+    them alone would fold (their workgroups read 2.5 million partials per slot and
+    iteration).  Slots of small load end after the first FP32 phase, slots of low
+    contrast leave the map early within a phase, and later solves on the same context
+    run two slots, one, and all of them again (captured iterations of every depth are
+    replayed).  Each slot is bit for bit its single solve, and meets the tolerance."""
+    dims, big, small = (128, 128, 10), 1e-2, 1e-8
+    contrast = [1.2, 1.2, 8.0, 60.0, 60.0]
+    ps = []
+    for s, f in enumerate(contrast):
+        p = _problem("elastic", dims, "Linfinity", "absolute", 1e-10, 400)
+        p.ms = np.random.default_rng(s).integers(0, 2, size=dims).astype(np.uint16)
+        p.groups = [MaterialGroup("LinearElasticIsotropic", [0, 1], {"bulk_modulus": [1.0, f], "shear_modulus": [0.6, 0.6 * f]})]
+        ps.append(p)
+    load = lambda a: [a] + [0.0] * 5
+    runs = [[small, small, big, big, big], [0.0, 0.0, 0.0, big, big], [0.0, 0.0, 0.0, 0.0, big],
+            [big, small, big, small, big]]
+    single = {}
+    for k, a in sorted({(k, a) for r in runs for k, a in enumerate(r) if a}):
+        print(f"[gpu-case] single mixed solve, slot {k} load {a}", flush=True)
+        g = gpu.GpuSolver(ps[k], precision="mixed")
+        try:
+            g.set_gradient(load(a))
+            g.solve()
+            assert g.stats.converged
+            single[k, a] = (int(g.stats.inner_iterations), g.homogenized_stress().copy(), g.get_u().copy())
+        finally:
+            g.close()
+    b = gpu.GpuBatch(ps, precision="mixed")
+    try:
+        for r in runs:
+            print(f"[gpu-case] mixed batch below the fold limit, loads {r}", flush=True)
+            for k, p in enumerate(ps):
+                b.load_slot(k, p, load(r[k]))
+            b.solve()
+            its, conv, _ = b.results()
+            its, conv, st = list(its), list(conv), b.stresses()
+            assert all(conv)
+            for k, a in enumerate(r):
+                b.select(k)
+                u = b.get_u()
+                if not a:
+                    assert its[k] == 0 and not u.any()
+                    continue
+                assert its[k] == single[k, a][0]
+                assert np.array_equal(st[k], single[k, a][1])
+                assert np.array_equal(u, single[k, a][2])
+    finally:
+        b.close()
