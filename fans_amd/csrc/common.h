@@ -72,11 +72,13 @@ __device__ __forceinline__ double wave_max(double v)
 }
 
 // Block-wide reduction of NV doubles; result valid in thread 0.  `sm` must hold
-// NV * (blockDim.x / 64) doubles.  is_max selects max instead of sum per slot.
+// NV doubles per wave, a last wave of fewer than 64 threads included (its shuffles
+// read zeros from the missing lanes, which leave a sum, or a maximum of
+// non-negative values, as it is).  is_max selects max instead of sum per slot.
 template <int NV>
 __device__ __forceinline__ void block_reduce(double (&v)[NV], const bool (&is_max)[NV], double *sm)
 {
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
 #pragma unroll
     for (int k = 0; k < NV; ++k)
         v[k] = is_max[k] ? wave_max(v[k]) : wave_sum(v[k]);

@@ -216,7 +216,7 @@ __global__ __launch_bounds__(C *N2) void k_fft_x_green_reg(cplx<T> *__restrict__
         gv.G += sb * sl.green;
         partial = slot_ptr(partial, sb * sl.part);
     }
-    __shared__ double red[(C * N2) / 64];
+    __shared__ double red[(C * N2 + 63) / 64];
     double            acc = 0.0;
     constexpr int  N    = N1 * N2;
     constexpr bool GRP3 = H == 3 && C == 3 * KB + 1;
