@@ -1119,7 +1119,9 @@ int solve_cg_fp64(fans_gpu_ctx *c)
     hs.done         = is[IS_DONE];
     hs.iter         = is[IS_ITER];
     double *d       = c->dA;
-    while (!hs.done) {
+    // left after the wait below: hs is read nowhere else, the reductions that store it
+    // may still be running (done stored, iter not yet)
+    while (!is[IS_DONE]) {
         const size_t mark = c->ev_used.size();
         // deltamid = <r, s>
         hipLaunchKernelGGL((k_dot<double>), dim3(c->nblk_vec), dim3(kThreads), 0, c->stream, c->r, c->s, c->Nh,

@@ -65,3 +65,38 @@ def test_strain_control_and_converged_start(precision):
         assert relerr(g.macro_gradient(), g0) < 1e-15
     finally:
         g.close()
+
+
+@pytest.mark.parametrize("timing", [False, True])
+@pytest.mark.parametrize("mixed_bc", [False, True])
+def test_iterations_and_history_of_the_stopping_iteration(mixed_bc, timing):
+    """The host takes the stop flag and the iteration from memory that the device
+    writes: read before the stream is waited for, a run could report the iteration
+    before its last.  Runs cut at n_it and one to convergence, many of each, on a grid
+    whose kernels end before the host looks; exact comparisons only."""
+    print(f"[gpu-case] nonlinear stop, mixed_bc={mixed_bc} timing={timing}", flush=True)
+    p = cases.j2(dims=(4, 6, 8), seed=3, count=1, rmin=1.0, rmax=1.5)
+    for n_it in (1, 2, 3, 300):
+        p.n_it, p.tol = n_it, (1e-300 if n_it < 300 else 1e-9)
+        g = gpu.GpuSolver(p, timing=timing)
+        try:
+            first = None
+            for _ in range(25):
+                g.reset_state()
+                if mixed_bc:
+                    g.enable_mixed_bc(cases.uniaxial_mixed(2, 0.02), 0)
+                else:
+                    g.set_gradient([0.004, 0.0, -0.001, 0.0, 0.002, 0.0])
+                n, h = g.solve(), g.error_history().copy()
+                assert h.shape == (n + 1,) and (h > 0.0).all()
+                assert h[-1] == g.stats.final_error
+                assert bool(g.stats.converged) == (h[-1] <= p.tol)
+                if n_it < 300:
+                    assert n == n_it
+                else:
+                    assert g.stats.converged and (h[:-1] > p.tol).all()
+                if first is None:
+                    first = h
+                assert np.array_equal(h, first)
+        finally:
+            g.close()
